@@ -429,6 +429,10 @@ int q3_layer_rows(q3_model *m, int l, float *out, int rows) {
     return ork_dev_download(m->ctx, out, m->trace + (size_t)l * m->c.max_rows * H, (size_t)rows * H * 4) ? -1 : 0;
 }
 
+/* Prefill attention by blocks of rows from this many rows: below, its third launch costs more than it saves (two
+ * layers at Qwen3-1.7B widths, blocks / row by row, us: M=8 166 / 161, M=16 166 / 163, M=24 178 / 173; M=64 161 / 167). */
+#define Q3_ATTN_BLOCK_ROWS 32
+
 /* ---- one pass of the decoder over M rows ------------------------------------------------------------------- */
 static int pass(q3_model *m, int M, int decode) {
     const q3_cfg *c = &m->c;
@@ -468,7 +472,7 @@ static int pass(q3_model *m, int M, int decode) {
         const int Sa = decode ? m->S : (M + Q3_CHUNK - 1) / Q3_CHUNK;
         q3_att at = {.M = M, .NH = NH, .NKV = NKV, .HD = HD, .S = Sa, .max_ctx = decode ? c->max_ctx : M,
                      .q = m->q, .kc = Ly->kc, .vc = Ly->vc, .st = m->st, .scale = 1.0f / sqrtf((float)HD),
-                     .part = m->part, .rows = m->fused};
+                     .part = m->part};
         if (M == 1) { /* one row: attention does the q/k/v post-processing itself */
             at.cq = m->cq;
             at.ck = m->ck;
@@ -488,9 +492,20 @@ static int pass(q3_model *m, int M, int decode) {
                                m->rcos, m->rsin, m->st, m->q, Ly->kc, Ly->vc};
             CK(q3k_qkv_post(&qp, s));
         }
-        CK(q3k_attn_part(&at, s));
-        const q3_aq aq = {M, NH, HD, Sa, m->part, m->a8att, m->asatt};
-        CK(q3k_attn_quant(&aq, s));
+        if (M >= Q3_ATTN_BLOCK_ROWS && m->fused) {
+            /* part holds the scores and the chunk statistics: pad64(M) + 2 Sa floats per (row, head), of the
+             * S * (HD + 2) it has (HD >= 64); the attention rows replace the queries */
+            at.sc = m->part;
+            at.ml = m->part + (size_t)M * NH * ((M + 63) / 64 * 64);
+            at.o = m->q;
+            CK(q3k_attn_rows(&at, s));
+            const q3_qr qr = {M, NH * HD, m->q, m->a8att, m->asatt};
+            CK(q3k_quant_rows(&qr, s));
+        } else {
+            CK(q3k_attn_part(&at, s));
+            const q3_aq aq = {M, NH, HD, Sa, m->part, m->a8att, m->asatt};
+            CK(q3k_attn_quant(&aq, s));
+        }
         CK(ork_i8_mm_run(m->ctx, Ly->l[Q3_WO].w, M, m->a8att, m->co));
         q3_nq n2 = nq;
         n2.emb = NULL;

@@ -60,7 +60,11 @@ typedef struct q3_att { /* grid (NKV * query-head sub-groups, S, M): Q3_CHUNK-ke
     const int *st;
     float scale;
     float *part; /* [M][NH][S][HD + 2]: P.V, then max and sum */
-    int rows;    /* unfused form: 1 = one workgroup per block of rows (k_attn_rows), 0 = per row; same partials */
+    /* prefill by blocks of rows (q3k_attn_rows): row t is at position t, LP = M rounded up to 64 */
+    int sr;    /* rows of a scores workgroup (set by the launcher) */
+    float *sc; /* scratch [M][NH][LP]: exp(score - chunk max) */
+    float *ml; /* scratch [M][NH][S][2]: chunk max and sum */
+    float *o;  /* [M][NH * HD] out: the attention rows; may be q */
     /* fused form (M = 1, cq != NULL): the q/k/v matmul results and what k_qkv_post takes */
     const int32_t *cq, *ck, *cv;
     const float *as, *wsq, *wsk, *wsv, *qn, *kn;
@@ -74,6 +78,13 @@ typedef struct q3_aq { /* chunk combine -> int8 rows */
     int8_t *a8; /* [M][NH*HD] */
     float *as;
 } q3_aq;
+
+typedef struct q3_qr { /* fp32 rows -> int8 rows */
+    int M, n;
+    const float *y; /* [M][n] */
+    int8_t *a8;
+    float *as;
+} q3_qr;
 
 typedef struct q3_glu { /* silu(gate) * up -> int8 rows */
     int M, F;
@@ -107,6 +118,8 @@ int q3k_norm_quant(const q3_nq *p, void *stream);
 int q3k_copy_f32(float *dst, const float *src, long long n, void *stream); /* n floats, device to device */
 int q3k_qkv_post(const q3_qkv *p, void *stream);
 int q3k_attn_part(const q3_att *p, void *stream);
+int q3k_attn_rows(const q3_att *p, void *stream); /* the same rows as q3k_attn_part + the chunk combine, bit for bit */
+int q3k_quant_rows(const q3_qr *p, void *stream);
 int q3k_attn_quant(const q3_aq *p, void *stream);
 int q3k_swiglu_quant(const q3_glu *p, void *stream);
 int q3k_argmax(const q3_amax *p, void *stream);

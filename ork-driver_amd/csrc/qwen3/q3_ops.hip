@@ -7,6 +7,7 @@
 //   k_norm_quant_*    [embedding lookup | residual add of a matmul result] + RMSNorm + per-row int8 quant
 //   k_qkv_post        q/k/v dequant + per-head RMSNorm (Qwen3 q_norm / k_norm) + RoPE + KV-cache append
 //   k_attn_part       causal GQA attention over one Q3_CHUNK-key chunk: running max, sum and P.V per query head
+//   k_attn_scores / k_attn_pv  the same rows for a prefill by blocks of rows (chunks combined in registers)
 //   k_attn_quant      combine the chunks (log-sum-exp) + per-row int8 quant of the attention output
 //   k_swiglu_quant    gate/up dequant + silu(g) * u + per-row int8 quant
 //   k_argmax          greedy sampling: dequantised logits -> one 64-bit atomic max per workgroup
@@ -17,6 +18,8 @@
 #include <hip/hip_fp16.h>
 #include <math.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "q3_ops.h"
 #include "orkh_rowops.h"
@@ -292,116 +295,198 @@ __global__ __launch_bounds__(256) void k_attn_part(q3_att p) {
     }
 }
 
-// k_attn_rows: the prefill form of k_attn_part (M > 1 rows, rotated queries in p.q): one workgroup per (kv head's
-// query-head group, key chunk, block of HD / Q3_CHUNK rows). The chunk's keys go to LDS and its values to registers
-// once and serve every row of the block, every thread scoring one (row, head, key), instead of one workgroup
-// reloading the chunk for each row. (Blocks of 16 rows measured slower, both as four such passes per workgroup and
-// with register-blocked scores -- each wave scoring four rows per K row read from LDS: the scoring is per-thread
-// latency, and 4x fewer workgroups left most CUs idle.) Each row's partials are computed with
-// k_attn_part's operations in its order (the score sums, the 32-lane max and sum, the P.V accumulation), and a row
-// with no key in the chunk gets k_attn_part's empty partial, so the partials are bit-identical to it.
-template <int GW>
-__global__ __launch_bounds__(256) void k_attn_rows(q3_att p) {
-    extern __shared__ float sm[];
-    const int HD = p.HD, G = p.NH / p.NKV, KVD = p.NKV * HD, QD = p.NH * HD;
-    const int nsub = G / GW, sub = blockIdx.x % nsub;
-    const int kvh = blockIdx.x / nsub, h0 = kvh * G + sub * GW; // first query head
-    const int s = blockIdx.y, tid = threadIdx.x;
-    const int g = tid / HD, d = tid - g * HD;
-    const int RR = HD / Q3_CHUNK; // rows per workgroup: GW * Q3_CHUNK * RR threads score them together
-    const int t0 = blockIdx.z * RR, t1 = min(t0 + RR, p.M); // rows t0 .. t1 - 1
-    const int j0 = s * Q3_CHUNK;
-    const int nmax = min(Q3_CHUNK, min(p.st[0] + t1, p.max_ctx) - j0); // keys of the block's last row
-    if (nmax <= 0) { // no row of the block reaches this chunk
-        for (int t = t0; t < t1; t++) {
-            float *out = p.part + (((size_t)t * p.NH + h0 + g) * p.S + s) * (HD + 2);
-            out[d] = 0.f;
-            if (d == 0) {
-                out[HD] = -INFINITY;
-                out[HD + 1] = 0.f;
-            }
-        }
-        return;
-    }
-    const int KS = HD + 4; // LDS row stride: 16-byte rows, 8 consecutive lanes of a float4 read hit distinct banks
-    float *Ks = sm;
-    float *qs = Ks + Q3_CHUNK * KS; // [RR][GW][HD]
-    float *P = qs + RR * GW * HD;   // [RR][GW][Q3_CHUNK]
-    float *ml = P + RR * GW * Q3_CHUNK; // [RR][GW][2]
-    const float *__restrict__ kb = p.kc + (size_t)j0 * KVD + kvh * HD;
-    const float *__restrict__ vb = p.vc + (size_t)j0 * KVD + kvh * HD + d;
-    float vv[Q3_CHUNK];
-#pragma unroll
-    for (int j = 0; j < Q3_CHUNK; j++) vv[j] = vb[(size_t)min(j, nmax - 1) * KVD];
-    const int HD4 = HD >> 2;
-    constexpr int KR = Q3_CHUNK / 4 / GW;
-    float4 kreg[KR];
-#pragma unroll
-    for (int k = 0; k < KR; k++) {
-        const int f = tid + k * blockDim.x, j = f / HD4, c4 = f - j * HD4;
-        kreg[k] = *(const float4 *)(kb + (size_t)min(j, nmax - 1) * KVD + 4 * c4);
-    }
-#pragma unroll
-    for (int k = 0; k < KR; k++) {
-        const int f = tid + k * blockDim.x, j = f / HD4, c4 = f - j * HD4;
-        *(float4 *)(Ks + j * KS + 4 * c4) = kreg[k];
-    }
-    for (int r0 = t0; r0 < t1; r0 += RR) {
-        for (int rr = 0; rr < RR; rr++) {
-            const int t = min(r0 + rr, t1 - 1);
-            qs[rr * GW * HD + tid] = p.q[(size_t)t * QD + h0 * HD + tid];
-        }
-        __syncthreads(); // keys (first pass) and this pass's queries
-        {   // scores: thread = (row rr, head gg, key j)
-            const int rr = tid / (GW * Q3_CHUNK), gg = (tid / Q3_CHUNK) % GW, j = tid % Q3_CHUNK;
-            const int t = r0 + rr;
-            const int n = min(Q3_CHUNK, min(p.st[0] + t + 1, p.max_ctx) - j0);
-            const float4 *qr = (const float4 *)(qs + (rr * GW + gg) * HD), *kr = (const float4 *)(Ks + j * KS);
-            float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
-#pragma unroll 8
-            for (int e = 0; e < HD4; e++) {
-                const float4 qv = qr[e], kv = kr[e];
-                a0 += qv.x * kv.x;
-                a1 += qv.y * kv.y;
-                a2 += qv.z * kv.z;
-                a3 += qv.w * kv.w;
-            }
-            const float sc = j < n ? ((a0 + a1) + (a2 + a3)) * p.scale : -INFINITY;
-            const float m = group_max<Q3_CHUNK>(sc);
-            const float pj = j < n ? expf(sc - m) : 0.f;
-            const float l = group_sum<Q3_CHUNK>(pj);
-            P[(rr * GW + gg) * Q3_CHUNK + j] = pj;
-            if (j == 0) {
-                ml[2 * (rr * GW + gg)] = m;
-                ml[2 * (rr * GW + gg) + 1] = l;
-            }
-        }
-        __syncthreads();
-        for (int rr = 0; rr < RR && r0 + rr < t1; rr++) {
-            const int t = r0 + rr;
-            float *out = p.part + (((size_t)t * p.NH + h0 + g) * p.S + s) * (HD + 2);
-            const int n = min(Q3_CHUNK, min(p.st[0] + t + 1, p.max_ctx) - j0);
-            if (n <= 0) { // k_attn_part's empty partial
-                out[d] = 0.f;
-                if (d == 0) {
-                    out[HD] = -INFINITY;
-                    out[HD + 1] = 0.f;
-                }
-                continue;
-            }
-            float acc = 0.f;
-#pragma unroll
-            for (int j = 0; j < Q3_CHUNK; j++) acc += P[(rr * GW + g) * Q3_CHUNK + j] * vv[j];
-            out[d] = acc;
-            if (d == 0) {
-                out[HD] = ml[2 * (rr * GW + g)];
-                out[HD + 1] = ml[2 * (rr * GW + g) + 1];
-            }
-        }
-        __syncthreads(); // this pass's P and queries read before the next pass writes them
+// Prefill attention (M > 1 rows, rotated queries in p.q): scores and softmax terms of every (row, query head, key) by
+// k_attn_scores, then P.V and the chunk combine in registers by k_attn_pv, with k_attn_part's and attn_quant_body's
+// operations in their order (the four score sums, the 32-key chunk's max and sum, the chunk's P.V accumulation over
+// ascending keys, the log-sum-exp combine over ascending chunks), so the rows are bit-identical to the row-by-row
+// kernels'. Both are bound by the VALU: mul and add round separately (no FMA), 4 * HD operations per (row, head, key).
+// What the split is for: the operand that the lanes share (16 dimensions of a query row, 16 of a row's probabilities)
+// sits in one register and is broadcast by the multiply itself, the other comes from registers or one LDS read per 16
+// products, and only the probabilities cross HBM (4 bytes per score), where one workgroup per (32-key chunk, 4 rows)
+// wrote every chunk's P.V row (HD + 2 floats) and a combine launch read it back. Per layer at Qwen3-1.7B widths,
+// traced, that form -> this one (with the row quantisation): M=1000 295 -> 184 us, M=500 81 -> 68; whole prefills of
+// two layers M=64 168 -> 161, M=128 188 -> 180, M=256 236 -> 228, M=500 377 -> 353, M=700 574 -> 461, M=1000 855 -> 634.
+// At M=1000 the mul / add pairs alone take 104 us at the VALU's rate.
+// Lane N of each 16-lane row, in every lane of the row: folded into the multiply that uses it (a DPP operand).
+template <int N> __device__ __forceinline__ float bc16(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x150 + N, 0xF, 0xF, true));
+}
+template <int I, int N, typename F> __device__ __forceinline__ void static_for(F &&f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<I + 1, N>(f);
     }
 }
 
+// k_attn_scores: grid (NKV, 64-key tiles, blocks of p.sr rows), 4 waves. The tile's keys are staged in LDS as
+// [HD / 4][64] float4 (lane = key: one conflict-free 128-bit read per four dimensions); a wave scores four (row, head)
+// pairs at a time against all 64 keys, 16 dimensions of a query row in one register (lane % 16) and broadcast by the
+// multiply. Each half wave is a 32-key chunk: its max, exp and sum are one lane-group reduction. Writes
+// P = exp(s - chunk max), 0 past the row's keys.
+// padded so that the stores of one key's float4s fall in different banks, where that fits 64 KiB
+__host__ __device__ constexpr int q3_kt_row(int hd) { return hd < 256 ? 65 : 64; }
+template <int HD> __global__ __launch_bounds__(256) void k_attn_scores(q3_att p) {
+    extern __shared__ float4 Kt[]; // [HD / 4][KR]
+    constexpr int KR = q3_kt_row(HD), HD4 = HD / 4, NQ = HD / 16;
+    const int G = p.NH / p.NKV, KVD = p.NKV * HD, QD = p.NH * HD;
+    const int kvh = blockIdx.x, j0 = blockIdx.y * 64, t0 = blockIdx.z * p.sr;
+    const int t1 = min(t0 + p.sr, p.M);
+    const int nmax = min(64, t1 - j0); // keys of the block's last row
+    if (nmax <= 0) return; // no row of the block reaches this tile (k_attn_pv does not read it either)
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int LP = (p.M + 63) & ~63; // row stride of P
+    const int npair = (t1 - t0) * G;       // (row, head) pairs of the block: u = row * G + head
+    const float *__restrict__ kb = p.kc + (size_t)j0 * KVD + kvh * HD;
+#pragma unroll
+    for (int f0 = 0; f0 < 64 * HD4; f0 += 256) {
+        const int f = f0 + threadIdx.x, j = f / HD4, c = f - j * HD4;
+        Kt[c * KR + j] = *(const float4 *)(kb + (size_t)min(j, nmax - 1) * KVD + 4 * c);
+    }
+    __syncthreads();
+    for (int u0 = wv * 4; u0 < npair; u0 += 16) {
+        if (t0 + min(u0 + 3, npair - 1) / G < j0) continue; // the four rows end before this tile
+        const float *__restrict__ qr[4];
+        float a[4][4], q[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int u = min(u0 + i, npair - 1), r = u / G;
+            qr[i] = p.q + (size_t)(t0 + r) * QD + (kvh * G + u - r * G) * HD + (lane & 15);
+            q[i] = qr[i][0];
+#pragma unroll
+            for (int x = 0; x < 4; x++) a[i][x] = 0.f;
+        }
+        float4 k[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) k[c] = Kt[c * KR + lane];
+#pragma unroll 2
+        for (int x = 0; x < NQ; x++) { // 16 dimensions; the next 16 are requested before this one's products
+            const int xn = min(x + 1, NQ - 1);
+            float qn[4];
+            float4 kn[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) qn[i] = qr[i][16 * xn];
+#pragma unroll
+            for (int c = 0; c < 4; c++) kn[c] = Kt[(4 * xn + c) * KR + lane];
+            __builtin_amdgcn_sched_barrier(0);
+            static_for<0, 4>([&](auto oc) {
+                constexpr int c = decltype(oc)::value, o = 4 * c;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    a[i][0] += bc16<o>(q[i]) * k[c].x;
+                    a[i][1] += bc16<o + 1>(q[i]) * k[c].y;
+                    a[i][2] += bc16<o + 2>(q[i]) * k[c].z;
+                    a[i][3] += bc16<o + 3>(q[i]) * k[c].w;
+                }
+            });
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) q[i] = qn[i], k[i] = kn[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int u = u0 + i;
+            if (u >= npair) break; // wave-uniform
+            const int r = u / G, t = t0 + r, h = kvh * G + u - r * G;
+            const bool in = j0 + lane <= t; // causal
+            const float sc = in ? ((a[i][0] + a[i][1]) + (a[i][2] + a[i][3])) * p.scale : -INFINITY;
+            const float m = group_max<Q3_CHUNK>(sc);
+            const float pj = in ? expf(sc - m) : 0.f;
+            const float l = group_sum<Q3_CHUNK>(pj);
+            const size_t th = (size_t)t * p.NH + h;
+            p.sc[th * LP + j0 + lane] = pj;
+            const int c = (j0 + lane) / Q3_CHUNK;
+            if (lane % Q3_CHUNK == 0 && c < p.S) {
+                p.ml[(th * p.S + c) * 2] = m;
+                p.ml[(th * p.S + c) * 2 + 1] = l;
+            }
+        }
+    }
+}
+
+// k_attn_pv: grid (NKV, groups of PW (row, head) pairs, the last rows' first: they have the most keys), HD threads: thread
+// d = dimension d. A wave keeps 32 keys' V of its 64 dimensions in registers and runs them against its pairs,
+// whose probabilities sit 16 to a register and are broadcast by the multiply; the chunk's row is scaled by its
+// log-sum-exp weight and added to the pair's running row, so no chunk result leaves the registers.
+template <int PW> __global__ __launch_bounds__(Q3_MAX_HD) void k_attn_pv(q3_att p) {
+    static_assert(Q3_CHUNK == 32 && Q3_MAX_S <= 64, "a chunk per lane, 32 keys in registers");
+    const int HD = p.HD, G = p.NH / p.NKV, KVD = p.NKV * HD, QD = p.NH * HD, S = p.S;
+    const int kvh = blockIdx.x, npair = p.M * G, u0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * PW;
+    const int lane = threadIdx.x & 63, d = threadIdx.x;
+    const int LP = (p.M + 63) & ~63;
+    struct chunk_in {
+        float v[Q3_CHUNK], w[PW][2]; // V of 32 keys, and the pairs' probabilities
+    };
+    int L[PW];
+    size_t th[PW], orow[PW];
+#pragma unroll
+    for (int i = 0; i < PW; i++) {
+        const int u = min(u0 + i, npair - 1), t = u / G, h = kvh * G + u - t * G;
+        th[i] = (size_t)t * p.NH + h;
+        L[i] = t + 1;
+        orow[i] = (size_t)t * QD + h * HD;
+    }
+    const int Lm = L[PW - 1], ns = (Lm + Q3_CHUNK - 1) / Q3_CHUNK; // rows ascend: the most keys
+    const float *__restrict__ vb = p.vc + kvh * HD + d;
+    auto load = [&](int s, chunk_in &x) { // keys past the last row's repeat its last (probability 0)
+#pragma unroll
+        for (int i = 0; i < PW; i++) { // a pair whose keys end earlier reads its last chunk again and skips it
+            const float *__restrict__ w = p.sc + th[i] * LP + min(s, (L[i] - 1) / Q3_CHUNK) * Q3_CHUNK + (lane & 15);
+            x.w[i][0] = w[0];
+            x.w[i][1] = w[16];
+        }
+#pragma unroll
+        for (int j = 0; j < Q3_CHUNK; j++) x.v[j] = vb[(size_t)min(s * Q3_CHUNK + j, Lm - 1) * KVD];
+    };
+    chunk_in x[2];
+    float e[PW], inv[PW], num[PW], m0[PW], l0[PW]; // e: the weight of chunk `lane`
+#pragma unroll
+    for (int i = 0; i < PW; i++) {
+        const int c = min(lane, (L[i] - 1) / Q3_CHUNK); // chunks with a key of the row
+        m0[i] = p.ml[(th[i] * S + c) * 2];
+        l0[i] = p.ml[(th[i] * S + c) * 2 + 1];
+    }
+    load(0, x[0]);
+#pragma unroll
+    for (int i = 0; i < PW; i++) {
+        const bool has = lane <= (L[i] - 1) / Q3_CHUNK;
+        const float m = has ? m0[i] : -INFINITY;
+        const float mx = wave_max(m);
+        e[i] = m == -INFINITY ? 0.f : expf(m - mx);
+        const float den = wave_sum(has ? l0[i] * e[i] : 0.f);
+        inv[i] = den > 0.f ? 1.0f / den : 0.f;
+        num[i] = 0.f;
+    }
+    auto chunk = [&](int s, const chunk_in &x) {
+#pragma unroll
+        for (int i = 0; i < PW; i++) {
+            if (s * Q3_CHUNK >= L[i]) continue; // wave-uniform: no key of this row
+            float acc = 0.f;
+            static_for<0, Q3_CHUNK>([&](auto jc) {
+                constexpr int j = decltype(jc)::value;
+                acc += bc16<j % 16>(x.w[i][j / 16]) * x.v[j];
+            });
+            num[i] += acc * __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, e[i]), s));
+        }
+    };
+    for (int s = 0; s < ns; s += 2) { // the next chunk's values are requested before this one's products
+        if (s + 1 < ns) load(s + 1, x[1]);
+        chunk(s, x[0]);
+        if (s + 1 < ns) {
+            if (s + 2 < ns) load(s + 2, x[0]);
+            chunk(s + 1, x[1]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < PW; i++)
+        if (u0 + i < npair) p.o[orow[i] + d] = num[i] * inv[i];
+}
+
+// fp32 rows -> int8 rows (the attention rows of a prefill)
+template <int E> __global__ __launch_bounds__(1024) void k_quant_rows(q3_qr p) {
+    float y[E];
+    load_row(y, p.y + (size_t)blockIdx.x * p.n, p.n);
+    quant_regs(y, p.n, p.a8 + (size_t)blockIdx.x * p.n, p.as + blockIdx.x);
+}
 
 // Combine the chunks of every head (log-sum-exp weights), then quantise the row. Each thread's partial
 // sums are loaded before the chunk weights are known, so the kernel pays one round trip to memory.
@@ -600,17 +685,6 @@ int q3k_attn_part(const q3_att *p, void *stream) {
     const dim3 grid(p->NKV * (G / GW), p->S, p->M), block(GW * p->HD);
     const hipStream_t st = (hipStream_t)stream;
     const bool fused = p->cq != nullptr;
-    if (!fused && p->rows) { // prefill: the chunk once per block of rows
-        const size_t lr = (size_t)(Q3_CHUNK * (p->HD + 4) + (p->HD / Q3_CHUNK) * GW * (p->HD + Q3_CHUNK + 2)) * 4;
-        const int rr = p->HD / Q3_CHUNK;
-        const dim3 gr(p->NKV * (G / GW), p->S, (p->M + rr - 1) / rr);
-        if (lr > 64 * 1024) return -2;
-        if (GW == 1) hipLaunchKernelGGL((k_attn_rows<1>), gr, block, lr, st, *p);
-        else if (GW == 2) hipLaunchKernelGGL((k_attn_rows<2>), gr, block, lr, st, *p);
-        else if (GW == 4) hipLaunchKernelGGL((k_attn_rows<4>), gr, block, lr, st, *p);
-        else return -2;
-        return launch_ok();
-    }
     if (GW == 1) {
         if (fused) hipLaunchKernelGGL((k_attn_part<1, true>), grid, block, lds, st, *p);
         else hipLaunchKernelGGL((k_attn_part<1, false>), grid, block, lds, st, *p);
@@ -623,6 +697,39 @@ int q3k_attn_part(const q3_att *p, void *stream) {
     } else {
         return -2;
     }
+    return launch_ok();
+}
+
+int q3k_attn_rows(const q3_att *p, void *stream) {
+    const int G = p->NKV > 0 ? p->NH / p->NKV : 0;
+    if (p->M < 1 || G < 1 || G * p->NKV != p->NH || p->HD % 64 || p->HD < 64 || p->HD > Q3_MAX_HD || p->S < 1 ||
+        p->S > Q3_MAX_S || (long)p->S * Q3_CHUNK < p->M || !p->q || !p->sc || !p->ml || !p->o)
+        return -2;
+    const hipStream_t st = (hipStream_t)stream;
+    /* A scores workgroup takes the rows whose pairs are one quad a wave, and a P.V wave two pairs up to 256 rows, else
+     * four: with few rows the waves' chains are the time, with many their reads of V. Whole prefills of two layers at
+     * Qwen3-1.7B widths (16 heads, 8 kv heads; us): M=128 4 / 8 / 16 / 32 rows 200 / 197 / 202 / 219, M=1000 730 / 658
+     * / 658 / 666; two / four pairs M=128 196.7 / 198.9, M=256 245.0 / 249.3, M=384 298.2 / 297.6, M=1000 719 / 658. */
+    const int pw = p->M <= 256 ? 2 : 4;
+    const long groups = ((long)p->M * G + pw - 1) / pw;
+    q3_att a = *p;
+    a.sr = G >= 16 ? 1 : 16 / G;
+    const dim3 grid(p->NKV, (p->M + 63) / 64, (p->M + a.sr - 1) / a.sr);
+    const size_t lds = (size_t)(p->HD / 4) * q3_kt_row(p->HD) * 16;
+    if (lds > 64 * 1024 || groups > 65535) return -2;
+    if (p->HD == 64) hipLaunchKernelGGL(k_attn_scores<64>, grid, dim3(256), lds, st, a);
+    else if (p->HD == 128) hipLaunchKernelGGL(k_attn_scores<128>, grid, dim3(256), lds, st, a);
+    else if (p->HD == 192) hipLaunchKernelGGL(k_attn_scores<192>, grid, dim3(256), lds, st, a);
+    else hipLaunchKernelGGL(k_attn_scores<256>, grid, dim3(256), lds, st, a);
+    if (launch_ok()) return -1;
+    if (pw == 2) hipLaunchKernelGGL(k_attn_pv<2>, dim3(p->NKV, (unsigned)groups), dim3(p->HD), 0, st, *p);
+    else hipLaunchKernelGGL(k_attn_pv<4>, dim3(p->NKV, (unsigned)groups), dim3(p->HD), 0, st, *p);
+    return launch_ok();
+}
+
+int q3k_quant_rows(const q3_qr *p, void *stream) {
+    if (p->M < 1 || p->n < 1 || p->n > 1024 * 16) return -2;
+    Q3_ROW_DISPATCH(k_quant_rows, 1024, p->n, dim3(p->M), 0, (hipStream_t)stream, *p);
     return launch_ok();
 }
 

@@ -151,6 +151,35 @@ def test_fused_decode_equals_unfused(npu, case):
     assert np.array_equal(out[0][1], out[1][1])
 
 
+@pytest.mark.parametrize("case", [
+    dict(name="gqa2-hd128", over={}, n=(2, 31, 33, 64, 65, 127, 300)),
+    dict(name="gqa4-hd64", over=dict(heads=8, kv_heads=2, head_dim=64), n=(3, 32, 97, 257)),
+    dict(name="mha-hd128", over=dict(heads=2, kv_heads=2), n=(17, 66)),
+    dict(name="gqa3-hd192", over=dict(heads=3, kv_heads=1, head_dim=192), n=(5, 70)),
+    dict(name="gqa2-hd256", over=dict(heads=2, kv_heads=1, head_dim=256), n=(63, 130)),
+])
+def test_prefill_attention_by_blocks_equals_rows(npu, case):
+    """Prefill attention by blocks of rows against row by row, at the edges of the key tiles (64), the chunks (32), the
+    row blocks (16) and the (row, head) quads: every layer's rows and the logits bit for bit (the same float operations
+    in the same order)."""
+    _say("prefill rows", case["name"])
+    cfg = _cfg(max_ctx=320, max_rows=max(case["n"]), **case["over"])
+    W, Nm = _weights(cfg, 61)
+    m = _model(npu, cfg, W, Nm)
+    try:
+        assert m.set_trace(1) == 0
+        for n in case["n"]:
+            prompt = np.random.default_rng(67 + n).integers(0, cfg.vocab, n).astype(np.int32)
+            out = []
+            for fused in (0, 1):
+                assert m.set_fused(fused) == 0 and m.prefill(prompt) == 0
+                out.append([m.last_logits()] + [m.layer_rows(l, n) for l in range(cfg.layers + 1)])
+            for a, b in zip(*out):
+                assert np.array_equal(a, b), n
+    finally:
+        m.close()
+
+
 def test_second_prefill_restarts(npu):
     _say("second prefill")
     cfg = _cfg()
