@@ -89,7 +89,7 @@ int         orkh_stream_capturing(void *stream);
 int         orkh_ptr_is_device(const void *p);
 
 /* ---- matmul launch ---- */
-enum { ORKH_ALGO_STREAM = 0, ORKH_ALGO_TILED = 1, ORKH_ALGO_GEMV = 2, ORKH_ALGO_TILED2 = 3 };
+enum { ORKH_ALGO_STREAM = 0, ORKH_ALGO_TILED = 1, ORKH_ALGO_GEMV = 2, ORKH_ALGO_TILED2 = 3, ORKH_ALGO_BIG = 4 };
 
 /* One C[M][N] = A[M][K] x B[K][N] launch on resident panels. A is row-major with row stride lda
  * elements (int8 for the integer kinds, fp16 for ORKH_F16); C is row-major int32 (integer kinds) or
@@ -112,7 +112,7 @@ typedef struct orkh_mm {
 
 /* Launch plan chosen by the host planner (ork-driver_amd/csrc/host/plan.c). */
 typedef struct orkh_plan {
-    int algo;             /* ORKH_ALGO_STREAM | ORKH_ALGO_TILED | ORKH_ALGO_GEMV | ORKH_ALGO_TILED2 */
+    int algo;             /* ORKH_ALGO_STREAM | ORKH_ALGO_TILED | ORKH_ALGO_GEMV | ORKH_ALGO_TILED2 | ORKH_ALGO_BIG */
     /* GEMV (M = 1 only): the STREAM grid and fields below, VALU dot products instead of MFMA.
      * STREAM: grid (N/16, ksplit), wpg waves per workgroup, each wave kbw K-blocks of one panel,
      * mt = ceil(M/16) row tiles (1..4). ksplit > 1 writes partials to ws and adds a reduce pass. */
@@ -124,7 +124,8 @@ typedef struct orkh_plan {
     int aline;
     /* TILED2: 2 = a two-slot ring (two workgroups per CU on the tiles whose 4-slot ring fills one), else 0 */
     int ring;
-    /* TILED2: 1 = write-through C stores, else write-back */
+    /* BIG (many rows, orkh_big.hip): bm x bn of 256 x 256, 256 x 192, 128 x 256, 128 x 192; never K-split */
+    /* TILED2 and BIG: 1 = write-through C stores, else write-back */
     int cwt;
     /* STREAM: np = 2 pairs panels: npg workgroups, the first N/16 - npg owning two adjacent panels each */
     int np, npg;
@@ -137,9 +138,12 @@ typedef struct orkh_plan {
 int orkh_mm_launch(const orkh_mm *p, const orkh_plan *plan, void *stream);
 
 /* Grouped tiled launch (multi-matmul submit, M > 1): n (2..ORKH_TGROUP_MAX) matmuls of one kind, one M and one K in
- * a single k_tiled2 launch under one plan (algo ORKH_ALGO_TILED2, ksplit 1: the tile the planner picks for their
+ * a single k_tiled2 or k_big launch under one plan (algo ORKH_ALGO_TILED2 or ORKH_ALGO_BIG, ksplit 1: the tile the planner picks for their
  * columns together); each matmul keeps its own A, B, C, N and ldc. 0 / -2 inconsistent tasks or plan / -1 HIP. */
 #define ORKH_TGROUP_MAX 8
+/* The ORKH_ALGO_BIG launch of 1, or 2..ORKH_TGROUP_MAX, such matmuls (orkh_big.hip; called by the two above and below,
+ * which check them). */
+int orkh_big_launch(const orkh_mm *p, int n, const orkh_plan *plan, void *stream);
 int orkh_mm_launch_tgroup(const orkh_mm *p, int n, const orkh_plan *plan, void *stream);
 
 /* Grouped M = 1 launch (multi-matmul submit): n independent GEMVs of one kind (p.kind equal, p.M == 1)

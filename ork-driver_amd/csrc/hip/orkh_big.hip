@@ -1,0 +1,328 @@
+// orkh_big.hip -- the tiled MFMA kernel for many rows (long prompts, batched prefill): 128- and 256-row tiles, every
+// weight kind.
+//
+// k_big: one workgroup per BM x BN output tile. Like k_tiled2 (orkh_kernels.hip) it brings both operands HBM/L2 -> LDS
+// with direct-to-LDS loads into a ring of stages and reads MFMA operands from there; what differs is what a large grid
+// needs. Bound by operand delivery to the CUs (an L1's outstanding requests to L2 pass ~22-25 bytes per clock and CU),
+// then by MFMA:
+//  - tiles of up to 256 x 256, so that a byte delivered to a CU feeds up to 256 multiply-accumulates, in four shapes so
+//    that a grid fills its last round of the CUs (256 x 192 takes K=2048 N=6144 M=4096 in two full rounds where
+//    256 x 256 takes one and a half);
+//  - stages of 128 activation bytes a row (whole cache lines, a_lds's swizzle) and one barrier per stage, with the
+//    next phase's LDS operands read into registers before the current phase's MFMAs;
+//  - load addresses as one per-lane offset plus a scalar stage offset, so a load costs one instruction;
+//  - an XCD's run of tiles covers GM rows of tiles x several columns instead of one column of all rows, so its L2 takes
+//    about a third less from the next level;
+//  - the MFMA operands swapped (D = B^T A^T), so that a lane holds four consecutive columns of one row and C goes out
+//    16 bytes a store;
+//  - int4 blocks decoded in registers by 8 waves of 128 x 64 (two decodes per block), int8 and fp16 on 16 waves.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+#include <stdio.h>
+#include <string.h>
+
+#include <type_traits>
+
+#include "orkh_dev.h"
+
+namespace {
+
+template <int KIND, int BM, int BN> struct BG {
+    using T = KT<KIND>;
+    static constexpr bool NIB = KIND == ORKH_I4U || KIND == ORKH_NF4;
+    static constexpr int NW = NIB ? 8 : 16, WM = NIB ? 2 : 4, WN = 4;
+    static constexpr int MTW = BM / 16 / WM, NTW = BN / 16 / WN; // 16 x 16 blocks per wave
+    static constexpr int MHN = MTW >= 4 ? 2 : 1, MH = MTW / MHN; // a phase: one K step x MH row blocks
+    static constexpr int BPP = NIB ? 1 : 2;                      // panel blocks per panel and stage
+    static constexpr int NA = BM / 8, NL = NA + BN / 16 * BPP;   // 1 KiB loads per stage: 8 rows of A, or one block
+    static constexpr int LPW = (NL + NW - 1) / NW;               // per wave; a last one without work lands in a junk block
+    static constexpr int SLOT = (NL + (LPW * NW > NL)) * 64;     // 16-byte units
+    static constexpr int RMAX = 163840 / (SLOT * 16), R = RMAX < 4 ? RMAX : 4;
+    static constexpr int LDS = R * SLOT * 16;
+    static constexpr int GM = 1024 / BM; // tile rows of an XCD's run: 1024 rows
+    static_assert(R >= 2 && MTW * WM * 16 == BM && NTW * WN * 16 == BN && MH * MHN == MTW, "tile");
+};
+
+// MFMA operand of K step kk from a lane's panel chunk (nibble kinds: half the chunk per step, as decode())
+template <int KIND> __device__ __forceinline__ v4i step_op(v4i raw, int kk, const Lut &L) {
+    const uint32_t x = kk ? raw.z : raw.x, y = kk ? raw.w : raw.y;
+    if constexpr (KIND == ORKH_I4U) {
+        return v4i{(int)((x << 4) & 0xf0f0f0f0u), (int)(x & 0xf0f0f0f0u), (int)((y << 4) & 0xf0f0f0f0u), (int)(y & 0xf0f0f0f0u)};
+    } else {
+        uint32_t a, b, c, d;
+        nf4_map8(x, L, a, b);
+        nf4_map8(y, L, c, d);
+        return v4i{(int)a, (int)b, (int)c, (int)d};
+    }
+}
+
+// Direct-to-LDS load at a per-lane offset plus a scalar one (the range check covers the per-lane offset only: a lane
+// whose sum would leave the resource carries OOB)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void lds_dma16s(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, uint32_t lds_byte) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_byte), "v"(voff), "s"(r),
+                 "s"(soff)
+                 : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+template <int KIND, int BM, int BN>
+__device__ __forceinline__ void big_body(const orkh_mm &p, int mtiles, int ntiles, int bid) {
+    using T = KT<KIND>;
+    using P = BG<KIND, BM, BN>;
+    typedef typename T::acc_t acc_t;
+    typedef typename T::c_t c_t;
+    constexpr int R = P::R, LPW = P::LPW, NW = P::NW, NA = P::NA;
+    extern __shared__ v4i sm[];
+    // every kernel argument in one batch of scalar loads behind one wait (as tiled2_body)
+    asm volatile("" ::"s"(p.M), "s"(p.K), "s"(p.N), "s"(p.KB), "s"(p.lda), "s"(p.A), "s"(p.B), "s"(p.C), "s"(p.ldc),
+                 "s"(p.c_wt), "s"(mtiles), "s"(ntiles));
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wv % P::WM, wn = wv / P::WM;
+    // XCD-aware order: workgroup b runs on XCD b % 8, each XCD a contiguous run of tiles; runs go down GM tile rows at a
+    // time, M fastest, so that a run is about as many rows of A as columns of B
+    const int nT = mtiles * ntiles, per = nT / 8, rem = nT % 8, x = bid % 8, j = bid / 8;
+    const int tl = x < rem ? x * (per + 1) + j : rem * (per + 1) + (x - rem) * per + j;
+    int g, in, tn, tm;
+    udivmod(tl, P::GM * ntiles, g, in);
+    const int gm = min(mtiles - g * P::GM, P::GM);
+    udivmod(in, gm, tn, tm);
+    const int m0 = (g * P::GM + tm) * BM, nb0 = tn * (BN / 16), NBt = p.N / 16;
+    const uint32_t lda_b = (uint32_t)p.lda * T::ESZ, kbytes = (uint32_t)p.K * T::ESZ;
+    const __amdgpu_buffer_rsrc_t Ar = make_rsrc(p.A, (uint32_t)p.M * lda_b);
+    const __amdgpu_buffer_rsrc_t Br = make_rsrc(p.B, (uint32_t)NBt * p.KB * 1024u);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)sm;
+    const Lut L = {p.lut[0], p.lut[1], p.lut[2], p.lut[3]};
+
+    // this wave's loads: i = wv + q * NW; rows 8 i .. 8 i + 7 of A (lane l: row l / 8, slot l % 8 holds chunk
+    // slot ^ (l / 8) ^ (i & 1)), or panel block i - NA
+    uint32_t vo[LPW];
+#pragma unroll
+    for (int q = 0; q < LPW; q++) {
+        const int i = wv + q * NW, ib = i - NA;
+        const int row = m0 + i * 8 + (lane >> 3), nb = nb0 + ib / P::BPP;
+        if (i < NA) vo[q] = row < p.M ? (uint32_t)row * lda_b + (uint32_t)(((lane & 7) ^ (lane >> 3) ^ (i & 1)) * 16) : OOB;
+        else vo[q] = i < P::NL && nb < NBt ? ((uint32_t)nb * p.KB + ib % P::BPP) * 1024u + lane * 16u : OOB;
+    }
+    const int nst = (p.KB + P::BPP - 1) / P::BPP;
+    auto issue = [&](int st) {
+        if (st >= nst) return;
+        const uint32_t slot = lds0 + (uint32_t)(st % R) * (P::SLOT * 16);
+        const bool tail = (uint32_t)st * 128 + 128 > kbytes; // the last stage of a K that is not whole stages
+#pragma unroll
+        for (int q = 0; q < LPW; q++) {
+            const int i = wv + q * NW;
+            uint32_t v = vo[q];
+            if (tail) { // A chunks and panel blocks past K read zeros
+                const uint32_t c = (uint32_t)(((lane & 7) ^ (lane >> 3) ^ (i & 1)) * 16);
+                if (i < NA ? (uint32_t)st * 128 + c >= kbytes : st * P::BPP + (i - NA) % P::BPP >= p.KB) v = OOB;
+            }
+            if (i < NA) lds_dma16s(Ar, v, (uint32_t)st * 128, slot + i * 1024);
+            else lds_dma16s(Br, v, (uint32_t)st * (P::BPP * 1024), slot + min(i, P::NL) * 1024);
+        }
+    };
+
+    acc_t acc[P::MTW][P::NTW];
+#pragma unroll
+    for (int a = 0; a < P::MTW; a++)
+#pragma unroll
+        for (int b = 0; b < P::NTW; b++) acc[a][b] = acc_t{0, 0, 0, 0};
+    // A operand of (row block mb, step kk): chunk c of row lane % 16, at (mb * 2 + h) * 64 + r7 * 8 + (c ^ r7 ^ h)
+    const int h = (lane >> 3) & 1, r7 = lane & 7;
+    const int c0 = P::NIB ? (lane >> 4) * 2 : lane >> 4, c1 = P::NIB ? c0 + 1 : c0 + 4;
+    const int ao0 = h * 64 + r7 * 8 + (c0 ^ r7 ^ h), ao1 = h * 64 + r7 * 8 + (c1 ^ r7 ^ h);
+    v4i a[2][P::MH], b[2][P::NTW], raw[P::NIB ? P::NTW : 1];
+    auto rdA = [&](int st, int kk, int hh, v4i (&d)[P::MH]) {
+        const v4i *As = sm + (st % R) * P::SLOT + (wm * P::MTW + hh * P::MH) * 128 + (kk ? ao1 : ao0);
+#pragma unroll
+        for (int i = 0; i < P::MH; i++) d[i] = As[i * 128];
+    };
+    auto rdB = [&](int st, int kk) { // nibble kinds: the stage's chunks (kk = 0), decoded by opB
+        const v4i *Bs = sm + (st % R) * P::SLOT + NA * 64 + (wn * P::NTW * P::BPP + kk) * 64 + lane;
+#pragma unroll
+        for (int i = 0; i < P::NTW; i++) {
+            if constexpr (P::NIB) raw[i] = Bs[i * 64];
+            else b[kk][i] = Bs[i * 128];
+        }
+    };
+    auto opB = [&](int kk) {
+        if constexpr (P::NIB) {
+#pragma unroll
+            for (int i = 0; i < P::NTW; i++) b[kk][i] = step_op<KIND>(raw[i], kk, L);
+        }
+    };
+    auto mm = [&](int hh, const v4i (&xa)[P::MH], const v4i (&xb)[P::NTW]) {
+#pragma unroll
+        for (int i = 0; i < P::MH; i++)
+#pragma unroll
+            for (int jn = 0; jn < P::NTW; jn++) acc[hh * P::MH + i][jn] = mma(xb[jn], xa[i], acc[hh * P::MH + i][jn]);
+    };
+    // keeps each phase's LDS reads in front of its MFMAs
+    auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
+
+#pragma unroll
+    for (int st = 0; st < R; st++) issue(st);
+    if (nst >= R) wait_vmcnt<(R - 1) * LPW>();
+    else wait_vmcnt<0>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    rdB(0, 0);
+    rdA(0, 0, 0, a[0]);
+    opB(0);
+    for (int s = 0; s < nst; s++) {
+        if constexpr (P::MHN == 2) {
+            rdA(s, 0, 1, a[1]);
+            fence();
+            mm(0, a[0], b[0]);
+            fence();
+            if constexpr (!P::NIB) rdB(s, 1);
+            rdA(s, 1, 0, a[0]);
+            opB(1);
+            fence();
+            mm(1, a[1], b[0]);
+            fence();
+            rdA(s, 1, 1, a[1]);
+            fence();
+            mm(0, a[0], b[1]);
+            fence();
+        } else {
+            if constexpr (!P::NIB) rdB(s, 1);
+            rdA(s, 1, 0, a[1]);
+            opB(1);
+            fence();
+            mm(0, a[0], b[0]);
+            fence();
+        }
+        // Stage s + 1 has landed (this wave's share of it; the barrier covers the others'), and every wave's reads of
+        // stage s are done, so its slot takes stage s + R
+        if (s + R <= nst) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"((R - 2) * LPW) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        issue(s + R);
+        if (s + 1 < nst) {
+            rdB(s + 1, 0);
+            rdA(s + 1, 0, 0, a[0]);
+        }
+        fence();
+        mm(P::MHN - 1, a[1], b[1]);
+        fence();
+        opB(0); // (after the last stage: of what it holds, unused)
+    }
+
+    // a lane holds row lane % 16, columns 4 (lane / 16) .. + 3 of each block
+    const int n0 = (nb0 + wn * P::NTW) * 16 + (lane >> 4) * 4;
+    const bool vec = p.ldc % 4 == 0 && ((uintptr_t)p.C & 15) == 0;
+#pragma unroll
+    for (int i = 0; i < P::MTW; i++) {
+        const int m = m0 + (wm * P::MTW + i) * 16 + (lane & 15);
+        if (m >= p.M) continue;
+        c_t *Cr = (c_t *)p.C + (size_t)m * p.ldc + n0;
+#pragma unroll
+        for (int jn = 0; jn < P::NTW; jn++) {
+            if (nb0 + wn * P::NTW + jn >= NBt) continue;
+            acc_t o = acc[i][jn];
+#pragma unroll
+            for (int r = 0; r < 4; r++) o[r] = finish<KIND>(o[r]);
+            c_t *dst = Cr + jn * 16;
+            if (vec) {
+                if (p.c_wt) store_wt4(dst, __builtin_bit_cast(v4i, o));
+                else *(acc_t *)dst = o;
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    if (p.c_wt) store_wt(&dst[r], o[r]);
+                    else dst[r] = o[r];
+                }
+            }
+        }
+    }
+}
+
+template <int KIND, int BM, int BN>
+__global__ __launch_bounds__((BG<KIND, BM, BN>::NW * 64), 1) void k_big(orkh_mm p, int mtiles, int ntiles) {
+    big_body<KIND, BM, BN>(p, mtiles, ntiles, (int)blockIdx.x);
+}
+
+// k_bigm: up to ORKH_TGROUP_MAX matmuls of one kind, M and K in one launch (the multi-matmul submit), as k_tiled2m: task
+// t's tiles are workgroups [wg0[t], wg0[t] + tiles), each start a multiple of 8; the padding workgroups exit at once.
+struct BigMulti {
+    int n, mtiles;
+    int wg0[ORKH_TGROUP_MAX], ntiles[ORKH_TGROUP_MAX];
+    orkh_mm p[ORKH_TGROUP_MAX];
+};
+template <int KIND, int BM, int BN>
+__global__ __launch_bounds__((BG<KIND, BM, BN>::NW * 64), 1) void k_bigm(BigMulti g) {
+    int t = 0;
+    while (t + 1 < g.n && (int)blockIdx.x >= g.wg0[t + 1]) t++;
+    const int local = (int)blockIdx.x - g.wg0[t];
+    if (local >= g.mtiles * g.ntiles[t]) return;
+    big_body<KIND, BM, BN>(g.p[t], g.mtiles, g.ntiles[t], local);
+}
+
+template <int KIND, int BM, int BN> int launch(const orkh_mm *p, int n, const orkh_plan *q, hipStream_t s) {
+    using P = BG<KIND, BM, BN>;
+    static lds_flags attr[2];
+    const int mtiles = (p->M + BM - 1) / BM;
+    if (n == 1) {
+        const int ntiles = (p->N + BN - 1) / BN;
+        if ((long)mtiles * ntiles >= (1L << 24)) { // the kernel's tile-index division is exact below 2^24
+            snprintf(g_lerr, sizeof g_lerr, "big: %ld workgroups", (long)mtiles * ntiles);
+            return -2;
+        }
+        auto kern = k_big<KIND, BM, BN>;
+        if (lds_limit((const void *)kern, P::LDS, attr[0])) return -1;
+        orkh_mm pc = *p;
+        pc.c_wt = q->cwt;
+        hipLaunchKernelGGL(kern, dim3(mtiles * ntiles), dim3(P::NW * 64), P::LDS, s, pc, mtiles, ntiles);
+        return 0;
+    }
+    BigMulti g;
+    memset(&g, 0, sizeof g);
+    g.n = n;
+    g.mtiles = mtiles;
+    long wg = 0;
+    for (int t = 0; t < n; t++) {
+        g.p[t] = p[t];
+        g.p[t].c_wt = q->cwt;
+        g.ntiles[t] = (p[t].N + BN - 1) / BN;
+        g.wg0[t] = (int)wg;
+        wg += ((long)mtiles * g.ntiles[t] + 7) / 8 * 8;
+    }
+    if (wg >= (1L << 24)) {
+        snprintf(g_lerr, sizeof g_lerr, "big group: %ld workgroups", wg);
+        return -2;
+    }
+    auto kern = k_bigm<KIND, BM, BN>;
+    if (lds_limit((const void *)kern, P::LDS, attr[1])) return -1;
+    hipLaunchKernelGGL(kern, dim3((unsigned)wg), dim3(P::NW * 64), P::LDS, s, g);
+    return 0;
+}
+
+template <int KIND> int launch_kind(const orkh_mm *p, int n, const orkh_plan *q, hipStream_t s) {
+    if (q->bm == 256 && q->bn == 256) return launch<KIND, 256, 256>(p, n, q, s);
+    if (q->bm == 256 && q->bn == 192) return launch<KIND, 256, 192>(p, n, q, s);
+    if (q->bm == 128 && q->bn == 256) return launch<KIND, 128, 256>(p, n, q, s);
+    if (q->bm == 128 && q->bn == 192) return launch<KIND, 128, 192>(p, n, q, s);
+    snprintf(g_lerr, sizeof g_lerr, "big plan: %dx%d unsupported", q->bm, q->bn);
+    return -2;
+}
+
+} // namespace
+
+// n = 1, or 2..ORKH_TGROUP_MAX matmuls of one kind, M and K (checked by the caller)
+extern "C" int orkh_big_launch(const orkh_mm *p, int n, const orkh_plan *q, void *stream) {
+    hipStream_t s = (hipStream_t)stream;
+    if (q->ksplit > 1) {
+        snprintf(g_lerr, sizeof g_lerr, "big plan: ksplit %d", q->ksplit);
+        return -2;
+    }
+    switch (p->kind) {
+    case ORKH_I8: return launch_kind<ORKH_I8>(p, n, q, s);
+    case ORKH_I4U: return launch_kind<ORKH_I4U>(p, n, q, s);
+    case ORKH_NF4: return launch_kind<ORKH_NF4>(p, n, q, s);
+    case ORKH_F16: return launch_kind<ORKH_F16>(p, n, q, s);
+    default: snprintf(g_lerr, sizeof g_lerr, "big plan: kind %d", p->kind); return -2;
+    }
+}

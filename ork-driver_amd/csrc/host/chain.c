@@ -106,7 +106,7 @@ static int chain_common(const char *who, ork_npu *c, int S, ctask *t, int want_d
     if (!q) { orki_err("%s: out of memory", who); return -1; }
     for (int i = 0; i < S; i++) {
         size_t wsi = 0;
-        orki_plan(c, t[i].w->rkind, t[i].M, t[i].w->K, t[i].w->N, t[i].w->KB, &q[i], &wsi);
+        orki_plan_mm(c, t[i].w->rkind, t[i].M, t[i].w->K, t[i].w->N, t[i].w->KB, &q[i], &wsi);
         if (wsi > ws) ws = wsi;
     }
     void *dws = NULL;
@@ -165,8 +165,8 @@ static int chain_common(const char *who, ork_npu *c, int S, ctask *t, int want_d
         if (n < 2) continue;
         orkh_plan gq;
         size_t gws = 0;
-        orki_plan(c, t[i].w->rkind, t[i].M, t[i].w->K, nsum, t[i].w->KB, &gq, &gws);
-        if (gq.algo != ORKH_ALGO_TILED2 || gq.ksplit > 1) continue;
+        orki_plan_mm(c, t[i].w->rkind, t[i].M, t[i].w->K, nsum, t[i].w->KB, &gq, &gws);
+        if ((gq.algo != ORKH_ALGO_TILED2 && gq.algo != ORKH_ALGO_BIG) || gq.ksplit > 1) continue;
         orkh_mm ps[ORKH_TGROUP_MAX];
         memset(ps, 0, sizeof ps);
         for (int k = 0; k < n; k++) {

@@ -12,6 +12,7 @@
  *   M <= 64  the streaming kernel (same grid, runs of 1-4 KiB) or the LDS-ring tiled kernel, whichever a
  *            delivery model of both prices lower, each with its best K split.
  *   M >  64  the LDS-ring tiled kernel: the tile and K split with the least modelled time.
+ *            Above 64 rows, large grids of every kind take the many-row kernel k_big instead (orki_plan_mm).
  *   NF4      (M > 1) the streaming kernel, k_tiled and the LDS-ring kernel, every tile and split, each priced by
  *            its own fit (nf4_best).
  * Both time models charge a workgroup for a fixed set-up, the operand bytes that must reach its CU and
@@ -537,6 +538,125 @@ static int plan_core(const ork_npu *c, int rkind, int M, int K, int N, int KB, o
     }
     q->algo = ORKH_ALGO_TILED;
     if (q->ksplit > 1) *ws_bytes = (size_t)q->ksplit * M * N * 4;
+    return 0;
+}
+
+/* When a run takes the many-row kernel (k_big, ../hip/orkh_big.hip) instead of orki_plan's pick.
+ * Above 64 rows both are priced, us, and the cheaper one runs:
+ *   k_big, per tile     rounds * (b + c * KiB) + e * MB            (rounds of the CUs; KiB: the A and B bytes a workgroup
+ *                                                                  loads; MB: C's megabytes, which the end of a round
+ *                                                                  writes with nothing to overlap)
+ *   orki_plan's pick    a + rounds * c[tile] * KiB + e * MB + [ks > 1] (d + f * ks * MB)      (e: e1 on one round, else e2)
+ * Each is a least-squares fit in relative error (non-negative terms) to launches timed back to back on MI355X: every
+ * k_big tile and orki_plan's pick at K x N = 2048 x 6144, 2048 x 2048, 4096 x 4096, 6144 x 2048, 2048 x 12288, 2048 x 4096
+ * and 18 row counts from 256 to 4096, per weight kind (108 shapes a kind; a k_big tile's fit takes the shapes where it ran
+ * within 1.6x of the fastest); 1-8% rms (k_big) and 4-7% (the picks). What the rule chooses over those shapes, total
+ * us: int8 3346 -> 3083 (the faster of the two everywhere would be 3081), fp16 5973 -> 5499 (5492), uniform int4 3625 ->
+ * 2891 (2891), NF4 4760 -> 3973 (3951), and no shape is slower than its former pick; NF4's 2% margin keeps two shapes
+ * where k_big ran 4-5% slower. 256 x 256 picks always move: k_big was ahead on each. Some shapes, us: int8 K=N=4096
+ * M=4096 65.0 -> 61.3, K=6144 N=2048 M=4096 63.3 -> 49.3, K=N=4096 M=2048 41.5 -> 35.2; fp16 K=2048 N=6144 M=4096 140.6
+ * -> 114.3; uniform int4 K=N=4096 M=4096 89.8 -> 55.5; NF4 112.0 -> 73.8, K=2048 N=6144 M=1000 29.5 -> 24.2. At 512 rows
+ * and fewer the smaller tiles fill the CUs better and keep the run (int8 K=2048 N=6144 M=500 11.9 against 16.6), except
+ * where N is large (N=12288 20.3 -> 17.6).
+ * A context's planner overrides (ORK_PLAN, ORK_TILE and the others of orki_plan) turn the rule off, and ORK_PLAN=big with
+ * ORK_TILE=BMxBN forces a k_big tile. */
+static const struct big_fit {
+    int rkind, bm, bn;
+    double b, c, e;
+} big_fits[] = {
+    {ORKH_I8, 256, 256, 3.832, 0.01899, 0.1932}, {ORKH_I8, 256, 192, 3.190, 0.01845, 0.2148},
+    {ORKH_I8, 128, 256, 2.128, 0.01653, 0.2067}, {ORKH_I8, 128, 192, 4.175, 0.01636, 0.1357},
+    {ORKH_F16, 256, 256, 0.000, 0.01968, 0.3515}, {ORKH_F16, 256, 192, 0.000, 0.01891, 0.3824},
+    {ORKH_F16, 128, 256, 0.000, 0.01663, 0.3665}, {ORKH_F16, 128, 192, 1.648, 0.01716, 0.3193},
+    {ORKH_I4U, 256, 256, 6.614, 0.02672, 0.1046}, {ORKH_I4U, 256, 192, 6.102, 0.02459, 0.0925},
+    {ORKH_I4U, 128, 256, 4.943, 0.02404, 0.0811}, {ORKH_I4U, 128, 192, 4.922, 0.02336, 0.0615},
+    {ORKH_NF4, 256, 256, 7.815, 0.03910, 0.0886}, {ORKH_NF4, 256, 192, 6.959, 0.03410, 0.0737},
+    {ORKH_NF4, 128, 256, 5.171, 0.04358, 0.0746}, {ORKH_NF4, 128, 192, 4.913, 0.03929, 0.0700},
+};
+static const struct pick_fit {
+    int rkind;
+    double margin, a, e1, e2, d, f;
+} pick_fits[] = {
+    {ORKH_I8, 1.00, 2.1398, 0.1758, 0.2503, 3.7309, 0.2135},
+    {ORKH_F16, 1.00, 0.0000, 0.3488, 0.4121, 0.7596, 0.5661},
+    {ORKH_I4U, 1.00, 1.6989, 0.2755, 0.2359, 0.0000, 0.6995},
+    {ORKH_NF4, 0.98, 2.2934, 0.1759, 0.2515, 8.4391, 0.0000},
+};
+static const struct pick_rate { /* c of a tile; bm 0: a tile that no timed shape picked */
+    int rkind, bm, bn, ring;
+    double c;
+} pick_rates[] = {
+    {ORKH_I8, 32, 64, 0, 0.0236}, {ORKH_I8, 64, 64, 0, 0.0167}, {ORKH_I8, 64, 192, 2, 0.0118}, {ORKH_I8, 128, 96, 0, 0.0157},
+    {ORKH_I8, 128, 96, 2, 0.0128}, {ORKH_I8, 128, 128, 0, 0.0155}, {ORKH_I8, 128, 128, 2, 0.0147}, {ORKH_I8, 0, 0, 0, 0.0150},
+    {ORKH_F16, 32, 64, 0, 0.0249}, {ORKH_F16, 64, 64, 0, 0.0203}, {ORKH_F16, 128, 96, 0, 0.0162}, {ORKH_F16, 128, 96, 2, 0.0126},
+    {ORKH_F16, 128, 128, 0, 0.0156}, {ORKH_F16, 128, 128, 2, 0.0147}, {ORKH_F16, 0, 0, 0, 0.0150},
+    {ORKH_I4U, 32, 64, 0, 0.0222}, {ORKH_I4U, 64, 64, 0, 0.0156}, {ORKH_I4U, 0, 0, 0, 0.0194},
+    {ORKH_NF4, 32, 64, 0, 0.0320}, {ORKH_NF4, 64, 64, 0, 0.0315}, {ORKH_NF4, 128, 96, 0, 0.0304}, {ORKH_NF4, 0, 0, 0, 0.0281},
+};
+
+/* any planner override of orki_plan in the environment of a context that honours them */
+static int overridden(const ork_npu *c) {
+    static const char *const names[] = {"ORK_PLAN", "ORK_TILE", "ORK_KSPLIT", "ORK_ALINE", "ORK_RING", "ORK_CWT"};
+    if (!c || !c->plan_knobs) return 0;
+    for (size_t i = 0; i < sizeof names / sizeof names[0]; i++)
+        if (getenv(names[i])) return 1;
+    return 0;
+}
+
+static void take_big(const ork_npu *c, int bm, int bn, int M, int N, int KB, orkh_plan *q, size_t *ws_bytes) {
+    const int cu = (c && c->cores > 0) ? c->cores : 256;
+    memset(q, 0, sizeof *q);
+    q->algo = ORKH_ALGO_BIG;
+    q->bm = bm;
+    q->bn = bn;
+    q->ksplit = 1;
+    q->kbs = KB;
+    q->cwt = (long)cdiv(M, bm) * cdiv(N, bn) <= cu; /* write-through C on one round, as orki_plan's tiles */
+    *ws_bytes = 0;
+}
+
+int orki_plan_mm(const ork_npu *c, int rkind, int M, int K, int N, int KB, orkh_plan *q, size_t *ws_bytes) {
+    const int rc = orki_plan(c, rkind, M, K, N, KB, q, ws_bytes);
+    if (rc || M <= 64) return rc;
+    if (overridden(c)) {
+        const char *f = getenv("ORK_PLAN"), *t = getenv("ORK_TILE");
+        int bm, bn;
+        if (f && !strcmp(f, "big") && t && sscanf(t, "%dx%d", &bm, &bn) == 2) take_big(c, bm, bn, M, N, KB, q, ws_bytes);
+        return 0;
+    }
+    if (q->algo != ORKH_ALGO_TILED2 && q->algo != ORKH_ALGO_TILED) return 0;
+    const int cu = (c && c->cores > 0) ? c->cores : 256;
+    const double abpk = rkind == ORKH_I4U || rkind == ORKH_NF4 ? 128 : 64; /* A bytes per row and K-block */
+    const double mb = (double)M * N * 4 / 1e6;
+    for (size_t i = 0; i < sizeof pick_fits / sizeof pick_fits[0]; i++) {
+        const struct pick_fit *p = &pick_fits[i];
+        if (p->rkind != rkind) continue;
+        const int ks = q->ksplit > 1 ? q->ksplit : 1, kbs = ks > 1 ? q->kbs : KB;
+        const long wgs = (long)cdiv(M, q->bm) * cdiv(N / 16, q->bn / 16) * ks;
+        const struct pick_rate *r = NULL;
+        for (size_t j = 0; j < sizeof pick_rates / sizeof pick_rates[0] && !r; j++) {
+            const struct pick_rate *x = &pick_rates[j];
+            if (x->rkind == rkind && (!x->bm || (x->bm == q->bm && x->bn == q->bn && x->ring == q->ring))) r = x;
+        }
+        const double rounds = (double)((wgs + cu - 1) / cu);
+        double best = p->a + rounds * r->c * (q->bm * abpk + q->bn * 64.0) * kbs / 1024 + (wgs <= cu ? p->e1 : p->e2) * mb +
+                      (ks > 1 ? p->d + p->f * ks * mb : 0);
+        best = q->bm == 256 && q->bn == 256 ? 1e30 : best * p->margin;
+        int bm = 0, bn = 0;
+        for (size_t j = 0; j < sizeof big_fits / sizeof big_fits[0]; j++) {
+            const struct big_fit *g = &big_fits[j];
+            if (g->rkind != rkind) continue;
+            const long w = (long)cdiv(M, g->bm) * cdiv(N, g->bn);
+            const double t = (double)((w + cu - 1) / cu) * (g->b + g->c * (g->bm * abpk + g->bn * 64.0) * KB / 1024) + g->e * mb;
+            if (t < best) {
+                best = t;
+                bm = g->bm;
+                bn = g->bn;
+            }
+        }
+        if (bm) take_big(c, bm, bn, M, N, KB, q, ws_bytes);
+        return 0;
+    }
     return 0;
 }
 

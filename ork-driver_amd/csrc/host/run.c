@@ -67,7 +67,7 @@ static int run_common(const char *who, ork_npu *c, ork_w *w, int want_dt, int M,
 
     orkh_plan q;
     size_t ws = 0;
-    orki_plan(c, w->rkind, M, K, N, w->KB, &q, &ws);
+    orki_plan_mm(c, w->rkind, M, K, N, w->KB, &q, &ws);
     if (ws) {
         q.ws = orki_ws_stage(c, ws, NULL);
         if (!q.ws) { orki_hip_fail(who); return -1; }
@@ -140,7 +140,7 @@ int ork_i8_mm_run_noalloc(ork_npu *c, ork_w *w, int M, const int8_t *A, int32_t 
     }
     orkh_plan q;
     size_t ws = 0;
-    orki_plan(c, w->rkind, M, K, N, w->KB, &q, &ws);
+    orki_plan_mm(c, w->rkind, M, K, N, w->KB, &q, &ws);
     if (ws > ORKH_SCRATCH_BYTES) {
         orki_err("%s: the plan's split-K partials need %zu B, above the %u B scratch array", who, ws,
                  (unsigned)ORKH_SCRATCH_BYTES);
@@ -391,7 +391,7 @@ const char *ork_w_plan_name(ork_npu *c, const ork_w *w, int M) {
     if (!c || !w || w->rkind < 0 || M < 1) return "none";
     orkh_plan q;
     size_t ws;
-    orki_plan(c, w->rkind, M, w->K, w->N, w->KB, &q, &ws);
+    orki_plan_mm(c, w->rkind, M, w->K, w->N, w->KB, &q, &ws);
     orkh_mm p;
     memset(&p, 0, sizeof p);
     p.kind = w->rkind;

@@ -893,3 +893,93 @@ def test_gemv_half_unaligned_activations(npu):
     L.ork_dev_free(npu.h, dA)
     L.ork_dev_free(npu.h, dC)
     ork.free(w)
+
+
+BIG_TILES = ["256x256", "256x192", "128x256", "128x192"]
+
+
+@pytest.mark.parametrize("tile", BIG_TILES)
+@pytest.mark.parametrize("kind", ["i8", "i4a8", "nf4", "w4a4", "f16"])
+def test_many_row_tiles(npu, kind, tile):
+    """The many-row kernel at every tile and kind: rows one short of, at and past a tile (and two tiles with a tail), K of
+    one K-block, of an odd count of them, of part of one, shorter and longer than its ring of stages, N with a partial
+    tile and a partial wave column. Integers exact; fp16 within the bar of fp64 accumulation."""
+    _say("many rows", kind, tile)
+    bm, bn = map(int, tile.split("x"))
+    rng = np.random.default_rng(bm + bn)
+    for M, K, N in ((65, 32, 64), (bm - 1, 160, bn), (bm, 96, bn + 64), (bm + 1, 1056, 2 * bn - 64), (2 * bm + 17, 608, 448)):
+        if kind == "f16":
+            B = (rng.standard_normal((K, N)) * 0.02).astype(np.float16)
+            A = rng.standard_normal((M, K)).astype(np.float16)
+            w, run, ref = npu.pack_f16(B), npu.run_f16, O.gemm_f16_f64acc(A, B)
+        elif kind == "w4a4":
+            B = rng.integers(-8, 8, size=(K, N), dtype=np.int8)
+            A = rng.integers(-8, 8, size=(M, K), dtype=np.int8)
+            w, run, ref = npu.pack_i4(B), npu.run_i4, O.gemm_i32(A, B)
+        elif kind == "i8":
+            B = rng.integers(-128, 128, size=(K, N), dtype=np.int8)
+            A = rng.integers(-128, 128, size=(M, K), dtype=np.int8)
+            w, run, ref = npu.pack_i8(B), npu.run_i8, O.gemm_i32(A, B)
+        else:
+            W = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+            with _env(**({"ORK_NF4": 1} if kind == "nf4" else {})):
+                w, _ = npu.pack_i4a8(W)
+            A = rng.integers(-128, 128, size=(M, K), dtype=np.int8)
+            run, ref = npu.run_i8, O.gemm_i32(A, O.pack_i4a8(W, nf4=kind == "nf4")[2])
+        with _env(ORK_PLAN="big", ORK_TILE=tile):
+            rc, C = run(w, A)
+            name = npu.plan_name(w, M)
+        assert rc == 0 and name.startswith("big_") and name.endswith(tile), name
+        if kind == "f16":
+            assert O.fp16_err(C, ref) <= FP16_TOL, (name, M, K, N)
+        else:
+            assert np.array_equal(C, ref), (name, M, K, N)
+        ork.free(w)
+
+
+@pytest.mark.parametrize("tile", BIG_TILES)
+def test_many_row_chain_and_stride(npu, tile):
+    """Two projections of one input as one many-row launch (int8 and uniform int4), into one buffer at a row stride that
+    keeps rows 16-byte aligned and one that does not (vector and word stores): exact, and nothing outside the blocks."""
+    _say("many-row chain", tile)
+    bm, bn = map(int, tile.split("x"))
+    rng = np.random.default_rng(7 * bm + bn)
+    M, K, Ns = bm + 9, 416, (bn + 32, 96)
+    for kind in ("i8", "u4"):
+        for ld in (640, 643):
+            A = rng.integers(-128, 128, size=(M, K), dtype=np.int8)
+            ws, refs = [], []
+            for N in Ns:
+                W = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+                if kind == "i8":
+                    w, _ = npu.pack_i8_f32(W)
+                    refs.append(O.gemm_i32(A, O.pack_i8_f32(W)[0]))
+                else:
+                    w, _ = npu.pack_i4a8(W)
+                    refs.append(O.gemm_i32(A, O.pack_i4a8(W)[2]))
+                ws.append(w)
+            C = np.full((M, ld), -77, np.int32)
+            with _env(ORK_PLAN="big", ORK_TILE=tile):
+                t = ork.tasks(ork.TaskI8, [(ws[0], M, A, C, ld), (ws[1], M, A, int(C.ctypes.data) + 4 * Ns[0], ld)])
+                assert ork.lib().ork_i8_mm_run_chain(npu.h, 2, t) == 0
+            assert np.array_equal(C[:, :Ns[0]], refs[0]) and np.array_equal(C[:, Ns[0]:sum(Ns)], refs[1]), (kind, ld)
+            assert np.all(C[:, sum(Ns):] == -77)
+            for w in ws:
+                ork.free(w)
+
+
+def test_many_row_rule(npu):
+    """Where the many-row kernel takes the run: grids that fill the CUs with its tiles, per kind (the measured shapes beside
+    the rule), never at 64 rows or fewer, never past an override."""
+    K, N = 2048, 6144
+    B = np.zeros((K, N), np.int8)
+    w, w4 = npu.pack_i8(B), npu.pack_i4(B)
+    try:
+        assert npu.plan_name(w, 4096).startswith("big_i8_") and npu.plan_name(w4, 4096).startswith("big_i4u_")
+        assert npu.plan_name(w4, 1000).startswith("big_i4u_128x192")
+        assert npu.plan_name(w, 512) == "tiled2_i8_128x96_al" and not npu.plan_name(w, 64).startswith("big_")
+        with _env(ORK_TILE="128x128"):
+            assert npu.plan_name(w, 4096).startswith("tiled2_i8_128x128")
+    finally:
+        ork.free(w)
+        ork.free(w4)
