@@ -166,6 +166,8 @@ typedef struct orkh_group {
  * int8 and uniform int4). 0 / -2 bad arguments / -1 HIP error. */
 int orkh_mm_launch_grouped(const orkh_mm *p, const orkh_plan *plan, int G, const float *aS, const float *bS, float *C,
                            int ldc, void *stream);
+/* its ORKH_ALGO_TILED2 launch (orkh_grouped.hip; p carries C, ldc and c_wt): 64 x 64, 64 x 192, 128 x 128, 128 x 256 */
+int orkh_tiled2g_launch(const orkh_mm *p, const orkh_plan *plan, int G, const float *aS, const float *bS, void *stream);
 int orkh_mm_launch_group(const orkh_group *g, int wpg, void *stream);
 /* One-row run with a fused row prologue and column epilogue (k_gemv_row, orkh_rowrun.hip): every workgroup builds the
  * int8 row in LDS from a float row (pro: ORKH_ROW_RMSNORM = RMSNorm with weight nw, then the per-row quant;
@@ -195,8 +197,6 @@ typedef struct orkh_row {
 } orkh_row;
 /* 0 / -2 an unbuilt combination or bad fields / -1 HIP error */
 int orkh_row_launch(const orkh_row *p, void *stream);
-/* Bytes of LDS the stage ring of k_tiled2 takes for (kind, bm x bn); -1 for a tile that is not built. */
-int orkh_tiled2_ring_lds(int kind, int bm, int bn);
 /* 1 where the LDS-ring kernel has a two-slot ring for the tile (plan.ring = 2): tiles whose ring of up to 4 slots
  * leaves room for one workgroup per CU, and two with 2 slots; never NF4 */
 int orkh_tiled2_ring2_ok(int kind, int bm, int bn);

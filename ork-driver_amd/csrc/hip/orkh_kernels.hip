@@ -609,7 +609,7 @@ template <int KIND, int BM, int BN, int KS, int XG = 0, int RC = 0> struct T2 {
     static_assert(!LINE_OK || NIA * 8 == BM * ALN, "line-loaded A: one instruction per 8 row lines");
 };
 
-// Wave grids other than 4 x 4 (grouped runs always keep it):
+// Wave grids other than 4 x 4:
 // 1: 2 x 4 with 2 K groups (each B block decoded by two waves instead of four), for the uniform-int4 64 x 192
 //    tile. Measured against 4 x 4 (us): W4A8 K=2048 N=6144 M=512 14.7 -> 13.4, M=256 13.3 -> 12.5; W4A4 M=512
 //    K=N=4096 22.0 -> 19.9. Not kept elsewhere: int8 M=512 64 x 192 13.9 -> 14.7, fp16 M=1024 20.5 -> 21.1,
@@ -617,8 +617,7 @@ template <int KIND, int BM, int BN, int KS, int XG = 0, int RC = 0> struct T2 {
 // 2: 2 x 2 with 4 K groups (each wave 32 x 32 of C: half the LDS reads per MFMA of a 16 x 16 wave block, each B
 //    block decoded by two waves), for the uniform-int4 64 x 64 tile: W4A4 M=256 K=N=4096 14.76 -> 14.00. Not
 //    kept for fp16 (M=512 K=N=2048 13.98 -> 15.35).
-template <int KIND, int BM, int BN, int GR> constexpr int t2_xg() {
-    if (GR != 0) return 0;
+template <int KIND, int BM, int BN> constexpr int t2_xg() {
     if (KIND == ORKH_I4U && BM == 64 && BN == 192) return 1;
     if (KIND == ORKH_I4U && BM == 64 && BN == 64) return 2;
     return 0;
@@ -631,15 +630,14 @@ template <int KIND, int BM, int BN, int GR> constexpr int t2_xg() {
 // them; later, the MFMAs of the waves not held go on. Graph-timed against right after the barrier (one build each,
 // alternated twice on one box; int8 and fp16 through bench.py's config section too; exact): int8 64 x 192 M=512
 // K=2048 N=6144 13.56-13.68 -> 13.15-13.28 us (after the first of two K-blocks; after both: -0.4 to -0.9%); NF4
-// 128 x 128 M=512 16.62 -> 15.46 (after its one K-block); grouped W4A4 K=N=4096 G=128 64 x 64 M=256 18.33 -> 17.08
-// (after the first of four); uniform int4 64 x 192 W4A4 M=512 18.54 -> 17.95, W4A8 M=512 12.67 -> 12.54, 32 x 64
+// 128 x 128 M=512 16.62 -> 15.46 (after its one K-block); uniform int4 64 x 192 W4A4 M=512 18.54 -> 17.95, W4A8 M=512 12.67 -> 12.54, 32 x 64
 // W4A8 M=64 6.03 -> 5.94 (after their one); int8 32 x 64 (four chained M=256 runs) 13.92 -> 13.32-13.80. No gain, so
 // right after the barrier: fp16 64 x 64 M=512 (-0.3 to +0.6% either way), uniform int4 on the 2 x 2 x 4 wave grid
 // (64 x 64, W4A4 M=256: +0.4 to +0.8%) and NF4 on the K-group tiles (its decode runs a stage ahead; -0.1 to -0.6%);
 // the two-slot rings, whose second workgroup per CU already overlaps one's loads with the other's MFMAs, keep it too.
 template <int KIND, int BM, int BN, class P> constexpr int t2_issue_at() {
     if (P::R <= 2 || (KIND == ORKH_NF4 && P::WK > 1) || (KIND == ORKH_F16 && BM == 64 && BN == 64) ||
-        (KIND == ORKH_I4U && BM == 64 && BN == 64 && P::WK > 1)) // the 2 x 2 x 4 grid; grouped runs keep 4 x 4
+        (KIND == ORKH_I4U && BM == 64 && BN == 64 && P::WK > 1)) // the 2 x 2 x 4 grid
         return 0;
     return 1;
 }
@@ -695,22 +693,12 @@ __device__ __forceinline__ int a_lds(int mb, int kbl, int st, int lane) {
     }
 }
 
-// Grouped mode of k_tiled2 (ork_*_mm_run_grouped): C is fp32 and every output is the sum, in ascending g, of
-// ((float)P_g * aS[m][g]) * bS[g][n] with P_g the exact int32 partial over K-group g (src/npu/core/buf.c:501-520).
-struct T2Group {
-    int G;            // group size in k; G % 32 == 0 and K % G == 0
-    const float *aS;  // [M][K/G]
-    const float *bS;  // [K/G][N]
-};
-
 // bid, nT: this workgroup's index among the launch's nT workgroups of this matmul (blockIdx.x and gridDim.x, or a
 // task's share of a grouped launch, which starts at a multiple of 8 so that bid % 8 is still the XCD)
-template <int KIND, int BM, int BN, int KS, int GR, bool AL, int RC = 0>
-__device__ __forceinline__ void tiled2_body(const orkh_mm &p, int mtiles, int ntiles_all, int kbs, void *ws,
-                                            const T2Group &gp, int bid, int nT) {
-#pragma clang fp contract(off)
+template <int KIND, int BM, int BN, int KS, bool AL, int RC = 0>
+__device__ __forceinline__ void tiled2_body(const orkh_mm &p, int mtiles, int ntiles_all, int kbs, void *ws, int bid, int nT) {
     using T = KT<KIND>;
-    using P = T2<KIND, BM, BN, KS, t2_xg<KIND, BM, BN, GR>(), RC>;
+    using P = T2<KIND, BM, BN, KS, t2_xg<KIND, BM, BN>(), RC>;
     constexpr int R = P::R;
     constexpr bool LINE = AL && P::LINE_OK; // A stage as whole row lines (a_lds), else in fragment order
     typedef typename T::acc_t acc_t;
@@ -723,10 +711,8 @@ __device__ __forceinline__ void tiled2_body(const orkh_mm &p, int mtiles, int nt
     // 2 x 2 x 4 M=256 12.28 -> 12.00.
     asm volatile("" ::"s"(p.M), "s"(p.K), "s"(p.N), "s"(p.KB), "s"(p.lda), "s"(p.A), "s"(p.B), "s"(p.C), "s"(p.ldc),
                  "s"(p.c_wt), "s"(mtiles), "s"(ntiles_all), "s"(kbs), "s"(ws), "s"(nT));
-    if constexpr (GR != 0) asm volatile("" ::"s"(gp.G), "s"(gp.aS), "s"(gp.bS));
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    static_assert(GR == 0 || P::WK == 1, "grouped runs walk every K-block in one wave");
     const int wk = P::WK > 1 ? wv / (P::WM * P::WN) : 0, wr = P::WK > 1 ? wv % (P::WM * P::WN) : wv;
     const int wm = wr % P::WM, wn = wr / P::WM;
     // XCD-aware order: WG b runs on XCD b%8; each XCD gets a contiguous run of tiles, M fastest, so every
@@ -746,10 +732,8 @@ __device__ __forceinline__ void tiled2_body(const orkh_mm &p, int mtiles, int nt
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)sm;
     const Lut L = {p.lut[0], p.lut[1], p.lut[2], p.lut[3]};
 
-    // this wave's loads: i = wv + q * LW (waves wv >= LW issue none); A fragment (mb, kbl, step) or B block (nbl, kbl).
-    // Grouped runs: 8 loader waves, which also issue the tile's scale loads (before their ring loads, so their first
-    // wait covers them): W4A4 K=N=4096 G=128 M=256 16.64-16.85 -> 16.07-16.26 us against every wave issuing, exact
-    constexpr int LW = GR == 0 ? t2_loaders<KIND, BM, BN, P>() : (P::NI % 8 == 0 ? 8 : P::NW);
+    // this wave's loads: i = wv + q * LW (waves wv >= LW issue none); A fragment (mb, kbl, step) or B block (nbl, kbl)
+    constexpr int LW = t2_loaders<KIND, BM, BN, P>();
     constexpr int IPW = LW == P::NW ? P::IPW : P::NI / LW;
     static_assert(LW == P::NW || P::NI % LW == 0, "loader waves");
     static_assert((R - 2) * IPW < 64, "vmcnt");
@@ -806,65 +790,7 @@ __device__ __forceinline__ void tiled2_body(const orkh_mm &p, int mtiles, int nt
 #pragma unroll
         for (int b = 0; b < P::NTW; b++) acc[a][b] = acc_t{0, 0, 0, 0};
 
-    // grouped mode: fp32 running sums, and this tile's scales in LDS after the ring -- aS rows m0.. (BM x Sk,
-    // one contiguous run of aS) and bS columns n0.. of every group (Sk x BN) -- brought in by direct-to-LDS
-    // loads issued before the ring's, so the first stage's wait covers them and no later wait drains the
-    // ring. Rows past M read zeros and columns past N read a neighbouring row; neither is stored.
-    const int Sk = GR ? p.K / gp.G : 1;
-    const int sca_kib = GR ? (BM * Sk * 4 + 1023) / 1024 : 0;
-    const int scb_kib = GR ? (Sk * BN * 4 + 1023) / 1024 : 0;
-    const float *sAl = (const float *)(sm + P::LDS / 16);
-    const float *sBl = sAl + sca_kib * 256;
-    float cacc[P::MTW][P::NTW][4];
-    float sa[P::MTW][4], sb[P::NTW]; // scales of the next group to close
-    int gcur = 0, gend = GR ? gp.G : 0; // that group and the k where it ends
-    const int gps = GR == 2 ? gp.G / T::KPB : 1; // K-blocks per group (groups of whole K-blocks)
-    int sgs = 0;                                   // K-blocks of the current group done
-    auto load_sc = [&](int g) {
-#pragma unroll
-        for (int i = 0; i < P::MTW; i++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) sa[i][r] = sAl[((wm * P::MTW + i) * 16 + (lane >> 4) * 4 + r) * Sk + g];
-#pragma unroll
-        for (int jn = 0; jn < P::NTW; jn++) sb[jn] = sBl[g * BN + (wn * P::NTW + jn) * 16 + (lane & 15)];
-    };
-    // close group gcur: its exact partial, scaled, joins the fp32 sums in group order; read the next scales
-    auto close_group = [&]() {
-#pragma unroll
-        for (int i = 0; i < P::MTW; i++)
-#pragma unroll
-            for (int jn = 0; jn < P::NTW; jn++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const float t = ((float)finish<KIND>(acc[i][jn][r]) * sa[i][r]) * sb[jn];
-                    cacc[i][jn][r] = cacc[i][jn][r] + t;
-                    acc[i][jn][r] = 0;
-                }
-        gcur++;
-        if (gcur < Sk) load_sc(gcur); // read ahead: waited for at the next close
-    };
-    if constexpr (GR) {
-#pragma unroll
-        for (int i = 0; i < P::MTW; i++)
-#pragma unroll
-            for (int jn = 0; jn < P::NTW; jn++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) cacc[i][jn][r] = 0.0f;
-        const uint32_t scl = lds0 + (uint32_t)P::LDS;
-        const __amdgpu_buffer_rsrc_t Sa = make_rsrc(gp.aS, (uint32_t)p.M * Sk * 4u);
-        const __amdgpu_buffer_rsrc_t Sb = make_rsrc(gp.bS, (uint32_t)Sk * p.N * 4u);
-        for (int i = wv; wv < LW && i < sca_kib + scb_kib; i += LW) {
-            if (i < sca_kib) {
-                lds_dma16<8>(Sa, (uint32_t)m0 * Sk * 4u + (uint32_t)i * 1024u + lane * 16u, scl + i * 1024);
-            } else {
-                const int f = (i - sca_kib) * 256 + lane * 4; // first float of this lane within the Sk x BN tile
-                const int g = f / BN, c = f - g * BN;
-                lds_dma16<9>(Sb, g < Sk ? ((uint32_t)g * p.N + nb0 * 16 + c) * 4u : OOB, scl + i * 1024);
-            }
-        }
-    }
-
-    // NF4 (plain runs): a stage's B blocks are decoded once, into int8 MFMA operands in LDS, one stage ahead of
+    // NF4: a stage's B blocks are decoded once, into int8 MFMA operands in LDS, one stage ahead of
     // their MFMAs -- iteration s decodes stage s + 1 into one half of Dec while its MFMAs read stage s from the
     // other, so the codebook decode (VALU) overlaps the matrix work and the stage keeps a single barrier.
     // Measured against decoding each stage before its MFMAs behind a second barrier (us, K=2048 N=6144 unless
@@ -875,7 +801,7 @@ __device__ __forceinline__ void tiled2_body(const orkh_mm &p, int mtiles, int nt
     // per wave after them); on the others a block per wave decodes after the wave's MFMAs (64 x 64 M=256 15.54
     // -> 14.49, 128 x 128 M=1024 32.96 -> 29.58 against equal shares before them). Equal shares with half the
     // waves of each SIMD decoding first and half after measured slower than both.
-    constexpr bool PIPE = P::DEC2 && GR == 0;
+    constexpr bool PIPE = P::DEC2;
     constexpr bool EARLY = PIPE && P::WK > 1;
     static_assert(!PIPE || R >= 3, "NF4 ring: the decode runs a stage ahead");
     v4i *const Dec = sm + P::R * (P::SLOT / 16); // [stage parity, if PIPE][block][step]
@@ -921,9 +847,8 @@ __device__ __forceinline__ void tiled2_body(const orkh_mm &p, int mtiles, int nt
         }
     };
 
-    // where in a stage the waves issue the loads of the stage R - 1 ahead (t2_issue_at; grouped runs whose groups
-    // close inside K-blocks walk the stage in another loop: right after the barrier)
-    constexpr int IA = GR == 1 ? 0 : t2_issue_at<KIND, BM, BN, P>() < P::KPW ? t2_issue_at<KIND, BM, BN, P>() : P::KPW;
+    // where in a stage the waves issue the loads of the stage R - 1 ahead (t2_issue_at)
+    constexpr int IA = t2_issue_at<KIND, BM, BN, P>() < P::KPW ? t2_issue_at<KIND, BM, BN, P>() : P::KPW;
 #pragma unroll
     for (int st = 0; st < R - 1; st++) issue(st, std::integral_constant<int, 0>{});
     if constexpr (PIPE) {
@@ -943,9 +868,6 @@ __device__ __forceinline__ void tiled2_body(const orkh_mm &p, int mtiles, int nt
         if constexpr (IA == 0) issue(s + R - 1, std::integral_constant<int, 1>{});
         const v4i *As = sm + (s % R) * (P::SLOT / 16);
         const v4i *Bs = As + P::NIA * 64;
-        if constexpr (GR) {
-            if (s == 0) load_sc(0); // the scales landed with stage 0 (older loads, same wait)
-        }
         const v4i *Ds = Dec + (PIPE ? (s & 1) : 0) * (P::NIB * T::STEPS * 64);
         if constexpr (KIND == ORKH_NF4 && !PIPE) {
             decode_stage(s);
@@ -954,86 +876,33 @@ __device__ __forceinline__ void tiled2_body(const orkh_mm &p, int mtiles, int nt
         if constexpr (EARLY) {
             if (s + 1 < nst) decode_stage(s + 1);
         }
-        if constexpr (GR != 1) {
 #pragma unroll
-            for (int kk = 0; kk < P::KPW; kk++) {
-                if (kk > 0 && kk == IA) issue(s + R - 1, std::integral_constant<int, 2>{});
-                const int kbl = wk * P::KPW + kk; // this wave's K-blocks of the stage
-                v4i op[P::NTW][T::STEPS];
+        for (int kk = 0; kk < P::KPW; kk++) {
+            if (kk > 0 && kk == IA) issue(s + R - 1, std::integral_constant<int, 2>{});
+            const int kbl = wk * P::KPW + kk; // this wave's K-blocks of the stage
+            v4i op[P::NTW][T::STEPS];
 #pragma unroll
-                for (int jn = 0; jn < P::NTW; jn++) {
-                    const int b = (wn * P::NTW + jn) * KS + kbl;
-                    if constexpr (KIND == ORKH_NF4) {
+            for (int jn = 0; jn < P::NTW; jn++) {
+                const int b = (wn * P::NTW + jn) * KS + kbl;
+                if constexpr (KIND == ORKH_NF4) {
 #pragma unroll
-                        for (int st = 0; st < T::STEPS; st++) op[jn][st] = Ds[(b * T::STEPS + st) * 64 + lane];
-                    } else {
-                        decode<KIND>(Bs[b * 64 + lane], op[jn], L);
-                    }
-                }
-#pragma unroll
-                for (int st = 0; st < T::STEPS; st++)
-#pragma unroll
-                    for (int i = 0; i < P::MTW; i++) {
-                        const v4i a = As[a_lds<KIND, KS, LINE, BM / 8>(wm * P::MTW + i, kbl, st, lane)];
-#pragma unroll
-                        for (int jn = 0; jn < P::NTW; jn++) acc[i][jn] = mma(a, op[jn][st], acc[i][jn]);
-                    }
-                if constexpr (GR == 2) {
-                    // groups of whole K-blocks: close the group this K-block ends (the zero-filled K-blocks past
-                    // the end, in a last stage of fewer, count for none)
-                    if (kb_lo + s * KS + kbl < kb_hi && ++sgs == gps) {
-                        sgs = 0;
-                        close_group();
-                    }
+                    for (int st = 0; st < T::STEPS; st++) op[jn][st] = Ds[(b * T::STEPS + st) * 64 + lane];
+                } else {
+                    decode<KIND>(Bs[b * 64 + lane], op[jn], L);
                 }
             }
-            if constexpr (IA > 0 && IA == P::KPW) issue(s + R - 1, std::integral_constant<int, 3>{});
+#pragma unroll
+            for (int st = 0; st < T::STEPS; st++)
+#pragma unroll
+                for (int i = 0; i < P::MTW; i++) {
+                    const v4i a = As[a_lds<KIND, KS, LINE, BM / 8>(wm * P::MTW + i, kbl, st, lane)];
+#pragma unroll
+                    for (int jn = 0; jn < P::NTW; jn++) acc[i][jn] = mma(a, op[jn][st], acc[i][jn]);
+                }
         }
+        if constexpr (IA > 0 && IA == P::KPW) issue(s + R - 1, std::integral_constant<int, 3>{});
         if constexpr (PIPE && !EARLY) {
             if (s + 1 < nst) decode_stage(s + 1);
-        }
-        if constexpr (GR == 1) {
-            // every fragment of the stage is read first, as above, so the LDS latencies overlap; then the
-            // K-blocks run group by group. A 16-k A chunk lies wholly inside one group (G % 32 == 0).
-            v4i afr[KS][T::STEPS][P::MTW], bop[KS][P::NTW][T::STEPS];
-#pragma unroll
-            for (int kbl = 0; kbl < KS; kbl++) {
-#pragma unroll
-                for (int jn = 0; jn < P::NTW; jn++)
-                    decode<KIND>(Bs[((wn * P::NTW + jn) * KS + kbl) * 64 + lane], bop[kbl][jn], L);
-#pragma unroll
-                for (int st = 0; st < T::STEPS; st++)
-#pragma unroll
-                    for (int i = 0; i < P::MTW; i++)
-                        afr[kbl][st][i] = As[a_lds<KIND, KS, LINE, BM / 8>(wm * P::MTW + i, kbl, st, lane)];
-            }
-#pragma unroll
-            for (int kbl = 0; kbl < KS; kbl++) {
-                const int kb = kb_lo + s * KS + kbl;
-                if (kb >= kb_hi) break;
-                const int kb_k0 = kb * T::KPB, kb_k1 = min(kb_k0 + T::KPB, p.K);
-                // the groups meeting [kb_k0, kb_k1) in order, from the running group gcur (no division: a
-                // division per block on every wave saturates the CU's scalar unit)
-                for (;;) {
-                    const int ghi = gend, glo = gend - gp.G;
-                    const bool whole = glo <= kb_k0 && ghi >= kb_k1;
-#pragma unroll
-                    for (int st = 0; st < T::STEPS; st++) {
-                        const int kk = kb_k0 + a_koff<KIND>(st, lane >> 4);
-                        const bool in = whole || (kk >= glo && kk < ghi);
-#pragma unroll
-                        for (int i = 0; i < P::MTW; i++) {
-                            const v4i a = in ? afr[kbl][st][i] : v4i{0, 0, 0, 0};
-#pragma unroll
-                            for (int jn = 0; jn < P::NTW; jn++) acc[i][jn] = mma(a, bop[kbl][jn][st], acc[i][jn]);
-                        }
-                    }
-                    if (ghi > kb_k1) break; // the group runs on into the next block
-                    close_group(); // group gcur closes in this block
-                    gend += gp.G;
-                    if (ghi == kb_k1) break;
-                }
-            }
         }
     }
     wait_vmcnt<0>();
@@ -1044,7 +913,7 @@ __device__ __forceinline__ void tiled2_body(const orkh_mm &p, int mtiles, int nt
     // W4A4 M=256 K=N=4096 12.93 -> 12.62 us, fp16 M=128 K=N=2048 8.91 -> 8.77; slower on the other K-group tiles
     // (int8 M=128 32 x 32 6.35 -> 6.57, W4A8 M=64 32 x 64 7.16 -> 7.20) and on the tiles without K groups (int8
     // M=512 64 x 192 13.88 -> 14.51), so only here.
-    if constexpr (GR == 0 && (t2_xg<KIND, BM, BN, GR>() == 2 || (KIND == ORKH_F16 && BM == 32 && BN == 32))) {
+    if constexpr (t2_xg<KIND, BM, BN>() == 2 || (KIND == ORKH_F16 && BM == 32 && BN == 32)) {
         constexpr int SPAD = BN + 4; // words per parked row: a row's 16-lane store groups start in different banks
         static_assert((size_t)P::WK * BM * SPAD * sizeof(c_t) <= (size_t)R * P::SLOT, "partial tiles fit the ring");
         c_t *Ts = (c_t *)sm;
@@ -1115,10 +984,9 @@ __device__ __forceinline__ void tiled2_body(const orkh_mm &p, int mtiles, int nt
 
     // epilogue: one 64-bit base per lane (its first row and column), 32-bit offsets from it
     const int mr0 = m0 + wm * P::MTW * 16 + (lane >> 4) * 4, nc0 = (nb0 + wn * P::NTW) * 16 + (lane & 15);
-    const bool split = !GR && nT > ntiles_all;
+    const bool split = nT > ntiles_all;
     const size_t ldc = split ? (size_t)p.N : (size_t)p.ldc;
-    using o_t = typename std::conditional<GR != 0, float, c_t>::type;
-    o_t *Cl = (split ? (o_t *)ws + (size_t)ks * p.M * p.N : (o_t *)p.C) + (size_t)mr0 * ldc + nc0;
+    c_t *Cl = (split ? (c_t *)ws + (size_t)ks * p.M * p.N : (c_t *)p.C) + (size_t)mr0 * ldc + nc0;
 #pragma unroll
     for (int i = 0; i < P::MTW; i++)
 #pragma unroll
@@ -1128,10 +996,7 @@ __device__ __forceinline__ void tiled2_body(const orkh_mm &p, int mtiles, int nt
             for (int r = 0; r < 4; r++) {
                 if (mr0 + i * 16 + r >= p.M) continue;
                 const uint32_t off = (uint32_t)(i * 16 + r) * (uint32_t)ldc + (uint32_t)(jn * 16);
-                if constexpr (GR) {
-                    if (p.c_wt) store_wt(&Cl[off], cacc[i][jn][r]);
-                    else Cl[off] = cacc[i][jn][r];
-                } else if (p.c_wt) store_wt(&Cl[off], finish<KIND>(acc[i][jn][r]));
+                if (p.c_wt) store_wt(&Cl[off], finish<KIND>(acc[i][jn][r]));
                 else Cl[off] = finish<KIND>(acc[i][jn][r]);
             }
         }
@@ -1139,8 +1004,7 @@ __device__ __forceinline__ void tiled2_body(const orkh_mm &p, int mtiles, int nt
 
 template <int KIND, int BM, int BN, int KS, bool AL, int RC = 0>
 __global__ __launch_bounds__(1024) void k_tiled2(orkh_mm p, int mtiles, int ntiles_all, int kbs, void *ws) {
-    tiled2_body<KIND, BM, BN, KS, 0, AL, RC>(p, mtiles, ntiles_all, kbs, ws, T2Group{0, nullptr, nullptr},
-                                             (int)blockIdx.x, (int)gridDim.x);
+    tiled2_body<KIND, BM, BN, KS, AL, RC>(p, mtiles, ntiles_all, kbs, ws, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // k_tiled2m: up to ORKH_TGROUP_MAX matmuls of one kind, M and K in one launch (the multi-matmul submit): task t's
@@ -1158,16 +1022,7 @@ __global__ __launch_bounds__(1024) void k_tiled2m(T2Multi g) {
     while (t + 1 < g.n && (int)blockIdx.x >= g.wg0[t + 1]) t++;
     const int local = (int)blockIdx.x - g.wg0[t];
     if (local >= g.tiles[t]) return;
-    tiled2_body<KIND, BM, BN, KS, 0, AL>(g.p[t], g.mtiles[t], g.tiles[t], g.p[t].KB, nullptr, T2Group{0, nullptr, nullptr},
-                                         local, g.tiles[t]);
-}
-
-// Grouped runs (never K-split: the groups close in order inside one workgroup). GR 2: every group is whole
-// K-blocks (G % KPB == 0), so the stage runs as in the plain kernel and a group closes after the K-block that ends
-// it; GR 1: any G % 32 == 0, walked K-block by K-block with a group test per MFMA step.
-template <int KIND, int BM, int BN, int KS, int GR, bool AL>
-__global__ __launch_bounds__(1024) void k_tiled2g(orkh_mm p, int mtiles, int ntiles_all, T2Group gp) {
-    tiled2_body<KIND, BM, BN, KS, GR, AL>(p, mtiles, ntiles_all, p.KB, nullptr, gp, (int)blockIdx.x, (int)gridDim.x);
+    tiled2_body<KIND, BM, BN, KS, AL>(g.p[t], g.mtiles[t], g.tiles[t], g.p[t].KB, nullptr, local, g.tiles[t]);
 }
 
 // Dynamic LDS of k_tiled: KG groups x 2 stage buffers of A fragments, or (KG > 1) the 4-wave partial
@@ -1500,7 +1355,7 @@ constexpr bool t2_ring2_ok() {
 
 template <int KIND, int BM, int BN>
 int launch_tiled2_v(const orkh_mm *p, const orkh_plan *q, hipStream_t s) {
-    constexpr int XG = t2_xg<KIND, BM, BN, 0>();
+    constexpr int XG = t2_xg<KIND, BM, BN>();
     constexpr int KS = t2_ks<KIND, BM, BN, XG>();
     if (q->ring == 2) {
         if constexpr (t2_ring2_ok<KIND, BM, BN, XG, KS>()) return launch_tiled2_r<KIND, BM, BN, 2>(p, q, s);
@@ -1512,7 +1367,7 @@ int launch_tiled2_v(const orkh_mm *p, const orkh_plan *q, hipStream_t s) {
 
 template <int KIND, int BM, int BN, int RC>
 int launch_tiled2_r(const orkh_mm *p, const orkh_plan *q, hipStream_t s) {
-    constexpr int XG = t2_xg<KIND, BM, BN, 0>();
+    constexpr int XG = t2_xg<KIND, BM, BN>();
     constexpr int KS = t2_ks<KIND, BM, BN, XG>();
     using P = T2<KIND, BM, BN, KS, XG, RC>;
     const bool al = q->aline && P::LINE_OK;
@@ -1536,7 +1391,7 @@ int launch_tiled2_r(const orkh_mm *p, const orkh_plan *q, hipStream_t s) {
 
 template <int KIND, int BM, int BN>
 int launch_tiled2m_v(T2Multi &g, const orkh_plan *q, hipStream_t s) {
-    constexpr int XG = t2_xg<KIND, BM, BN, 0>();
+    constexpr int XG = t2_xg<KIND, BM, BN>();
     constexpr int KS = t2_ks<KIND, BM, BN, XG>();
     using P = T2<KIND, BM, BN, KS, XG>;
     const bool al = q->aline && P::LINE_OK;
@@ -1750,76 +1605,14 @@ extern "C" int orkh_mm_launch_group(const orkh_group *g, int wpg, void *stream) 
     return 0;
 }
 
-namespace {
-// Stage depth of a grouped run whose groups are whole K-blocks: the plain kernel's, except for uniform int4, whose
-// one-K-block stages (12 KiB on 64 x 64, whose plain runs take four K-blocks on the 2 x 2 x 4 wave grid that grouped
-// runs cannot use) keep too few bytes in flight per CU: four K-blocks on 64 x 64, two on 64 x 192, or two, or the plain
-// depth, where the larger ring and the tile's scales do not fit the LDS together. Measured against one K-block
-// (graph-timed, us, W4A4 K=N=4096 unless given): 64 x 64 G=128 M=256 20.11 -> 18.54, M=128 19.72 -> 18.10, G=256
-// 17.34 -> 15.65, K=8192 G=128 (two K-blocks) 36.49 -> 33.11; 64 x 192 M=512 35.79 -> 35.17, K=2048 N=6144 M=256
-// 19.83 -> 19.48. With groups inside a K-block (GR 1) two K-blocks measured slower (G=64 34.88 -> 35.34), so those
-// keep the plain depth.
-template <int KIND, int BM, int BN> constexpr int t2g_ks() {
-    return KIND != ORKH_I4U ? t2_ks<KIND, BM, BN>() : BN == 64 ? 4 : 2;
-}
-
-template <int KIND, int BM, int BN, int KS>
-int launch_tiled2g_k(const orkh_mm *p, const T2Group &gp, hipStream_t s, size_t sc, bool aline) {
-    using P = T2<KIND, BM, BN, KS>;
-    const bool whole = gp.G % KT<KIND>::KPB == 0;
-    const bool al = aline && P::LINE_OK;
-    auto kern = whole ? (al ? k_tiled2g<KIND, BM, BN, KS, 2, true> : k_tiled2g<KIND, BM, BN, KS, 2, false>)
-                      : (al ? k_tiled2g<KIND, BM, BN, KS, 1, true> : k_tiled2g<KIND, BM, BN, KS, 1, false>);
-    const size_t lds = P::LDS + sc;
-    const int Sk = p->K / gp.G;
-    if (lds > 163840) {
-        snprintf(g_lerr, sizeof g_lerr, "grouped tiled2 %dx%d: %d groups need %zu B of LDS", BM, BN, Sk, lds);
-        return -2;
-    }
-    static lds_flags attr[2][2]; // per instantiation: allow up to 160 KiB of dynamic LDS
-    if (lds_limit((const void *)kern, 163840, attr[whole][al])) return -1;
-    const int mtiles = (p->M + BM - 1) / BM;
-    const int ntiles = (p->N / 16 + P::NB - 1) / P::NB;
-    if ((long)mtiles * ntiles >= (1L << 24)) { // the kernel's tile-index division is exact below 2^24
-        snprintf(g_lerr, sizeof g_lerr, "grouped tiled2: %ld workgroups", (long)mtiles * ntiles);
-        return -2;
-    }
-    hipLaunchKernelGGL(kern, dim3(mtiles * ntiles), dim3(1024), lds, s, *p, mtiles, mtiles * ntiles, gp);
-    return 0;
-}
-
-template <int KIND, int BM, int BN>
-int launch_tiled2g_v(const orkh_mm *p, const T2Group &gp, hipStream_t s, bool al) {
-    const int Sk = p->K / gp.G;
-    const size_t sc = (size_t)((BM * Sk * 4 + 1023) / 1024 + (Sk * BN * 4 + 1023) / 1024) * 1024; // the tile's scales
-    constexpr int KD = t2g_ks<KIND, BM, BN>(), K1 = t2_ks<KIND, BM, BN>();
-    const bool whole = gp.G % KT<KIND>::KPB == 0;
-    if constexpr (KD != K1) {
-        if (whole && T2<KIND, BM, BN, KD>::LDS + sc <= 163840) return launch_tiled2g_k<KIND, BM, BN, KD>(p, gp, s, sc, al);
-    }
-    if constexpr (KD > 2 && K1 < 2) {
-        if (whole && T2<KIND, BM, BN, 2>::LDS + sc <= 163840) return launch_tiled2g_k<KIND, BM, BN, 2>(p, gp, s, sc, al);
-    }
-    return launch_tiled2g_k<KIND, BM, BN, K1>(p, gp, s, sc, al);
-}
-
-template <int KIND>
-int launch_tiled2g(const orkh_mm *p, const orkh_plan *q, const T2Group &gp, hipStream_t s) {
-    if (q->bm == 64 && q->bn == 192) return launch_tiled2g_v<KIND, 64, 192>(p, gp, s, q->aline);
-    if (q->bm == 64 && q->bn == 64) return launch_tiled2g_v<KIND, 64, 64>(p, gp, s, q->aline);
-    snprintf(g_lerr, sizeof g_lerr, "grouped tiled2 plan: %dx%d unsupported", q->bm, q->bn);
-    return -2;
-}
-} // namespace
-
 extern "C" int orkh_tiled2_ring2_ok(int kind, int bm, int bn) {
 #define ORKH_RING2(KIND)                                                                                     \
-    if (bm == 128 && bn == 128) return (int)t2_ring2_ok<KIND, 128, 128, t2_xg<KIND, 128, 128, 0>(),            \
-                                                        t2_ks<KIND, 128, 128, t2_xg<KIND, 128, 128, 0>()>()>(); \
-    if (bm == 128 && bn == 96) return (int)t2_ring2_ok<KIND, 128, 96, t2_xg<KIND, 128, 96, 0>(),               \
-                                                       t2_ks<KIND, 128, 96, t2_xg<KIND, 128, 96, 0>()>()>();    \
-    if (bm == 64 && bn == 192) return (int)t2_ring2_ok<KIND, 64, 192, t2_xg<KIND, 64, 192, 0>(),               \
-                                                       t2_ks<KIND, 64, 192, t2_xg<KIND, 64, 192, 0>()>()>();    \
+    if (bm == 128 && bn == 128) return (int)t2_ring2_ok<KIND, 128, 128, t2_xg<KIND, 128, 128>(),            \
+                                                        t2_ks<KIND, 128, 128, t2_xg<KIND, 128, 128>()>()>(); \
+    if (bm == 128 && bn == 96) return (int)t2_ring2_ok<KIND, 128, 96, t2_xg<KIND, 128, 96>(),               \
+                                                       t2_ks<KIND, 128, 96, t2_xg<KIND, 128, 96>()>()>();    \
+    if (bm == 64 && bn == 192) return (int)t2_ring2_ok<KIND, 64, 192, t2_xg<KIND, 64, 192>(),               \
+                                                       t2_ks<KIND, 64, 192, t2_xg<KIND, 64, 192>()>()>();    \
     return 0;
     switch (kind) {
     case ORKH_I8: ORKH_RING2(ORKH_I8)
@@ -1828,24 +1621,6 @@ extern "C" int orkh_tiled2_ring2_ok(int kind, int bm, int bn) {
     default: return 0;
     }
 #undef ORKH_RING2
-}
-
-extern "C" int orkh_tiled2_ring_lds(int kind, int bm, int bn) {
-#define ORKH_RING(KIND)                                                                                      \
-    if (bm == 64 && bn == 64) return (int)T2<KIND, 64, 64, t2_ks<KIND, 64, 64>()>::LDS;                       \
-    if (bm == 64 && bn == 192) return (int)T2<KIND, 64, 192, t2_ks<KIND, 64, 192>()>::LDS;                    \
-    if (bm == 128 && bn == 128) return (int)T2<KIND, 128, 128, t2_ks<KIND, 128, 128>()>::LDS;                 \
-    if (bm == 128 && bn == 96) return (int)T2<KIND, 128, 96, t2_ks<KIND, 128, 96>()>::LDS;                    \
-    if (bm == 256 && bn == 256) return (int)T2<KIND, 256, 256, t2_ks<KIND, 256, 256>()>::LDS;                 \
-    return -1;
-    switch (kind) {
-    case ORKH_I8: ORKH_RING(ORKH_I8)
-    case ORKH_I4U: ORKH_RING(ORKH_I4U)
-    case ORKH_NF4: ORKH_RING(ORKH_NF4)
-    case ORKH_F16: ORKH_RING(ORKH_F16)
-    default: return -1;
-    }
-#undef ORKH_RING
 }
 
 extern "C" int orkh_mm_launch_grouped(const orkh_mm *p, const orkh_plan *q, int G, const float *aS, const float *bS,
@@ -1887,8 +1662,7 @@ extern "C" int orkh_mm_launch_grouped(const orkh_mm *p, const orkh_plan *q, int 
         pc.C = C;
         pc.ldc = ldc;
         pc.c_wt = q->cwt;
-        const T2Group gp = {G, aS, bS};
-        const int rc = p->kind == ORKH_I8 ? launch_tiled2g<ORKH_I8>(&pc, q, gp, s) : launch_tiled2g<ORKH_I4U>(&pc, q, gp, s);
+        const int rc = orkh_tiled2g_launch(&pc, q, G, aS, bS, stream);
         if (rc) return rc;
     } else {
         const int MT = p->M > 16 ? 4 : 1;

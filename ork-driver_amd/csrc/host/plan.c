@@ -661,55 +661,66 @@ int orki_plan_mm(const ork_npu *c, int rkind, int M, int K, int N, int KB, orkh_
 }
 
 /* Grouped-scale runs (ork_*_mm_run_grouped). The groups must close in ascending order inside one workgroup, so
- * K is never split. Few rows: k_grouped streams each 16-column panel (and re-reads A per panel). With more
- * rows, int8 and uniform int4 take the LDS-ring kernel at the unsplit 64-row tile (64x192 or 64x64) the time
- * model prices lowest, when the tile's scales fit in LDS beside its ring (else 64x64, else k_grouped):
- *   from 32 rows when every group is whole 128-k spans (G % 128 == 0: the stage runs as in the plain kernel and a
- *   group closes after the K-block that ends it; e.g. W4A4 K=N=4096 G=128: 42.9 -> 21.6 us at M=256, since 18.5
- *   with deeper stages);
- *   from 128 rows otherwise (groups can end inside K-blocks and the kernel walks them K-block by K-block).
+ * K is never split. Few rows: k_grouped streams each 16-column panel (and re-reads A per panel, 64 rows at a time above
+ * 16). With more rows, int8 and uniform int4 take k_tiled2g at the tile that the prices below make cheapest:
+ *   from 32 rows where every group is whole 128-k spans (W4A4 K=N=4096 G=128 M=32: 16.0 us k_grouped, 12.0 64 x 64);
+ *   from 17 where groups are one MFMA step (G = 32 or 64), K >= 1024 and N >= 512 (M=17, K=N=4096, W4A4 G=64: 25.9 ->
+ *   15.4 us, int8 G=32: 49.1 -> 24.2; they meet at K=1024, N=1536: int8 G=64 6.8 and 6.3; at 16 rows k_grouped wins,
+ *   12.2 to 15.4);
+ *   from 128 otherwise (a run-time count of steps per group: int8 K=3072 N=512 G=192 M=64 11.4 k_grouped, 12.1 64 x 64,
+ *   M=256 12.8 and 12.1).
+ * The kernel's index divisions are exact below 2^24, hence the bound on K.
  * NF4 stays on k_grouped (its codebook decode would repeat in every wave row).
- * ORK_PLAN=stream|tiled forces either (tests, A/B). */
+ * ORK_PLAN=stream|tiled forces either (tests, A/B), ORK_TILE=BMxBN one of the tiles. */
 #define ORKI_GROUPED_TILED_M 32
+#define ORKI_GROUPED_TILED_M_STEP 17
 #define ORKI_GROUPED_TILED_M_PARTIAL 128
+/* A k_tiled2g tile's time in us: a + rounds * (b + K / 1024 * (c + d * 64 / G)), rounds of one workgroup a CU: c is the
+ * operands' delivery, d the closing of groups. Fitted to 13 row counts from 32 to 2048 at five (K, N) from 1024 to 6144
+ * and seven G from 32 to 512; over them the cheapest by price is within 8% of the fastest, 0.03% in the mean, e.g. (us)
+ * W4A4 K=N=4096 G=128: 12.8 on 64 x 64 at M=256 (25.6 on 64 x 192), 24.8 on it and 30.5 on 128 x 128 at M=512, 31.3 on
+ * 128 x 128 at M=1000 (48.0 on 64 x 64), 56.5 on 128 x 256 at M=2048 (62.6 on 128 x 128). */
+static const struct grouped_fit { int rkind, bm, bn; double a, b, c, d; } grouped_fits[] = {
+    {ORKH_I4U, 64, 64, 0.80, 2.41, 1.59, 2.08},  {ORKH_I4U, 64, 128, 0.38, 3.13, 2.94, 3.23},
+    {ORKH_I4U, 64, 192, 0.00, 3.74, 3.56, 4.78}, {ORKH_I4U, 128, 128, 0.00, 4.16, 3.94, 6.21},
+    {ORKH_I4U, 128, 256, 0.00, 5.53, 7.55, 9.97},
+    {ORKH_I8, 64, 64, 0.89, 2.32, 2.05, 1.60},   {ORKH_I8, 64, 128, 0.15, 3.18, 2.64, 3.11},
+    {ORKH_I8, 64, 192, 0.12, 3.54, 4.19, 3.84},  {ORKH_I8, 128, 128, 0.00, 3.74, 4.92, 5.03},
+    {ORKH_I8, 128, 256, 0.00, 5.16, 7.56, 7.85},
+};
 void orki_plan_grouped(const ork_npu *c, int rkind, int M, int K, int N, int KB, int G, orkh_plan *q) {
     memset(q, 0, sizeof *q);
     const int cu = (c && c->cores > 0) ? c->cores : 256;
     const char *force = knob(c, "ORK_PLAN");
-    int tiled = M >= (G % 128 == 0 ? ORKI_GROUPED_TILED_M : ORKI_GROUPED_TILED_M_PARTIAL);
+    int tiled = M >= (G % 128 == 0                       ? ORKI_GROUPED_TILED_M
+                      : G <= 64 && K >= 1024 && N >= 512 ? ORKI_GROUPED_TILED_M_STEP
+                                                         : ORKI_GROUPED_TILED_M_PARTIAL);
     if (force && !strcmp(force, "stream")) tiled = 0;
     if (force && !strcmp(force, "tiled")) tiled = 1;
-    if (tiled && rkind != ORKH_NF4) {
+    if (tiled && rkind != ORKH_NF4 && K < 1 << 24) {
         const char *tf = knob(c, "ORK_TILE");
         int fbm, fbn;
-        if (tf && sscanf(tf, "%dx%d", &fbm, &fbn) == 2 && fbm == 64 && (fbn == 64 || fbn == 192)) {
-            q->algo = ORKH_ALGO_TILED2;
-            q->bm = fbm;
-            q->bn = fbn;
-        } else {
-            tiled2_best(rkind, M, N, KB, cu, 1, 2, q); /* the 64-row tiles: the larger ones spill with the fp32 sums */
+        if (!tf || sscanf(tf, "%dx%d", &fbm, &fbn) != 2) fbm = fbn = 0;
+        double best = -1;
+        for (size_t i = 0; i < sizeof grouped_fits / sizeof grouped_fits[0]; i++) {
+            const struct grouped_fit *f = &grouped_fits[i];
+            if (f->rkind != rkind || (f->bn == 256 && G % 64)) continue;
+            const long w = (long)cdiv(M, f->bm) * cdiv(N, f->bn);
+            const double t = f->a + (double)((w + cu - 1) / cu) * (f->b + K / 1024.0 * (f->c + f->d * 64 / G));
+            const int forced = f->bm == fbm && f->bn == fbn;
+            if (best >= 0 && t >= best - 1e-9 && !forced) continue;
+            best = t;
+            q->bm = f->bm;
+            q->bn = f->bn;
+            if (forced) break;
         }
-        /* the tile's scales (BM x K/G and K/G x BN floats) sit in LDS beside the stage ring */
-        const int Sk = K / G;
-        for (int pass = 0; pass < 2 && q->algo == ORKH_ALGO_TILED2; pass++) {
-            const long sc = ((long)q->bm * Sk * 4 + 1023) / 1024 * 1024 + ((long)Sk * q->bn * 4 + 1023) / 1024 * 1024;
-            const int ring = orkh_tiled2_ring_lds(rkind, q->bm, q->bn);
-            if (ring > 0 && ring + sc <= 163840) {
-                q->ksplit = 1;
-                q->kbs = KB;
-                /* A stages as whole row lines where the stage row is whole lines (the kernel checks) */
-                const char *fa = knob(c, "ORK_ALINE");
-                q->aline = fa ? atoi(fa) != 0 : 1;
-                /* write-through C stores on a grid of one round, as for the plain runs */
-                const char *fc = knob(c, "ORK_CWT");
-                q->cwt = fc ? atoi(fc) != 0 : (long)cdiv(M, q->bm) * cdiv(N / 16, q->bn / 16) <= cu;
-                return;
-            }
-            if (q->bm == 64 && q->bn == 64) break;
-            q->bm = 64; /* the smallest ring */
-            q->bn = 64;
-        }
-        memset(q, 0, sizeof *q);
+        q->algo = ORKH_ALGO_TILED2;
+        q->ksplit = 1;
+        q->kbs = KB;
+        /* write-through C stores on a grid of one round, as for the plain runs */
+        const char *fc = knob(c, "ORK_CWT");
+        q->cwt = fc ? atoi(fc) != 0 : (long)cdiv(M, q->bm) * cdiv(N / 16, q->bn / 16) <= cu;
+        return;
     }
     /* one row: the half-panel VALU kernel (k_grouped_gemv) where the groups' partials fit its LDS (K/G <= 512), runs
      * as the GEMV's (ORK_PLAN=stream keeps k_grouped). Graph-timed against k_grouped (us): W4A4 K=N=4096 G=128

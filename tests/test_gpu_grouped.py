@@ -245,6 +245,64 @@ def test_grouped_tiled_exact(npu, tile, kind, M, K, N, G):
     L.ork_mm_free(npu.h, w)
 
 
+@pytest.mark.parametrize("tile", ["64x64", "64x128", "64x192", "128x128", "128x256"])
+@pytest.mark.parametrize("M,K,N,G", [
+    (1, 1024, 64, 32),      # one row, one panel group; two closes per 64 k
+    (129, 1056, 192, 32),   # one row past a tile; the last stage holds 32 k
+    (127, 1088, 320, 64),   # a close per step; the last stage holds 64 k, half a panel block of int4
+    (65, 1152, 448, 128),   # odd K-blocks per stage
+    (130, 1280, 256, 256),  # half a four-line stage at the end
+    (64, 1920, 256, 384),   # groups end inside stages; run-time step counts
+    (200, 1152, 320, 192),  # the same, 64-k steps; K tail
+    (97, 672, 192, 96),     # 32-k steps; K tail
+    (257, 2048, 512, 512),  # whole stages per group; two row tiles and one row
+])
+def test_grouped_tiles_exact(npu, tile, M, K, N, G):
+    """Every tile of the grouped kernel in each form of its groups' ends, int8 and W4A4, at partial tiles and stages:
+    the oracle's bits (each float operation is the oracle's, in its order), and no store outside C."""
+    L = ork.lib()
+    rng = np.random.default_rng(M + K + N + G)
+    aS = rng.uniform(1e-3, 1e-2, size=(M, K // G)).astype(np.float32)
+    bS = rng.uniform(1e-3, 1e-2, size=(K // G, N)).astype(np.float32)
+    for kind, lo in (("i8", -128), ("w4a4", -8)):
+        _say("grouped tiles", kind, M, K, N, G, tile)
+        A, B = (rng.integers(lo, -lo, size=z, dtype=np.int8) for z in ((M, K), (K, N)))
+        if kind == "i8":
+            w = npu.pack_i8(B)
+            assert L.ork_w_set_group(w, G) == 0
+        else:
+            w = L.ork_i4_mm_pack_grouped(npu.h, K, N, ork.ptr(B), G)
+        assert w
+        C = np.full((M + 2, N), -7, np.float32)
+        fn = L.ork_i8_mm_run_grouped if kind == "i8" else L.ork_i4_mm_run_grouped
+        env = {"ORK_PLAN": "tiled", "ORK_TILE": tile}
+        rc, _ = _env_run(env, lambda h, w_, m, a, s, t, c: fn(h, w_, m, a, s, t, ork.ptr(C[1:])), npu, w, A, aS, bS)
+        assert rc == 0 and np.array_equal(C[1:-1], O.gemm_grouped(A, B, aS, bS, G))
+        assert (C[0] == -7).all() and (C[-1] == -7).all()
+        L.ork_mm_free(npu.h, w)
+
+
+@pytest.mark.parametrize("G", [32, 64, 96, 128])
+def test_grouped_rule_either_side(npu, G):
+    """The default plan on both sides of each row count where the rule changes kernel, against the oracle's bits."""
+    L = ork.lib()
+    K, N = 1152, 512
+    first = {32: 17, 64: 17, 96: 128, 128: 32}[G]
+    rng = np.random.default_rng(G)
+    B = rng.integers(-128, 128, size=(K, N), dtype=np.int8)
+    w = npu.pack_i8(B)
+    assert L.ork_w_set_group(w, G) == 0
+    bS = rng.uniform(1e-3, 1e-2, size=(K // G, N)).astype(np.float32)
+    for M in (first - 1, first):
+        _say("grouped rule", G, M)
+        assert npu.grouped_plan_name(w, M).startswith("tiled2g_i8_" if M == first else "grouped_i8_mt")
+        A = rng.integers(-127, 128, size=(M, K), dtype=np.int8)
+        aS = rng.uniform(1e-3, 1e-2, size=(M, K // G)).astype(np.float32)
+        rc, C = _run(L.ork_i8_mm_run_grouped, npu, w, A, aS, bS)
+        assert rc == 0 and np.array_equal(C, O.gemm_grouped(A, B, aS, bS, G))
+    L.ork_mm_free(npu.h, w)
+
+
 def test_grouped_plan_names(npu):
     """Default plans: one row runs the half-panel VALU kernel (k_grouped_gemv), a few rows stream panels
     (k_grouped); int8 / uniform int4 take the LDS-ring kernel from 32 rows when G % 128 == 0 and from 128 rows
