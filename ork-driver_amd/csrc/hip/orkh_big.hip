@@ -10,7 +10,9 @@
 //    256 x 256 takes one and a half);
 //  - stages of 128 activation bytes a row (whole cache lines, a_lds's swizzle) and one barrier per stage, with the
 //    next phase's LDS operands read into registers before the current phase's MFMAs;
-//  - load addresses as one per-lane offset plus a scalar stage offset, so a load costs one instruction;
+//  - load addresses as one per-lane offset plus a scalar stage offset, and each load's kind known at compile time, so a
+//    load costs one instruction (us at M=K=N=4096 with a test of the kind per load: uniform int4 54.8, now 53.4, NF4 73.7,
+//    now 70.4, fp16 117.5, now 116.4; fp16 K=N=4096 M=500 on 128 x 192 48.3, now 44.5);
 //  - an XCD's run of tiles covers GM rows of tiles x several columns instead of one column of all rows, so its L2 takes
 //    about a third less from the next level;
 //  - the MFMA operands swapped (D = B^T A^T), so that a lane holds four consecutive columns of one row and C goes out
@@ -34,13 +36,16 @@ template <int KIND, int BM, int BN> struct BG {
     static constexpr int MTW = BM / 16 / WM, NTW = BN / 16 / WN; // 16 x 16 blocks per wave
     static constexpr int MHN = MTW >= 4 ? 2 : 1, MH = MTW / MHN; // a phase: one K step x MH row blocks
     static constexpr int BPP = NIB ? 1 : 2;                      // panel blocks per panel and stage
-    static constexpr int NA = BM / 8, NL = NA + BN / 16 * BPP;   // 1 KiB loads per stage: 8 rows of A, or one block
-    static constexpr int LPW = (NL + NW - 1) / NW;               // per wave; a last one without work lands in a junk block
-    static constexpr int SLOT = (NL + (LPW * NW > NL)) * 64;     // 16-byte units
+    // 1 KiB loads per stage: 8 rows of A, or one block of B. QA and QB per wave (so that a load's kind is known at compile
+    // time); a B load without work (QB * NW > NBL) lands in a junk block
+    static constexpr int NA = BM / 8, NBL = BN / 16 * BPP;
+    static constexpr int QA = NA / NW, QB = (NBL + NW - 1) / NW, LPW = QA + QB;
+    static constexpr int SLOT = (NA + NBL + (QB * NW > NBL)) * 64; // 16-byte units
     static constexpr int RMAX = 163840 / (SLOT * 16), R = RMAX < 4 ? RMAX : 4;
     static constexpr int LDS = R * SLOT * 16;
     static constexpr int GM = 1024 / BM; // tile rows of an XCD's run: 1024 rows
-    static_assert(R >= 2 && MTW * WM * 16 == BM && NTW * WN * 16 == BN && MH * MHN == MTW, "tile");
+    static_assert(R >= 2 && MTW * WM * 16 == BM && NTW * WN * 16 == BN && MH * MHN == MTW && QA * NW == NA && NW % BPP == 0,
+                  "tile");
 };
 
 // MFMA operand of K step kk from a lane's panel chunk (nibble kinds: half the chunk per step, as decode())
@@ -95,32 +100,33 @@ __device__ __forceinline__ void big_body(const orkh_mm &p, int mtiles, int ntile
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)sm;
     const Lut L = {p.lut[0], p.lut[1], p.lut[2], p.lut[3]};
 
-    // this wave's loads: i = wv + q * NW; rows 8 i .. 8 i + 7 of A (lane l: row l / 8, slot l % 8 holds chunk
-    // slot ^ (l / 8) ^ (i & 1)), or panel block i - NA
-    uint32_t vo[LPW];
+    // this wave's loads: A rows 8 i .. 8 i + 7, i = wv + q * NW (lane l: row l / 8, slot l % 8 holds chunk
+    // slot ^ (l / 8) ^ (i & 1)), and panel blocks i = wv + q * NW
+    uint32_t va[P::QA], vb[P::QB];
+    const uint32_t ch = (uint32_t)(((lane & 7) ^ (lane >> 3) ^ (wv & 1)) * 16); // the chunk's byte in the stage row (NW is even)
 #pragma unroll
-    for (int q = 0; q < LPW; q++) {
-        const int i = wv + q * NW, ib = i - NA;
-        const int row = m0 + i * 8 + (lane >> 3), nb = nb0 + ib / P::BPP;
-        if (i < NA) vo[q] = row < p.M ? (uint32_t)row * lda_b + (uint32_t)(((lane & 7) ^ (lane >> 3) ^ (i & 1)) * 16) : OOB;
-        else vo[q] = i < P::NL && nb < NBt ? ((uint32_t)nb * p.KB + ib % P::BPP) * 1024u + lane * 16u : OOB;
+    for (int q = 0; q < P::QA; q++) {
+        const int row = m0 + (wv + q * NW) * 8 + (lane >> 3);
+        va[q] = row < p.M ? (uint32_t)row * lda_b + ch : OOB;
+    }
+#pragma unroll
+    for (int q = 0; q < P::QB; q++) {
+        const int i = wv + q * NW, nb = nb0 + i / P::BPP;
+        vb[q] = i < P::NBL && nb < NBt ? ((uint32_t)nb * p.KB + i % P::BPP) * 1024u + lane * 16u : OOB;
     }
     const int nst = (p.KB + P::BPP - 1) / P::BPP;
-    auto issue = [&](int st) {
-        if (st >= nst) return;
-        const uint32_t slot = lds0 + (uint32_t)(st % R) * (P::SLOT * 16);
-        const bool tail = (uint32_t)st * 128 + 128 > kbytes; // the last stage of a K that is not whole stages
+    int ist = 0, islot = 0; // the next stage to issue and its slot
+    auto issue = [&] { // one stage per call, in order; straight-line: past K, A chunks and panel blocks read zeros
+        if (ist >= nst) return;
+        const uint32_t slot = lds0 + (uint32_t)islot * (P::SLOT * 16), sa = (uint32_t)ist * 128;
+        const bool oka = sa + ch < kbytes, okb = ist * P::BPP + wv % P::BPP < p.KB;
 #pragma unroll
-        for (int q = 0; q < LPW; q++) {
-            const int i = wv + q * NW;
-            uint32_t v = vo[q];
-            if (tail) { // A chunks and panel blocks past K read zeros
-                const uint32_t c = (uint32_t)(((lane & 7) ^ (lane >> 3) ^ (i & 1)) * 16);
-                if (i < NA ? (uint32_t)st * 128 + c >= kbytes : st * P::BPP + (i - NA) % P::BPP >= p.KB) v = OOB;
-            }
-            if (i < NA) lds_dma16s(Ar, v, (uint32_t)st * 128, slot + i * 1024);
-            else lds_dma16s(Br, v, (uint32_t)st * (P::BPP * 1024), slot + min(i, P::NL) * 1024);
-        }
+        for (int q = 0; q < P::QA; q++) lds_dma16s(Ar, oka ? va[q] : OOB, sa, slot + (wv + q * NW) * 1024);
+#pragma unroll
+        for (int q = 0; q < P::QB; q++)
+            lds_dma16s(Br, okb ? vb[q] : OOB, (uint32_t)ist * (P::BPP * 1024), slot + (NA + min(wv + q * NW, P::NBL)) * 1024);
+        ist++;
+        islot = islot + 1 == R ? 0 : islot + 1;
     };
 
     acc_t acc[P::MTW][P::NTW];
@@ -133,13 +139,13 @@ __device__ __forceinline__ void big_body(const orkh_mm &p, int mtiles, int ntile
     const int c0 = P::NIB ? (lane >> 4) * 2 : lane >> 4, c1 = P::NIB ? c0 + 1 : c0 + 4;
     const int ao0 = h * 64 + r7 * 8 + (c0 ^ r7 ^ h), ao1 = h * 64 + r7 * 8 + (c1 ^ r7 ^ h);
     v4i a[2][P::MH], b[2][P::NTW], raw[P::NIB ? P::NTW : 1];
-    auto rdA = [&](int st, int kk, int hh, v4i (&d)[P::MH]) {
-        const v4i *As = sm + (st % R) * P::SLOT + (wm * P::MTW + hh * P::MH) * 128 + (kk ? ao1 : ao0);
+    auto rdA = [&](int slot, int kk, int hh, v4i (&d)[P::MH]) {
+        const v4i *As = sm + slot * P::SLOT + (wm * P::MTW + hh * P::MH) * 128 + (kk ? ao1 : ao0);
 #pragma unroll
         for (int i = 0; i < P::MH; i++) d[i] = As[i * 128];
     };
-    auto rdB = [&](int st, int kk) { // nibble kinds: the stage's chunks (kk = 0), decoded by opB
-        const v4i *Bs = sm + (st % R) * P::SLOT + NA * 64 + (wn * P::NTW * P::BPP + kk) * 64 + lane;
+    auto rdB = [&](int slot, int kk) { // nibble kinds: the stage's chunks (kk = 0), decoded by opB
+        const v4i *Bs = sm + slot * P::SLOT + NA * 64 + (wn * P::NTW * P::BPP + kk) * 64 + lane;
 #pragma unroll
         for (int i = 0; i < P::NTW; i++) {
             if constexpr (P::NIB) raw[i] = Bs[i * 64];
@@ -161,8 +167,8 @@ __device__ __forceinline__ void big_body(const orkh_mm &p, int mtiles, int ntile
     // keeps each phase's LDS reads in front of its MFMAs
     auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
 
-#pragma unroll
-    for (int st = 0; st < R; st++) issue(st);
+#pragma unroll 1
+    for (int st = 0; st < R; st++) issue();
     if (nst >= R) wait_vmcnt<(R - 1) * LPW>();
     else wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();
@@ -170,25 +176,27 @@ __device__ __forceinline__ void big_body(const orkh_mm &p, int mtiles, int ntile
     rdB(0, 0);
     rdA(0, 0, 0, a[0]);
     opB(0);
+    int rs = 0; // slot of stage s
     for (int s = 0; s < nst; s++) {
+        const int rn = rs + 1 == R ? 0 : rs + 1;
         if constexpr (P::MHN == 2) {
-            rdA(s, 0, 1, a[1]);
+            rdA(rs, 0, 1, a[1]);
             fence();
             mm(0, a[0], b[0]);
             fence();
-            if constexpr (!P::NIB) rdB(s, 1);
-            rdA(s, 1, 0, a[0]);
+            if constexpr (!P::NIB) rdB(rs, 1);
+            rdA(rs, 1, 0, a[0]);
             opB(1);
             fence();
             mm(1, a[1], b[0]);
             fence();
-            rdA(s, 1, 1, a[1]);
+            rdA(rs, 1, 1, a[1]);
             fence();
             mm(0, a[0], b[1]);
             fence();
         } else {
-            if constexpr (!P::NIB) rdB(s, 1);
-            rdA(s, 1, 0, a[1]);
+            if constexpr (!P::NIB) rdB(rs, 1);
+            rdA(rs, 1, 0, a[1]);
             opB(1);
             fence();
             mm(0, a[0], b[0]);
@@ -200,15 +208,16 @@ __device__ __forceinline__ void big_body(const orkh_mm &p, int mtiles, int ntile
         else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        issue(s + R);
+        issue();
         if (s + 1 < nst) {
-            rdB(s + 1, 0);
-            rdA(s + 1, 0, 0, a[0]);
+            rdB(rn, 0);
+            rdA(rn, 0, 0, a[0]);
         }
         fence();
         mm(P::MHN - 1, a[1], b[1]);
         fence();
         opB(0); // (after the last stage: of what it holds, unused)
+        rs = rn;
     }
 
     // a lane holds row lane % 16, columns 4 (lane / 16) .. + 3 of each block
