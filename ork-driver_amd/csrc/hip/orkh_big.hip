@@ -11,8 +11,8 @@
 //  - stages of 128 activation bytes a row (whole cache lines, a_lds's swizzle) and one barrier per stage, with the
 //    next phase's LDS operands read into registers before the current phase's MFMAs;
 //  - load addresses as one per-lane offset plus a scalar stage offset, and each load's kind known at compile time, so a
-//    load costs one instruction (us at M=K=N=4096 with a test of the kind per load: uniform int4 54.8, now 53.4, NF4 73.7,
-//    now 70.4, fp16 117.5, now 116.4; fp16 K=N=4096 M=500 on 128 x 192 48.3, now 44.5);
+//    load costs one instruction (us at M=K=N=4096 with a test of the kind per load: uniform int4 54.8, then 53.4, NF4 73.7,
+//    then 70.4, fp16 117.5, then 116.4; fp16 K=N=4096 M=500 on 128 x 192 48.3, then 44.5);
 //  - an XCD's run of tiles covers GM rows of tiles x several columns instead of one column of all rows, so its L2 takes
 //    about a third less from the next level;
 //  - the MFMA operands swapped (D = B^T A^T), so that a lane holds four consecutive columns of one row and C goes out
@@ -43,6 +43,13 @@ template <int KIND, int BM, int BN> struct BG {
     static constexpr int SLOT = (NA + NBL + (QB * NW > NBL)) * 64; // 16-byte units
     static constexpr int RMAX = 163840 / (SLOT * 16), R = RMAX < 4 ? RMAX : 4;
     static constexpr int LDS = R * SLOT * 16;
+    // Where the loads of a stage go out (us at K=N=4096, all at the barrier, then spread): between the MFMA phases of the stage
+    // that runs R - 1 before it, where they do not hold the waves back while no MFMA runs: uniform int4 M=4096 256 x 256
+    // 53.4 -> 52.3, M=1000 128 x 192 26.4 -> 24.2; NF4 M=4096 256 x 256 70.8 -> 67.3; int8 M=1000 128 x 256 29.3 -> 27.6; fp16
+    // M=1000 128 x 256 51.6 -> 48.8. All at once after the barrier, R stages ahead, on two-slot rings (spread, a stage
+    // would have less than a stage's time to arrive) and NF4's 128-row tiles (its decode fills the phases: 40.3 -> 41.0).
+    static constexpr bool SPREAD = R >= 3 && !(KIND == ORKH_NF4 && BM == 128);
+    static constexpr int RA = SPREAD ? R - 1 : R; // stages issued ahead
     static constexpr int GM = 1024 / BM; // tile rows of an XCD's run: 1024 rows
     static_assert(R >= 2 && MTW * WM * 16 == BM && NTW * WN * 16 == BN && MH * MHN == MTW && QA * NW == NA && NW % BPP == 0,
                   "tile");
@@ -116,18 +123,30 @@ __device__ __forceinline__ void big_body(const orkh_mm &p, int mtiles, int ntile
     }
     const int nst = (p.KB + P::BPP - 1) / P::BPP;
     int ist = 0, islot = 0; // the next stage to issue and its slot
-    auto issue = [&] { // one stage per call, in order; straight-line: past K, A chunks and panel blocks read zeros
+    // part j of n of stage ist's loads, the last part going on to the next stage; straight-line: past K, A chunks and panel
+    // blocks read zeros
+    auto issue = [&](auto j, auto n) {
+        constexpr int q0 = LPW * decltype(j)::value / decltype(n)::value, q1 = LPW * (decltype(j)::value + 1) / decltype(n)::value;
         if (ist >= nst) return;
         const uint32_t slot = lds0 + (uint32_t)islot * (P::SLOT * 16), sa = (uint32_t)ist * 128;
         const bool oka = sa + ch < kbytes, okb = ist * P::BPP + wv % P::BPP < p.KB;
 #pragma unroll
-        for (int q = 0; q < P::QA; q++) lds_dma16s(Ar, oka ? va[q] : OOB, sa, slot + (wv + q * NW) * 1024);
-#pragma unroll
-        for (int q = 0; q < P::QB; q++)
-            lds_dma16s(Br, okb ? vb[q] : OOB, (uint32_t)ist * (P::BPP * 1024), slot + (NA + min(wv + q * NW, P::NBL)) * 1024);
-        ist++;
-        islot = islot + 1 == R ? 0 : islot + 1;
+        for (int z = q0; z < q1; z++) {
+            const int q = z < P::QA ? z : z - P::QA;
+            if (z < P::QA) lds_dma16s(Ar, oka ? va[q] : OOB, sa, slot + (wv + q * NW) * 1024);
+            else lds_dma16s(Br, okb ? vb[q] : OOB, (uint32_t)ist * (P::BPP * 1024), slot + (NA + min(wv + q * NW, P::NBL)) * 1024);
+        }
+        if (q1 == LPW) {
+            ist++;
+            islot = islot + 1 == R ? 0 : islot + 1;
+        }
     };
+    auto part = [&](auto j) { // after the stage's j-th phase but the last
+        if constexpr (P::SPREAD) issue(j, std::integral_constant<int, 2 * P::MHN - 1>{});
+    };
+    using J0 = std::integral_constant<int, 0>;
+    using J1 = std::integral_constant<int, 1>;
+    using J2 = std::integral_constant<int, 2>;
 
     acc_t acc[P::MTW][P::NTW];
 #pragma unroll
@@ -168,8 +187,8 @@ __device__ __forceinline__ void big_body(const orkh_mm &p, int mtiles, int ntile
     auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
 
 #pragma unroll 1
-    for (int st = 0; st < R; st++) issue();
-    if (nst >= R) wait_vmcnt<(R - 1) * LPW>();
+    for (int st = 0; st < P::RA; st++) issue(J0{}, J1{});
+    if (nst >= P::RA) wait_vmcnt<(P::RA - 1) * LPW>();
     else wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -183,16 +202,19 @@ __device__ __forceinline__ void big_body(const orkh_mm &p, int mtiles, int ntile
             rdA(rs, 0, 1, a[1]);
             fence();
             mm(0, a[0], b[0]);
+            part(J0{});
             fence();
             if constexpr (!P::NIB) rdB(rs, 1);
             rdA(rs, 1, 0, a[0]);
             opB(1);
             fence();
             mm(1, a[1], b[0]);
+            part(J1{});
             fence();
             rdA(rs, 1, 1, a[1]);
             fence();
             mm(0, a[0], b[1]);
+            part(J2{});
             fence();
         } else {
             if constexpr (!P::NIB) rdB(rs, 1);
@@ -200,15 +222,16 @@ __device__ __forceinline__ void big_body(const orkh_mm &p, int mtiles, int ntile
             opB(1);
             fence();
             mm(0, a[0], b[0]);
+            part(J0{});
             fence();
         }
         // Stage s + 1 has landed (this wave's share of it; the barrier covers the others'), and every wave's reads of
-        // stage s are done, so its slot takes stage s + R
+        // stage s are done, so its slot takes stage s + R (spread: while stage s + 1 runs)
         if (s + R <= nst) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"((R - 2) * LPW) : "memory");
         else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        issue();
+        if constexpr (!P::SPREAD) issue(J0{}, J1{});
         if (s + 1 < nst) {
             rdB(rn, 0);
             rdA(rn, 0, 0, a[0]);

@@ -555,7 +555,7 @@ static int plan_core(const ork_npu *c, int rkind, int M, int K, int N, int KB, o
  * 2891 (2891), NF4 4760 -> 3973 (3951), and no shape is slower than its former pick; NF4's 2% margin keeps two shapes
  * where k_big ran 4-5% slower. 256 x 256 picks always move: k_big was ahead on each. Some shapes, us: int8 K=N=4096
  * M=4096 65.0 -> 61.3, K=6144 N=2048 M=4096 63.3 -> 49.3, K=N=4096 M=2048 41.5 -> 35.2; fp16 K=2048 N=6144 M=4096 140.6
- * -> 114.3; uniform int4 K=N=4096 M=4096 89.8 -> 53.4; NF4 112.0 -> 70.4, K=2048 N=6144 M=1000 29.5 -> 24.2. At 512 rows
+ * -> 114.3; uniform int4 K=N=4096 M=4096 89.8 -> 52.3; NF4 112.0 -> 67.3, K=2048 N=6144 M=1000 29.5 -> 24.2. At 512 rows
  * and fewer the smaller tiles fill the CUs better and keep the run (int8 K=2048 N=6144 M=500 11.9 against 16.6), except
  * where N is large (N=12288 20.3 -> 17.6).
  * A context's planner overrides (ORK_PLAN, ORK_TILE and the others of orki_plan) turn the rule off, and ORK_PLAN=big with
