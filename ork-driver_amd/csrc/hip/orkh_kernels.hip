@@ -20,6 +20,7 @@
 //   k_tiled   large M: 256-thread workgroup owns a BM x BN output tile; A fragments and B blocks are
 //             staged through double-buffered LDS, each B byte crosses HBM once per XCD (the tile order
 //             groups all M-tiles of an N-tile onto one XCD's L2).
+// Many rows and grouped scales on tiles: orkh_big.hip and orkh_grouped.hip.
 // Integer results are exact (int32 accumulation, k order irrelevant). Uniform int4 nibbles are
 // widened to 16*v in an int8 lane (v in [-8,7] -> [-128,112]); the int32 sum is then exactly 16x the
 // true sum and an arithmetic >>4 recovers it.
