@@ -429,9 +429,13 @@ int q3_layer_rows(q3_model *m, int l, float *out, int rows) {
     return ork_dev_download(m->ctx, out, m->trace + (size_t)l * m->c.max_rows * H, (size_t)rows * H * 4) ? -1 : 0;
 }
 
-/* Prefill attention by blocks of rows from this many rows: below, its third launch costs more than it saves (two
- * layers at Qwen3-1.7B widths, blocks / row by row, us: M=8 166 / 161, M=16 166 / 163, M=24 178 / 173; M=64 161 / 167). */
+/* Prefill attention by blocks of rows: below BLOCK rows the row-by-row kernel, up to 256 k_attn_block, above that
+ * k_attn_scores and k_attn_pv, whose third launch and tiles of 64 keys want more rows. Whole prefills at Qwen3-1.7B
+ * widths with new inputs each time, us: two layers, M=20 / 31 block 221 / 226, by row 209 / 222; block / scores and P.V:
+ * two layers M=45 236 / 242, M=100 238 / 240, M=256 288 / 290, M=350 357 / 345, M=413 383 / 358, one layer M=224 184 /
+ * 186 and 185 / 192, M=300 220 / 213. (One workgroup per row that quantises as well, to save the launch: M=100 249.) */
 #define Q3_ATTN_BLOCK_ROWS 32
+#define Q3_ATTN_MANY_ROWS 257
 
 /* ---- one pass of the decoder over M rows ------------------------------------------------------------------- */
 static int pass(q3_model *m, int M, int decode) {
@@ -472,7 +476,7 @@ static int pass(q3_model *m, int M, int decode) {
         const int Sa = decode ? m->S : (M + Q3_CHUNK - 1) / Q3_CHUNK;
         q3_att at = {.M = M, .NH = NH, .NKV = NKV, .HD = HD, .S = Sa, .max_ctx = decode ? c->max_ctx : M,
                      .q = m->q, .kc = Ly->kc, .vc = Ly->vc, .st = m->st, .scale = 1.0f / sqrtf((float)HD),
-                     .part = m->part};
+                     .part = m->part, .rows = m->fused && M >= Q3_ATTN_BLOCK_ROWS};
         if (M == 1) { /* one row: attention does the q/k/v post-processing itself */
             at.cq = m->cq;
             at.ck = m->ck;
@@ -492,7 +496,7 @@ static int pass(q3_model *m, int M, int decode) {
                                m->rcos, m->rsin, m->st, m->q, Ly->kc, Ly->vc};
             CK(q3k_qkv_post(&qp, s));
         }
-        if (M >= Q3_ATTN_BLOCK_ROWS && m->fused) {
+        if (M >= Q3_ATTN_MANY_ROWS && m->fused) {
             /* part holds the scores and the chunk statistics: pad64(M) + 2 Sa floats per (row, head), of the
              * S * (HD + 2) it has (HD >= 64); the attention rows replace the queries */
             at.sc = m->part;

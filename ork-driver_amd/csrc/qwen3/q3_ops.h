@@ -60,7 +60,8 @@ typedef struct q3_att { /* grid (NKV * query-head sub-groups, S, M): Q3_CHUNK-ke
     const int *st;
     float scale;
     float *part; /* [M][NH][S][HD + 2]: P.V, then max and sum */
-    /* prefill by blocks of rows (q3k_attn_rows): row t is at position t, LP = M rounded up to 64 */
+    int rows;    /* unfused form: 1 = one workgroup per block of rows (k_attn_block), 0 = per row; same partials */
+    /* many rows (q3k_attn_rows): row t is at position t, LP = M rounded up to 64 */
     int sr;    /* rows of a scores workgroup (set by the launcher) */
     float *sc; /* scratch [M][NH][LP]: exp(score - chunk max) */
     float *ml; /* scratch [M][NH][S][2]: chunk max and sum */

@@ -7,6 +7,7 @@
 //   k_norm_quant_*    [embedding lookup | residual add of a matmul result] + RMSNorm + per-row int8 quant
 //   k_qkv_post        q/k/v dequant + per-head RMSNorm (Qwen3 q_norm / k_norm) + RoPE + KV-cache append
 //   k_attn_part       causal GQA attention over one Q3_CHUNK-key chunk: running max, sum and P.V per query head
+//   k_attn_block      the same partials for a block of a prefill's rows
 //   k_attn_scores / k_attn_pv  the same rows for a prefill by blocks of rows (chunks combined in registers)
 //   k_attn_quant      combine the chunks (log-sum-exp) + per-row int8 quant of the attention output
 //   k_swiglu_quant    gate/up dequant + silu(g) * u + per-row int8 quant
@@ -295,7 +296,117 @@ __global__ __launch_bounds__(256) void k_attn_part(q3_att p) {
     }
 }
 
-// Prefill attention (M > 1 rows, rotated queries in p.q): scores and softmax terms of every (row, query head, key) by
+// k_attn_block: k_attn_part for a prefill of some tens to 256 rows (rotated queries in p.q): one workgroup per (kv head's
+// query-head group, key chunk, block of HD / Q3_CHUNK rows). The chunk's keys go to LDS and its values to registers
+// once and serve every row of the block, every thread scoring one (row, head, key), instead of one workgroup
+// reloading the chunk for each row. (Blocks of 16 rows measured slower, both as four such passes per workgroup and
+// with register-blocked scores -- each wave scoring four rows per K row read from LDS: the scoring is per-thread
+// latency, and 4x fewer workgroups left most CUs idle.) Each row's partials are computed with
+// k_attn_part's operations in its order (the score sums, the 32-lane max and sum, the P.V accumulation), and a row
+// with no key in the chunk gets k_attn_part's empty partial, so the partials are bit-identical to it.
+template <int GW>
+__global__ __launch_bounds__(256) void k_attn_block(q3_att p) {
+    extern __shared__ float sm[];
+    const int HD = p.HD, G = p.NH / p.NKV, KVD = p.NKV * HD, QD = p.NH * HD;
+    const int nsub = G / GW, sub = blockIdx.x % nsub;
+    const int kvh = blockIdx.x / nsub, h0 = kvh * G + sub * GW; // first query head
+    const int s = blockIdx.y, tid = threadIdx.x;
+    const int g = tid / HD, d = tid - g * HD;
+    const int RR = HD / Q3_CHUNK; // rows per workgroup: GW * Q3_CHUNK * RR threads score them together
+    const int t0 = blockIdx.z * RR, t1 = min(t0 + RR, p.M); // rows t0 .. t1 - 1
+    const int j0 = s * Q3_CHUNK;
+    const int nmax = min(Q3_CHUNK, min(p.st[0] + t1, p.max_ctx) - j0); // keys of the block's last row
+    if (nmax <= 0) { // no row of the block reaches this chunk
+        for (int t = t0; t < t1; t++) {
+            float *out = p.part + (((size_t)t * p.NH + h0 + g) * p.S + s) * (HD + 2);
+            out[d] = 0.f;
+            if (d == 0) {
+                out[HD] = -INFINITY;
+                out[HD + 1] = 0.f;
+            }
+        }
+        return;
+    }
+    const int KS = HD + 4; // LDS row stride: 16-byte rows, 8 consecutive lanes of a float4 read hit distinct banks
+    float *Ks = sm;
+    float *qs = Ks + Q3_CHUNK * KS; // [RR][GW][HD]
+    float *P = qs + RR * GW * HD;   // [RR][GW][Q3_CHUNK]
+    float *ml = P + RR * GW * Q3_CHUNK; // [RR][GW][2]
+    const float *__restrict__ kb = p.kc + (size_t)j0 * KVD + kvh * HD;
+    const float *__restrict__ vb = p.vc + (size_t)j0 * KVD + kvh * HD + d;
+    float vv[Q3_CHUNK];
+#pragma unroll
+    for (int j = 0; j < Q3_CHUNK; j++) vv[j] = vb[(size_t)min(j, nmax - 1) * KVD];
+    const int HD4 = HD >> 2;
+    constexpr int KR = Q3_CHUNK / 4 / GW;
+    float4 kreg[KR];
+#pragma unroll
+    for (int k = 0; k < KR; k++) {
+        const int f = tid + k * blockDim.x, j = f / HD4, c4 = f - j * HD4;
+        kreg[k] = *(const float4 *)(kb + (size_t)min(j, nmax - 1) * KVD + 4 * c4);
+    }
+#pragma unroll
+    for (int k = 0; k < KR; k++) {
+        const int f = tid + k * blockDim.x, j = f / HD4, c4 = f - j * HD4;
+        *(float4 *)(Ks + j * KS + 4 * c4) = kreg[k];
+    }
+    for (int r0 = t0; r0 < t1; r0 += RR) {
+        for (int rr = 0; rr < RR; rr++) {
+            const int t = min(r0 + rr, t1 - 1);
+            qs[rr * GW * HD + tid] = p.q[(size_t)t * QD + h0 * HD + tid];
+        }
+        __syncthreads(); // keys (first pass) and this pass's queries
+        {   // scores: thread = (row rr, head gg, key j)
+            const int rr = tid / (GW * Q3_CHUNK), gg = (tid / Q3_CHUNK) % GW, j = tid % Q3_CHUNK;
+            const int t = r0 + rr;
+            const int n = min(Q3_CHUNK, min(p.st[0] + t + 1, p.max_ctx) - j0);
+            const float4 *qr = (const float4 *)(qs + (rr * GW + gg) * HD), *kr = (const float4 *)(Ks + j * KS);
+            float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
+#pragma unroll 8
+            for (int e = 0; e < HD4; e++) {
+                const float4 qv = qr[e], kv = kr[e];
+                a0 += qv.x * kv.x;
+                a1 += qv.y * kv.y;
+                a2 += qv.z * kv.z;
+                a3 += qv.w * kv.w;
+            }
+            const float sc = j < n ? ((a0 + a1) + (a2 + a3)) * p.scale : -INFINITY;
+            const float m = group_max<Q3_CHUNK>(sc);
+            const float pj = j < n ? expf(sc - m) : 0.f;
+            const float l = group_sum<Q3_CHUNK>(pj);
+            P[(rr * GW + gg) * Q3_CHUNK + j] = pj;
+            if (j == 0) {
+                ml[2 * (rr * GW + gg)] = m;
+                ml[2 * (rr * GW + gg) + 1] = l;
+            }
+        }
+        __syncthreads();
+        for (int rr = 0; rr < RR && r0 + rr < t1; rr++) {
+            const int t = r0 + rr;
+            float *out = p.part + (((size_t)t * p.NH + h0 + g) * p.S + s) * (HD + 2);
+            const int n = min(Q3_CHUNK, min(p.st[0] + t + 1, p.max_ctx) - j0);
+            if (n <= 0) { // k_attn_part's empty partial
+                out[d] = 0.f;
+                if (d == 0) {
+                    out[HD] = -INFINITY;
+                    out[HD + 1] = 0.f;
+                }
+                continue;
+            }
+            float acc = 0.f;
+#pragma unroll
+            for (int j = 0; j < Q3_CHUNK; j++) acc += P[(rr * GW + g) * Q3_CHUNK + j] * vv[j];
+            out[d] = acc;
+            if (d == 0) {
+                out[HD] = ml[2 * (rr * GW + g)];
+                out[HD + 1] = ml[2 * (rr * GW + g) + 1];
+            }
+        }
+        __syncthreads(); // this pass's P and queries read before the next pass writes them
+    }
+}
+
+// Prefill attention (more than 256 rows, rotated queries in p.q): scores and softmax terms of every (row, query head, key) by
 // k_attn_scores, then P.V and the chunk combine in registers by k_attn_pv, with k_attn_part's and attn_quant_body's
 // operations in their order (the four score sums, the 32-key chunk's max and sum, the chunk's P.V accumulation over
 // ascending keys, the log-sum-exp combine over ascending chunks), so the rows are bit-identical to the row-by-row
@@ -304,8 +415,8 @@ __global__ __launch_bounds__(256) void k_attn_part(q3_att p) {
 // sits in one register and is broadcast by the multiply itself, the other comes from registers or one LDS read per 16
 // products, and only the probabilities cross HBM (4 bytes per score), where one workgroup per (32-key chunk, 4 rows)
 // wrote every chunk's P.V row (HD + 2 floats) and a combine launch read it back. Per layer at Qwen3-1.7B widths,
-// traced, that form -> this one (with the row quantisation): M=1000 295 -> 184 us, M=500 81 -> 68; whole prefills of
-// two layers M=64 168 -> 161, M=128 188 -> 180, M=256 236 -> 228, M=500 377 -> 353, M=700 574 -> 461, M=1000 855 -> 634.
+// traced, k_attn_block -> this (with the row quantisation): M=1000 295 -> 184 us, M=500 81 -> 68; whole prefills of
+// two layers M=500 377 -> 353, M=700 574 -> 461, M=1000 855 -> 634.
 // At M=1000 the mul / add pairs alone take 104 us at the VALU's rate.
 // Lane N of each 16-lane row, in every lane of the row: folded into the multiply that uses it (a DPP operand).
 template <int N> __device__ __forceinline__ float bc16(float x) {
@@ -685,6 +796,17 @@ int q3k_attn_part(const q3_att *p, void *stream) {
     const dim3 grid(p->NKV * (G / GW), p->S, p->M), block(GW * p->HD);
     const hipStream_t st = (hipStream_t)stream;
     const bool fused = p->cq != nullptr;
+    if (!fused && p->rows) { // the chunk once per block of rows
+        const int rr = p->HD / Q3_CHUNK;
+        const size_t lr = (size_t)(Q3_CHUNK * (p->HD + 4) + rr * GW * (p->HD + Q3_CHUNK + 2)) * 4;
+        const dim3 gr(p->NKV * (G / GW), p->S, (p->M + rr - 1) / rr);
+        if (lr > 64 * 1024) return -2;
+        if (GW == 1) hipLaunchKernelGGL((k_attn_block<1>), gr, block, lr, st, *p);
+        else if (GW == 2) hipLaunchKernelGGL((k_attn_block<2>), gr, block, lr, st, *p);
+        else if (GW == 4) hipLaunchKernelGGL((k_attn_block<4>), gr, block, lr, st, *p);
+        else return -2;
+        return launch_ok();
+    }
     if (GW == 1) {
         if (fused) hipLaunchKernelGGL((k_attn_part<1, true>), grid, block, lds, st, *p);
         else hipLaunchKernelGGL((k_attn_part<1, false>), grid, block, lds, st, *p);
@@ -706,12 +828,11 @@ int q3k_attn_rows(const q3_att *p, void *stream) {
         p->S > Q3_MAX_S || (long)p->S * Q3_CHUNK < p->M || !p->q || !p->sc || !p->ml || !p->o)
         return -2;
     const hipStream_t st = (hipStream_t)stream;
-    /* A scores workgroup takes the rows whose pairs are one quad a wave, and a P.V wave two pairs up to 256 rows, else
-     * four: with few rows the waves' chains are the time, with many their reads of V. Whole prefills of two layers at
-     * Qwen3-1.7B widths (16 heads, 8 kv heads; us): M=128 4 / 8 / 16 / 32 rows 200 / 197 / 202 / 219, M=1000 730 / 658
-     * / 658 / 666; two / four pairs M=128 196.7 / 198.9, M=256 245.0 / 249.3, M=384 298.2 / 297.6, M=1000 719 / 658. */
-    const int pw = p->M <= 256 ? 2 : 4;
-    const long groups = ((long)p->M * G + pw - 1) / pw;
+    /* A scores workgroup takes the rows whose pairs are one quad a wave, and a P.V wave four pairs, which read V once.
+     * Whole prefills of two layers at Qwen3-1.7B widths (16 heads, 8 kv heads; us), M=1000: 4 / 8 / 16 / 32 rows 730 /
+     * 658 / 658 / 666; two / four pairs 719 / 658. */
+    constexpr int PW = 4;
+    const long groups = ((long)p->M * G + PW - 1) / PW;
     q3_att a = *p;
     a.sr = G >= 16 ? 1 : 16 / G;
     const dim3 grid(p->NKV, (p->M + 63) / 64, (p->M + a.sr - 1) / a.sr);
@@ -722,8 +843,7 @@ int q3k_attn_rows(const q3_att *p, void *stream) {
     else if (p->HD == 192) hipLaunchKernelGGL(k_attn_scores<192>, grid, dim3(256), lds, st, a);
     else hipLaunchKernelGGL(k_attn_scores<256>, grid, dim3(256), lds, st, a);
     if (launch_ok()) return -1;
-    if (pw == 2) hipLaunchKernelGGL(k_attn_pv<2>, dim3(p->NKV, (unsigned)groups), dim3(p->HD), 0, st, *p);
-    else hipLaunchKernelGGL(k_attn_pv<4>, dim3(p->NKV, (unsigned)groups), dim3(p->HD), 0, st, *p);
+    hipLaunchKernelGGL(k_attn_pv<PW>, dim3(p->NKV, (unsigned)groups), dim3(p->HD), 0, st, *p);
     return launch_ok();
 }
 

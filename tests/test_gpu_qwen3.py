@@ -152,11 +152,11 @@ def test_fused_decode_equals_unfused(npu, case):
 
 
 @pytest.mark.parametrize("case", [
-    dict(name="gqa2-hd128", over={}, n=(2, 31, 33, 64, 65, 127, 300)),
-    dict(name="gqa4-hd64", over=dict(heads=8, kv_heads=2, head_dim=64), n=(3, 32, 97, 257)),
-    dict(name="mha-hd128", over=dict(heads=2, kv_heads=2), n=(17, 66)),
-    dict(name="gqa3-hd192", over=dict(heads=3, kv_heads=1, head_dim=192), n=(5, 70)),
-    dict(name="gqa2-hd256", over=dict(heads=2, kv_heads=1, head_dim=256), n=(63, 130)),
+    dict(name="gqa2-hd128", over={}, n=(2, 31, 33, 64, 65, 127, 256, 257, 300, 320)),
+    dict(name="gqa4-hd64", over=dict(heads=8, kv_heads=2, head_dim=64), n=(3, 32, 97, 257, 289)),
+    dict(name="mha-hd128", over=dict(heads=2, kv_heads=2), n=(17, 66, 258)),
+    dict(name="gqa3-hd192", over=dict(heads=3, kv_heads=1, head_dim=192), n=(5, 70, 260)),
+    dict(name="gqa2-hd256", over=dict(heads=2, kv_heads=1, head_dim=256), n=(63, 130, 257)),
 ])
 def test_prefill_attention_by_blocks_equals_rows(npu, case):
     """Prefill attention by blocks of rows against row by row, at the edges of the key tiles (64), the chunks (32), the
