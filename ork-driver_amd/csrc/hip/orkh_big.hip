@@ -36,6 +36,10 @@ template <int KIND, int BM, int BN> struct BG {
     static constexpr int MTW = BM / 16 / WM, NTW = BN / 16 / WN; // 16 x 16 blocks per wave
     static constexpr int MHN = MTW >= 4 ? 2 : 1, MH = MTW / MHN; // a phase: one K step x MH row blocks
     static constexpr int BPP = NIB ? 1 : 2;                      // panel blocks per panel and stage
+    // fp32 sums per output: two on fp16's 128-row tiles, over the even and the odd 32-k blocks, as the smaller tiles they
+    // replace have (relative error against fp64, one sum, two: K=2048 N=6144 M=1000 2.87e-7, 2.06e-7; K=8192 N=2048 M=2500
+    // 5.74e-7, 4.07e-7; time +0.5%). The 256-row tiles have no registers for a second one (MTW * NTW * 8 of 128 a lane)
+    static constexpr int CH = KIND == ORKH_F16 && BM == 128 ? 2 : 1;
     // 1 KiB loads per stage: 8 rows of A, or one block of B. QA and QB per wave (so that a load's kind is known at compile
     // time); a B load without work (QB * NW > NBL) lands in a junk block
     static constexpr int NA = BM / 8, NBL = BN / 16 * BPP;
@@ -148,11 +152,13 @@ __device__ __forceinline__ void big_body(const orkh_mm &p, int mtiles, int ntile
     using J1 = std::integral_constant<int, 1>;
     using J2 = std::integral_constant<int, 2>;
 
-    acc_t acc[P::MTW][P::NTW];
+    acc_t acc[P::CH][P::MTW][P::NTW];
 #pragma unroll
-    for (int a = 0; a < P::MTW; a++)
+    for (int c = 0; c < P::CH; c++)
 #pragma unroll
-        for (int b = 0; b < P::NTW; b++) acc[a][b] = acc_t{0, 0, 0, 0};
+        for (int a = 0; a < P::MTW; a++)
+#pragma unroll
+            for (int b = 0; b < P::NTW; b++) acc[c][a][b] = acc_t{0, 0, 0, 0};
     // A operand of (row block mb, step kk): chunk c of row lane % 16, at (mb * 2 + h) * 64 + r7 * 8 + (c ^ r7 ^ h)
     const int h = (lane >> 3) & 1, r7 = lane & 7;
     const int c0 = P::NIB ? (lane >> 4) * 2 : lane >> 4, c1 = P::NIB ? c0 + 1 : c0 + 4;
@@ -177,11 +183,13 @@ __device__ __forceinline__ void big_body(const orkh_mm &p, int mtiles, int ntile
             for (int i = 0; i < P::NTW; i++) b[kk][i] = step_op<KIND>(raw[i], kk, L);
         }
     };
-    auto mm = [&](int hh, const v4i (&xa)[P::MH], const v4i (&xb)[P::NTW]) {
+    auto mm = [&](int kk, int hh) { // K step kk (its operands are in a[] and b[]) of row blocks hh * MH ..
+        const int c = kk % P::CH;
 #pragma unroll
         for (int i = 0; i < P::MH; i++)
 #pragma unroll
-            for (int jn = 0; jn < P::NTW; jn++) acc[hh * P::MH + i][jn] = mma(xb[jn], xa[i], acc[hh * P::MH + i][jn]);
+            for (int jn = 0; jn < P::NTW; jn++)
+                acc[c][hh * P::MH + i][jn] = mma(b[kk][jn], a[P::MHN == 2 ? hh : kk][i], acc[c][hh * P::MH + i][jn]);
     };
     // keeps each phase's LDS reads in front of its MFMAs
     auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
@@ -201,19 +209,19 @@ __device__ __forceinline__ void big_body(const orkh_mm &p, int mtiles, int ntile
         if constexpr (P::MHN == 2) {
             rdA(rs, 0, 1, a[1]);
             fence();
-            mm(0, a[0], b[0]);
+            mm(0, 0);
             part(J0{});
             fence();
             if constexpr (!P::NIB) rdB(rs, 1);
             rdA(rs, 1, 0, a[0]);
             opB(1);
             fence();
-            mm(1, a[1], b[0]);
+            mm(0, 1);
             part(J1{});
             fence();
             rdA(rs, 1, 1, a[1]);
             fence();
-            mm(0, a[0], b[1]);
+            mm(1, 0);
             part(J2{});
             fence();
         } else {
@@ -221,7 +229,7 @@ __device__ __forceinline__ void big_body(const orkh_mm &p, int mtiles, int ntile
             rdA(rs, 1, 0, a[1]);
             opB(1);
             fence();
-            mm(0, a[0], b[0]);
+            mm(0, 0);
             part(J0{});
             fence();
         }
@@ -237,7 +245,7 @@ __device__ __forceinline__ void big_body(const orkh_mm &p, int mtiles, int ntile
             rdA(rn, 0, 0, a[0]);
         }
         fence();
-        mm(P::MHN - 1, a[1], b[1]);
+        mm(1, P::MHN - 1);
         fence();
         opB(0); // (after the last stage: of what it holds, unused)
         rs = rn;
@@ -254,7 +262,8 @@ __device__ __forceinline__ void big_body(const orkh_mm &p, int mtiles, int ntile
 #pragma unroll
         for (int jn = 0; jn < P::NTW; jn++) {
             if (nb0 + wn * P::NTW + jn >= NBt) continue;
-            acc_t o = acc[i][jn];
+            acc_t o = acc[0][i][jn];
+            if constexpr (P::CH == 2) o += acc[1][i][jn];
 #pragma unroll
             for (int r = 0; r < 4; r++) o[r] = finish<KIND>(o[r]);
             c_t *dst = Cr + jn * 16;

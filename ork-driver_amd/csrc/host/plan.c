@@ -351,6 +351,15 @@ static double tiled2_best(int rkind, int M, int N, int KB, int cu, int ks_force,
 
 static int plan_core(const ork_npu *c, int rkind, int M, int K, int N, int KB, orkh_plan *q, size_t *ws_bytes);
 
+/* Groups of waves that split a stage's K-blocks on a tile of the LDS-ring kernel, each with its own sums: k_tiled2's wave
+ * grid (t2_xg, t2_wn: 2 x 4 on the uniform-int4 64 x 192 tile, 2 x 2 on its 64 x 64 tile) */
+static int tiled2_kgroups(int rkind, int bm, int bn) {
+    const int xg = (rkind == ORKH_I4U && bm == 64) ? (bn == 192 ? 1 : bn == 64 ? 2 : 0) : 0;
+    const int nbt = bn / 16, mb = xg ? 2 : (bm / 16 < 4 ? bm / 16 : 4);
+    const int nb = xg == 2 ? 2 : (nbt < 4 ? nbt : (nbt % 4 == 0 ? 4 : 2));
+    return 16 / (mb * nb);
+}
+
 /* A-stage layout of the LDS-ring kernel: whole 128-byte row lines (swizzled LDS image; a stage row of 1, 2 or 4
  * lines) or MFMA fragment order. Measured on MI355X, graph-timed, both layouts alternated three times in one run,
  * exact (us, fragment -> line):
@@ -372,10 +381,7 @@ static int plan_core(const ork_npu *c, int rkind, int M, int K, int N, int KB, o
 static int aline_rule(const ork_npu *c, int rkind, const orkh_plan *q, int N) {
     /* the kernel has the line layout only where a stage row is whole 128-byte lines: K-blocks per stage as
      * k_tiled2's t2_ks (1 for int4 kinds, 1 for 256 x 256, else 2; at least the tile's K groups of waves) */
-    /* k_tiled2's wave grid (t2_xg, t2_wn): 2 x 4 on the uniform-int4 64 x 192 tile, 2 x 2 on its 64 x 64 tile */
-    const int xg = (rkind == ORKH_I4U && q->bm == 64) ? (q->bn == 192 ? 1 : q->bn == 64 ? 2 : 0) : 0;
-    const int nbt = q->bn / 16, mb = xg ? 2 : (q->bm / 16 < 4 ? q->bm / 16 : 4);
-    const int nb = xg == 2 ? 2 : (nbt < 4 ? nbt : (nbt % 4 == 0 ? 4 : 2)), wk = 16 / (mb * nb);
+    const int wk = tiled2_kgroups(rkind, q->bm, q->bn);
     const int base = (rkind == ORKH_I4U || rkind == ORKH_NF4) ? 1 : (q->bm * q->bn >= 65536 ? 1 : 2);
     const int ks = base > wk ? base : wk;
     const int row_bytes = ks * a_bytes_per_kb(rkind);
@@ -558,6 +564,9 @@ static int plan_core(const ork_npu *c, int rkind, int M, int K, int N, int KB, o
  * -> 114.3; uniform int4 K=N=4096 M=4096 89.8 -> 52.3; NF4 112.0 -> 67.3, K=2048 N=6144 M=1000 29.5 -> 24.2. At 512 rows
  * and fewer the smaller tiles fill the CUs better and keep the run (int8 K=2048 N=6144 M=500 11.9 against 16.6), except
  * where N is large (N=12288 20.3 -> 17.6).
+ * fp16: a tile is offered only where it keeps as many fp32 sums an output as the pick it would replace (the pick's K groups
+ * of waves times its K split), each over that share of K: with one sum over all of K in place of two the error against
+ * fp64 was 1.39 to 1.41 times the pick's (K=2048..8192); with two it is the pick's. k_big has two on its 128-row tiles, one on the 256-row ones.
  * A context's planner overrides (ORK_PLAN, ORK_TILE and the others of orki_plan) turn the rule off, and ORK_PLAN=big with
  * ORK_TILE=BMxBN forces a k_big tile. */
 static const struct big_fit {
@@ -573,6 +582,7 @@ static const struct big_fit {
     {ORKH_NF4, 256, 256, 7.815, 0.03910, 0.0886}, {ORKH_NF4, 256, 192, 6.959, 0.03410, 0.0737},
     {ORKH_NF4, 128, 256, 5.171, 0.04358, 0.0746}, {ORKH_NF4, 128, 192, 4.913, 0.03929, 0.0700},
 };
+#define BIG_F16_SUMS(bm) ((bm) == 128 ? 2 : 1) /* BG::CH of the kernel */
 static const struct pick_fit {
     int rkind;
     double margin, a, e1, e2, d, f;
@@ -642,10 +652,11 @@ int orki_plan_mm(const ork_npu *c, int rkind, int M, int K, int N, int KB, orkh_
         double best = p->a + rounds * r->c * (q->bm * abpk + q->bn * 64.0) * kbs / 1024 + (wgs <= cu ? p->e1 : p->e2) * mb +
                       (ks > 1 ? p->d + p->f * ks * mb : 0);
         best = q->bm == 256 && q->bn == 256 ? 1e30 : best * p->margin;
+        const int sums = rkind == ORKH_F16 ? tiled2_kgroups(rkind, q->bm, q->bn) * ks : 1;
         int bm = 0, bn = 0;
         for (size_t j = 0; j < sizeof big_fits / sizeof big_fits[0]; j++) {
             const struct big_fit *g = &big_fits[j];
-            if (g->rkind != rkind) continue;
+            if (g->rkind != rkind || BIG_F16_SUMS(g->bm) < sums) continue;
             const long w = (long)cdiv(M, g->bm) * cdiv(N, g->bn);
             const double t = (double)((w + cu - 1) / cu) * (g->b + g->c * (g->bm * abpk + g->bn * 64.0) * KB / 1024) + g->e * mb;
             if (t < best) {

@@ -1,5 +1,5 @@
 /* Prints the planner's choice for each "kind M K N" argument quadruple on a 256-CU device, one line each, named as
- * the library names its launches (orkh_mm_variant). Built from the host planner source alone, with no GPU code. */
+ * the library names its launches (orkh_mm_variant): orki_plan's, or after a first argument "mm" a run's (orki_plan_mm). Built from the host planner source alone, with no GPU code. */
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -31,6 +31,8 @@ static const char *name(int kind, const orkh_plan *q) {
     else if (q->algo == ORKH_ALGO_STREAM)
         snprintf(b, sizeof b, "stream_%s_mt%d_w%d_kbw%d_ks%d%s", k, q->mt, q->wpg, q->kbw, q->ksplit,
                  q->np == 2 ? "_p2" : q->half ? "_h" : "");
+    else if (q->algo == ORKH_ALGO_BIG)
+        snprintf(b, sizeof b, "big_%s_%dx%d", k, q->bm, q->bn);
     else if (q->ksplit > 1)
         snprintf(b, sizeof b, "%s_%s_%dx%d_ks%d%s%s", q->algo == ORKH_ALGO_TILED2 ? "tiled2" : "tiled", k, q->bm, q->bn,
                  q->ksplit, q->algo == ORKH_ALGO_TILED2 && q->aline ? "_al" : "",
@@ -45,12 +47,13 @@ int main(int argc, char **argv) {
     ork_npu c;
     memset(&c, 0, sizeof c);
     c.cores = 256;
-    for (int i = 1; i + 3 < argc; i += 4) {
+    const int mm = argc > 1 && !strcmp(argv[1], "mm");
+    for (int i = 1 + mm; i + 3 < argc; i += 4) {
         const int kind = atoi(argv[i]), M = atoi(argv[i + 1]), K = atoi(argv[i + 2]), N = atoi(argv[i + 3]);
         const int kpb = kind == ORKH_I8 ? 64 : kind == ORKH_F16 ? 32 : 128;
         orkh_plan q;
         size_t ws = 0;
-        orki_plan(&c, kind, M, K, N, (K + kpb - 1) / kpb, &q, &ws);
+        (mm ? orki_plan_mm : orki_plan)(&c, kind, M, K, N, (K + kpb - 1) / kpb, &q, &ws);
         printf("%d %d %d %d %s %zu\n", kind, M, K, N, name(kind, &q), ws);
     }
     return 0;

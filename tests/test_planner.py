@@ -30,8 +30,8 @@ def planner(tmp_path_factory):
                         "-o", exe, "-lm"], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stderr[-3000:]
 
-    def pick(cases):
-        args = [str(x) for c in cases for x in c]
+    def pick(cases, mm=False):
+        args = ["mm"] * mm + [str(x) for c in cases for x in c]
         out = subprocess.run([exe] + args, capture_output=True, text=True, timeout=60, env={}).stdout.split("\n")
         return [ln.split()[4] for ln in out if ln.strip()]
     return pick
@@ -108,3 +108,31 @@ def test_mma_picks_against_the_sweep(planner, kind):
         tot_best += best
     assert max(worst)[0] <= 1.20, max(worst)
     assert tot_pick <= 1.02 * tot_best, (tot_pick, tot_best, sorted(worst)[-3:])
+
+
+def _f16_sums(name):
+    """fp32 sums an output has under a plan: K groups of waves (k_tiled2's 16 waves over its tile; k_big's 128-row tiles:
+    2) times the K split"""
+    bm, bn = map(int, name.split("_")[2].split("x"))
+    if name.startswith("big_"):
+        return 2 if bm == 128 else 1
+    mb, nb = min(bm // 16, 4), bn // 16
+    nb = nb if nb < 4 else 4 if nb % 4 == 0 else 2
+    return 16 // (mb * nb) * int(name.split("_ks")[1].split("_")[0] if "_ks" in name else 1)
+
+
+def test_f16_sums_not_longer(planner):
+    """fp16 above 64 rows: a run on the many-row kernel keeps at least as many fp32 sums an output (each over that share
+    of K) as the LDS-ring pick it replaces, over 5,000 shapes; both kinds of move (one sum, two sums) occur."""
+    cases = [(3, M, K, N) for K in (256, 1024, 2048, 3072, 4096, 6144, 8192, 16384) for N in (512, 1024, 2048, 4096, 6144, 8192, 12288)
+             for M in list(range(65, 600, 31)) + list(range(600, 4200, 53))]
+    moved = {}
+    for lo in range(0, len(cases), 1000):
+        part = cases[lo:lo + 1000]
+        for c, a, b in zip(part, planner(part), planner(part, mm=True)):
+            if b.startswith("big_"):
+                assert _f16_sums(b) >= _f16_sums(a), (c, a, b)
+                moved[_f16_sums(a)] = moved.get(_f16_sums(a), 0) + 1
+            else:
+                assert a == b, (c, a, b)
+    assert moved.get(1) and moved.get(2), moved
