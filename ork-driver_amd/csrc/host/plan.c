@@ -549,60 +549,101 @@ static int plan_core(const ork_npu *c, int rkind, int M, int K, int N, int KB, o
 
 /* When a run takes the many-row kernel (k_big, ../hip/orkh_big.hip) instead of orki_plan's pick.
  * Above 64 rows both are priced, us, and the cheaper one runs:
- *   k_big, per tile     rounds * (b + c * KiB) + e * MB            (rounds of the CUs; KiB: the A and B bytes a workgroup
+ *   k_big, per tile     a + rounds * (b + c * KiB) + e * MB        (rounds of the CUs; KiB: the A and B bytes a workgroup
  *                                                                  loads; MB: C's megabytes, which the end of a round
  *                                                                  writes with nothing to overlap)
- *   orki_plan's pick    a + rounds * c[tile] * KiB + e * MB + [ks > 1] (d + f * ks * MB)      (e: e1 on one round, else e2)
- * Each is a least-squares fit in relative error (non-negative terms) to launches timed back to back on MI355X: every
- * k_big tile and orki_plan's pick at K x N = 2048 x 6144, 2048 x 2048, 4096 x 4096, 6144 x 2048, 2048 x 12288, 2048 x 4096
- * and 18 row counts from 256 to 4096, per weight kind (108 shapes a kind; a k_big tile's fit takes the shapes where it ran
- * within 1.6x of the fastest); 1-8% rms (k_big) and 4-7% (the picks). What the rule chooses over those shapes, total
- * us: int8 3346 -> 3083 (the faster of the two everywhere would be 3081), fp16 5973 -> 5499 (5492), uniform int4 3625 ->
- * 2891 (2891), NF4 4760 -> 3973 (3951), and no shape is slower than its former pick; NF4's 2% margin keeps two shapes
- * where k_big ran 4-5% slower. 256 x 256 picks always move: k_big was ahead on each. Some shapes, us: int8 K=N=4096
- * M=4096 65.0 -> 61.3, K=6144 N=2048 M=4096 63.3 -> 49.3, K=N=4096 M=2048 41.5 -> 35.2; fp16 K=2048 N=6144 M=4096 140.6
- * -> 114.3; uniform int4 K=N=4096 M=4096 89.8 -> 52.3; NF4 112.0 -> 67.3, K=2048 N=6144 M=1000 29.5 -> 24.2. At 512 rows
- * and fewer the smaller tiles fill the CUs better and keep the run (int8 K=2048 N=6144 M=500 11.9 against 16.6), except
- * where N is large (N=12288 20.3 -> 17.6).
+ *   orki_plan's pick    a + rounds * (b[tile] + c[tile] * KiB) + e * MB + [ks > 1] (d + f * ks * MB)
+ *                                                                  (e: e1 on one round, else e2)
+ * Each is a least-squares fit in relative error (non-negative terms) to launches timed on MI355X, every k_big tile and
+ * orki_plan's pick at 18 (K, N) with K from 256 to 8192 and N from 512 to 12288 and row counts from 65 to 4096, per weight
+ * kind (367 shapes a kind, tests/golden/big_plan_sweep.json); 3-8% rms. Total us over them, former picks, this rule, the
+ * faster of the two everywhere: int8 6438, 5974, 5951; fp16 10641, 9874, 9834; uniform int4 6099, 5271, 5270; NF4 8172, 7096,
+ * 7091. No shape runs 2% slower than its former pick. (Fits without the costs per launch and round, made from K = 2048 up,
+ * took tiles at K = 256 and 512 that ran up to 42% slower: fp16 K=256 N=6144 M=2689 33.4 us on 256 x 256, 23.5 on 128 x
+ * 128.) On 876 more shapes at 20 random (K, N), K from 160 to 7360: 12,126 us by the former picks, 11,015 by this rule,
+ * 10,909 the faster of the two everywhere; the worst 4.7% slower than its pick (int8 K=288 N=1920 M=3442 9.23 -> 9.66).
+ * The margin keeps a pick whose price is that close. Some shapes, us: int8 K=N=4096 M=4096 65.0 -> 61.3, K=6144 N=2048
+ * M=4096 63.3 -> 49.3; fp16 K=2048 N=6144 M=4096 140.6 -> 114.3; uniform int4 K=N=4096 M=4096 89.8 -> 52.3; NF4 112.0 ->
+ * 67.3, K=2048 N=6144 M=1000 29.5 -> 24.2. At 512 rows and fewer the smaller tiles fill the CUs better and keep the run
+ * (int8 K=2048 N=6144 M=500 11.9 against 16.6), except where N is large (N=12288 20.3 -> 17.6).
  * fp16: a tile is offered only where it keeps as many fp32 sums an output as the pick it would replace (the pick's K groups
  * of waves times its K split), each over that share of K: with one sum over all of K in place of two the error against
- * fp64 was 1.39 to 1.41 times the pick's (K=2048..8192); with two it is the pick's. k_big has two on its 128-row tiles, one on the 256-row ones.
+ * fp64 was 1.39 to 1.41 times the pick's (K=2048..8192); with two it is the pick's. k_big has two on its
+ * 128-row tiles, one on the 256-row ones.
  * A context's planner overrides (ORK_PLAN, ORK_TILE and the others of orki_plan) turn the rule off, and ORK_PLAN=big with
  * ORK_TILE=BMxBN forces a k_big tile. */
 static const struct big_fit {
     int rkind, bm, bn;
-    double b, c, e;
+    double a, b, c, e;
 } big_fits[] = {
-    {ORKH_I8, 256, 256, 3.832, 0.01899, 0.1932}, {ORKH_I8, 256, 192, 3.190, 0.01845, 0.2148},
-    {ORKH_I8, 128, 256, 2.128, 0.01653, 0.2067}, {ORKH_I8, 128, 192, 4.175, 0.01636, 0.1357},
-    {ORKH_F16, 256, 256, 0.000, 0.01968, 0.3515}, {ORKH_F16, 256, 192, 0.000, 0.01891, 0.3824},
-    {ORKH_F16, 128, 256, 0.000, 0.01663, 0.3665}, {ORKH_F16, 128, 192, 1.648, 0.01716, 0.3193},
-    {ORKH_I4U, 256, 256, 6.614, 0.02672, 0.1046}, {ORKH_I4U, 256, 192, 6.102, 0.02459, 0.0925},
-    {ORKH_I4U, 128, 256, 4.943, 0.02404, 0.0811}, {ORKH_I4U, 128, 192, 4.922, 0.02336, 0.0615},
-    {ORKH_NF4, 256, 256, 7.815, 0.03910, 0.0886}, {ORKH_NF4, 256, 192, 6.959, 0.03410, 0.0737},
-    {ORKH_NF4, 128, 256, 5.171, 0.04358, 0.0746}, {ORKH_NF4, 128, 192, 4.913, 0.03929, 0.0700},
+    {ORKH_I8, 256, 256, 0.0000, 5.7765, 0.0205, 0.1218},  {ORKH_I8, 256, 192, 0.0000, 5.1089, 0.0211, 0.1093},
+    {ORKH_I8, 128, 256, 0.0000, 4.8479, 0.0162, 0.0922},  {ORKH_I8, 128, 192, 0.2062, 4.4958, 0.0169, 0.0682},
+    {ORKH_F16, 256, 256, 0.0000, 5.6807, 0.0211, 0.1345}, {ORKH_F16, 256, 192, 0.0000, 4.7918, 0.0216, 0.1308},
+    {ORKH_F16, 128, 256, 0.0000, 4.5878, 0.0164, 0.1335}, {ORKH_F16, 128, 192, 0.0000, 4.2631, 0.0172, 0.1092},
+    {ORKH_I4U, 256, 256, 0.0000, 9.0208, 0.0249, 0.0493}, {ORKH_I4U, 256, 192, 0.8432, 4.6144, 0.0227, 0.1034},
+    {ORKH_I4U, 128, 256, 0.0000, 5.4960, 0.0243, 0.0511}, {ORKH_I4U, 128, 192, 0.6367, 4.1975, 0.0214, 0.0625},
+    {ORKH_NF4, 256, 256, 0.0000, 9.7801, 0.0335, 0.0432}, {ORKH_NF4, 256, 192, 0.7795, 5.3498, 0.0317, 0.0895},
+    {ORKH_NF4, 128, 256, 0.2060, 5.6790, 0.0433, 0.0402}, {ORKH_NF4, 128, 192, 0.5242, 4.5105, 0.0393, 0.0465},
 };
 #define BIG_F16_SUMS(bm) ((bm) == 128 ? 2 : 1) /* BG::CH of the kernel */
 static const struct pick_fit {
     int rkind;
     double margin, a, e1, e2, d, f;
 } pick_fits[] = {
-    {ORKH_I8, 1.00, 2.1398, 0.1758, 0.2503, 3.7309, 0.2135},
-    {ORKH_F16, 1.00, 0.0000, 0.3488, 0.4121, 0.7596, 0.5661},
-    {ORKH_I4U, 1.00, 1.6989, 0.2755, 0.2359, 0.0000, 0.6995},
-    {ORKH_NF4, 0.98, 2.2934, 0.1759, 0.2515, 8.4391, 0.0000},
+    {ORKH_I8, 0.99, 2.0978, 0.1376, 0.1707, 2.7595, 0.4158},
+    {ORKH_F16, 0.97, 1.9090, 0.1646, 0.1662, 2.6121, 0.4608},
+    {ORKH_I4U, 0.99, 2.9182, 0.0677, 0.1019, 2.8818, 0.4031},
+    {ORKH_NF4, 0.99, 2.1372, 0.0642, 0.1122, 2.5850, 0.3767},
 };
-static const struct pick_rate { /* c of a tile; bm 0: a tile that no timed shape picked */
-    int rkind, bm, bn, ring;
-    double c;
+static const struct pick_rate { /* b and c of a tile; bm 0: a tile that no timed shape picked, at the kind's lowest rate */
+    int rkind, algo, bm, bn, ring;
+    double b, c;
 } pick_rates[] = {
-    {ORKH_I8, 32, 64, 0, 0.0236}, {ORKH_I8, 64, 64, 0, 0.0167}, {ORKH_I8, 64, 192, 2, 0.0118}, {ORKH_I8, 128, 96, 0, 0.0157},
-    {ORKH_I8, 128, 96, 2, 0.0128}, {ORKH_I8, 128, 128, 0, 0.0155}, {ORKH_I8, 128, 128, 2, 0.0147}, {ORKH_I8, 0, 0, 0, 0.0150},
-    {ORKH_F16, 32, 64, 0, 0.0249}, {ORKH_F16, 64, 64, 0, 0.0203}, {ORKH_F16, 128, 96, 0, 0.0162}, {ORKH_F16, 128, 96, 2, 0.0126},
-    {ORKH_F16, 128, 128, 0, 0.0156}, {ORKH_F16, 128, 128, 2, 0.0147}, {ORKH_F16, 0, 0, 0, 0.0150},
-    {ORKH_I4U, 32, 64, 0, 0.0222}, {ORKH_I4U, 64, 64, 0, 0.0156}, {ORKH_I4U, 0, 0, 0, 0.0194},
-    {ORKH_NF4, 32, 64, 0, 0.0320}, {ORKH_NF4, 64, 64, 0, 0.0315}, {ORKH_NF4, 128, 96, 0, 0.0304}, {ORKH_NF4, 0, 0, 0, 0.0281},
+    {ORKH_I8, ORKH_ALGO_TILED2, 16, 64, 0, 0.0000, 0.0299},    {ORKH_I8, ORKH_ALGO_TILED2, 32, 32, 0, 0.5247, 0.0153},
+    {ORKH_I8, ORKH_ALGO_TILED2, 32, 64, 0, 0.7462, 0.0205},    {ORKH_I8, ORKH_ALGO_TILED2, 64, 64, 0, 0.3034, 0.0162},
+    {ORKH_I8, ORKH_ALGO_TILED2, 64, 192, 0, 0.0311, 0.0160},   {ORKH_I8, ORKH_ALGO_TILED2, 64, 192, 2, 0.1355, 0.0157},
+    {ORKH_I8, ORKH_ALGO_TILED2, 128, 96, 0, 1.5378, 0.0152},   {ORKH_I8, ORKH_ALGO_TILED2, 128, 96, 2, 1.5462, 0.0151},
+    {ORKH_I8, ORKH_ALGO_TILED2, 128, 128, 0, 0.3674, 0.0169},  {ORKH_I8, ORKH_ALGO_TILED2, 128, 128, 2, 0.0000, 0.0179},
+    {ORKH_I8, ORKH_ALGO_TILED2, 256, 256, 0, 1.3346, 0.0230},  {ORKH_I8, 0, 0, 0, 0, 0.0000, 0.0151},
+    {ORKH_F16, ORKH_ALGO_TILED2, 16, 64, 0, 0.0000, 0.0234},   {ORKH_F16, ORKH_ALGO_TILED2, 32, 32, 0, 0.8556, 0.0137},
+    {ORKH_F16, ORKH_ALGO_TILED2, 32, 64, 0, 0.8593, 0.0194},   {ORKH_F16, ORKH_ALGO_TILED2, 64, 64, 0, 0.4737, 0.0170},
+    {ORKH_F16, ORKH_ALGO_TILED2, 64, 192, 0, 0.4262, 0.0162},  {ORKH_F16, ORKH_ALGO_TILED2, 64, 192, 2, 0.0000, 0.0178},
+    {ORKH_F16, ORKH_ALGO_TILED2, 128, 96, 0, 1.1402, 0.0166},  {ORKH_F16, ORKH_ALGO_TILED2, 128, 96, 2, 0.6158, 0.0161},
+    {ORKH_F16, ORKH_ALGO_TILED2, 128, 128, 0, 0.0000, 0.0175}, {ORKH_F16, ORKH_ALGO_TILED2, 128, 128, 2, 0.0000, 0.0191},
+    {ORKH_F16, ORKH_ALGO_TILED2, 256, 256, 0, 1.7028, 0.0232}, {ORKH_F16, 0, 0, 0, 0, 0.0000, 0.0137},
+    {ORKH_I4U, ORKH_ALGO_TILED2, 16, 64, 0, 0.0000, 0.0225},   {ORKH_I4U, ORKH_ALGO_TILED2, 32, 32, 0, 0.0788, 0.0120},
+    {ORKH_I4U, ORKH_ALGO_TILED2, 32, 64, 0, 0.0253, 0.0183},   {ORKH_I4U, ORKH_ALGO_TILED2, 64, 64, 0, 0.6958, 0.0116},
+    {ORKH_I4U, ORKH_ALGO_TILED2, 64, 192, 0, 1.2931, 0.0178},  {ORKH_I4U, ORKH_ALGO_TILED2, 128, 96, 0, 0.0000, 0.0228},
+    {ORKH_I4U, ORKH_ALGO_TILED2, 128, 128, 0, 0.3711, 0.0220}, {ORKH_I4U, ORKH_ALGO_TILED2, 128, 128, 2, 0.5890, 0.0207},
+    {ORKH_I4U, 0, 0, 0, 0, 0.0000, 0.0116},
+    {ORKH_NF4, ORKH_ALGO_TILED, 64, 64, 0, 4.3708, 0.0232},    {ORKH_NF4, ORKH_ALGO_TILED2, 32, 64, 0, 0.7359, 0.0297},
+    {ORKH_NF4, ORKH_ALGO_TILED2, 64, 64, 0, 0.5259, 0.0326},   {ORKH_NF4, ORKH_ALGO_TILED2, 128, 96, 0, 2.4996, 0.0273},
+    {ORKH_NF4, ORKH_ALGO_TILED2, 128, 128, 0, 1.7391, 0.0284}, {ORKH_NF4, 0, 0, 0, 0, 0.0000, 0.0232},
 };
+
+/* A and B KiB that one workgroup of a bm x bn tile loads over kbs K-blocks */
+static double tile_kib(int rkind, int bm, int bn, int kbs) {
+    return ((double)bm * a_bytes_per_kb(rkind) + bn * 64.0) * kbs / 1024;
+}
+
+/* Price of orki_plan's pick q over its wgs workgroups, times the kind's margin; mb: C's megabytes */
+static double pick_us(int rkind, const orkh_plan *q, long wgs, int KB, double mb, int cu) {
+    const struct pick_fit *p = pick_fits;
+    while (p->rkind != rkind) p++;
+    const struct pick_rate *r = pick_rates;
+    while (r->rkind != rkind ||
+           (r->bm && (r->algo != q->algo || r->bm != q->bm || r->bn != q->bn || r->ring != q->ring)))
+        r++;
+    const int ks = q->ksplit > 1 ? q->ksplit : 1;
+    const double rounds = (double)((wgs + cu - 1) / cu);
+    double t = p->a + rounds * (r->b + r->c * tile_kib(rkind, q->bm, q->bn, ks > 1 ? q->kbs : KB)) + (wgs <= cu ? p->e1 : p->e2) * mb;
+    if (ks > 1) t += p->d + p->f * ks * mb;
+    return t * p->margin;
+}
+
+static double big_us(const struct big_fit *g, long wgs, int KB, double mb, int cu) {
+    return g->a + (double)((wgs + cu - 1) / cu) * (g->b + g->c * tile_kib(g->rkind, g->bm, g->bn, KB)) + g->e * mb;
+}
 
 /* any planner override of orki_plan in the environment of a context that honours them */
 static int overridden(const ork_npu *c) {
@@ -636,38 +677,22 @@ int orki_plan_mm(const ork_npu *c, int rkind, int M, int K, int N, int KB, orkh_
     }
     if (q->algo != ORKH_ALGO_TILED2 && q->algo != ORKH_ALGO_TILED) return 0;
     const int cu = (c && c->cores > 0) ? c->cores : 256;
-    const double abpk = rkind == ORKH_I4U || rkind == ORKH_NF4 ? 128 : 64; /* A bytes per row and K-block */
+    const int ks = q->ksplit > 1 ? q->ksplit : 1;
     const double mb = (double)M * N * 4 / 1e6;
-    for (size_t i = 0; i < sizeof pick_fits / sizeof pick_fits[0]; i++) {
-        const struct pick_fit *p = &pick_fits[i];
-        if (p->rkind != rkind) continue;
-        const int ks = q->ksplit > 1 ? q->ksplit : 1, kbs = ks > 1 ? q->kbs : KB;
-        const long wgs = (long)cdiv(M, q->bm) * cdiv(N / 16, q->bn / 16) * ks;
-        const struct pick_rate *r = NULL;
-        for (size_t j = 0; j < sizeof pick_rates / sizeof pick_rates[0] && !r; j++) {
-            const struct pick_rate *x = &pick_rates[j];
-            if (x->rkind == rkind && (!x->bm || (x->bm == q->bm && x->bn == q->bn && x->ring == q->ring))) r = x;
+    double best = pick_us(rkind, q, (long)cdiv(M, q->bm) * cdiv(N / 16, q->bn / 16) * ks, KB, mb, cu);
+    const int sums = rkind == ORKH_F16 ? tiled2_kgroups(rkind, q->bm, q->bn) * ks : 1;
+    int bm = 0, bn = 0;
+    for (size_t j = 0; j < sizeof big_fits / sizeof big_fits[0]; j++) {
+        const struct big_fit *g = &big_fits[j];
+        if (g->rkind != rkind || (rkind == ORKH_F16 && BIG_F16_SUMS(g->bm) < sums)) continue;
+        const double t = big_us(g, (long)cdiv(M, g->bm) * cdiv(N, g->bn), KB, mb, cu);
+        if (t < best) {
+            best = t;
+            bm = g->bm;
+            bn = g->bn;
         }
-        const double rounds = (double)((wgs + cu - 1) / cu);
-        double best = p->a + rounds * r->c * (q->bm * abpk + q->bn * 64.0) * kbs / 1024 + (wgs <= cu ? p->e1 : p->e2) * mb +
-                      (ks > 1 ? p->d + p->f * ks * mb : 0);
-        best = q->bm == 256 && q->bn == 256 ? 1e30 : best * p->margin;
-        const int sums = rkind == ORKH_F16 ? tiled2_kgroups(rkind, q->bm, q->bn) * ks : 1;
-        int bm = 0, bn = 0;
-        for (size_t j = 0; j < sizeof big_fits / sizeof big_fits[0]; j++) {
-            const struct big_fit *g = &big_fits[j];
-            if (g->rkind != rkind || BIG_F16_SUMS(g->bm) < sums) continue;
-            const long w = (long)cdiv(M, g->bm) * cdiv(N, g->bn);
-            const double t = (double)((w + cu - 1) / cu) * (g->b + g->c * (g->bm * abpk + g->bn * 64.0) * KB / 1024) + g->e * mb;
-            if (t < best) {
-                best = t;
-                bm = g->bm;
-                bn = g->bn;
-            }
-        }
-        if (bm) take_big(c, bm, bn, M, N, KB, q, ws_bytes);
-        return 0;
     }
+    if (bm) take_big(c, bm, bn, M, N, KB, q, ws_bytes);
     return 0;
 }
 

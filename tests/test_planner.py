@@ -110,6 +110,31 @@ def test_mma_picks_against_the_sweep(planner, kind):
     assert tot_pick <= 1.02 * tot_best, (tot_pick, tot_best, sorted(worst)[-3:])
 
 
+@pytest.mark.parametrize("kind", ["int8", "i4u", "nf4", "fp16"])
+def test_run_picks_against_the_sweep(planner, kind):
+    """What a run above 64 rows takes (orki_plan_mm: orki_plan's pick or a tile of the many-row kernel) against graph-timed
+    launches of both at 367 shapes a kind, K from 256 to 8192 and M from 65 to 4096 (tests/golden/big_plan_sweep.json): no
+    shape over 2% slower than orki_plan's pick, and the total within 1% of the faster of the two everywhere (fp16: of the
+    tiles with the pick's fp32 sums)."""
+    data = json.load(open(os.path.join(ROOT, "tests", "golden", "big_plan_sweep.json")))
+    runs = [r for r in data["runs"] if r[0] == kind]
+    assert len(runs) == 367
+    rk = {"int8": 0, "i4u": 1, "nf4": 2, "fp16": 3}[kind]
+    cases = [(rk, M, K, N) for _, K, N, M, *_ in runs]
+    tot_pick = tot_best = tot_former = 0.0
+    for (_, K, N, M, former, us, *big), old, p in zip(runs, planner(cases), planner(cases, mm=True)):
+        assert old == former, (K, N, M, old, former)
+        times = {"big_" + {"int8": "i8", "fp16": "f16"}.get(kind, kind) + "_" + t: x for t, x in zip(("256x256", "256x192", "128x256", "128x192"), big)}
+        if kind == "fp16":
+            times = {t: x for t, x in times.items() if _f16_sums(t) >= _f16_sums(former)}
+        times[former] = us
+        assert times[p] <= 1.02 * us, (K, N, M, former, us, p, times[p])
+        tot_pick += times[p]
+        tot_best += min(times.values())
+        tot_former += us
+    assert tot_pick <= 1.01 * tot_best and tot_pick < 0.94 * tot_former, (tot_pick, tot_best, tot_former)
+
+
 def _f16_sums(name):
     """fp32 sums an output has under a plan: K groups of waves (k_tiled2's 16 waves over its tile; k_big's 128-row tiles:
     2) times the K split"""
