@@ -557,10 +557,10 @@ static int plan_core(const ork_npu *c, int rkind, int M, int K, int N, int KB, o
  * Each is a least-squares fit in relative error (non-negative terms) to launches timed on MI355X, every k_big tile and
  * orki_plan's pick at 18 (K, N) with K from 256 to 8192 and N from 512 to 12288 and row counts from 65 to 4096, per weight
  * kind (367 shapes a kind, tests/golden/big_plan_sweep.json); 3-8% rms. Total us over them, former picks, this rule, the
- * faster of the two everywhere: int8 6438, 5974, 5951; fp16 10641, 9874, 9834; uniform int4 6099, 5271, 5270; NF4 8172, 7096,
- * 7091. No shape runs 2% slower than its former pick. (Fits without the costs per launch and round, made from K = 2048 up,
+ * faster of the two everywhere: int8 6438, 5957, 5951; fp16 10641, 9859, 9834; uniform int4 6099, 5271, 5270; NF4 8172, 7096,
+ * 7091. No shape runs 2% slower than its former pick (256 x 256: 5%). (Fits without the costs per launch and round, made from K = 2048 up,
  * took tiles at K = 256 and 512 that ran up to 42% slower: fp16 K=256 N=6144 M=2689 33.4 us on 256 x 256, 23.5 on 128 x
- * 128.) On 876 more shapes at 20 random (K, N), K from 160 to 7360: 12,126 us by the former picks, 11,015 by this rule,
+ * 128.) On 876 more shapes at 20 random (K, N), K from 160 to 7360: 12,126 us by the former picks, 11,016 by this rule,
  * 10,909 the faster of the two everywhere; the worst 4.7% slower than its pick (int8 K=288 N=1920 M=3442 9.23 -> 9.66).
  * The margin keeps a pick whose price is that close. Some shapes, us: int8 K=N=4096 M=4096 65.0 -> 61.3, K=6144 N=2048
  * M=4096 63.3 -> 49.3; fp16 K=2048 N=6144 M=4096 140.6 -> 114.3; uniform int4 K=N=4096 M=4096 89.8 -> 52.3; NF4 112.0 ->
@@ -604,13 +604,13 @@ static const struct pick_rate { /* b and c of a tile; bm 0: a tile that no timed
     {ORKH_I8, ORKH_ALGO_TILED2, 64, 192, 0, 0.0311, 0.0160},   {ORKH_I8, ORKH_ALGO_TILED2, 64, 192, 2, 0.1355, 0.0157},
     {ORKH_I8, ORKH_ALGO_TILED2, 128, 96, 0, 1.5378, 0.0152},   {ORKH_I8, ORKH_ALGO_TILED2, 128, 96, 2, 1.5462, 0.0151},
     {ORKH_I8, ORKH_ALGO_TILED2, 128, 128, 0, 0.3674, 0.0169},  {ORKH_I8, ORKH_ALGO_TILED2, 128, 128, 2, 0.0000, 0.0179},
-    {ORKH_I8, ORKH_ALGO_TILED2, 256, 256, 0, 1.3346, 0.0230},  {ORKH_I8, 0, 0, 0, 0, 0.0000, 0.0151},
+    {ORKH_I8, 0, 0, 0, 0, 0.0000, 0.0151},
     {ORKH_F16, ORKH_ALGO_TILED2, 16, 64, 0, 0.0000, 0.0234},   {ORKH_F16, ORKH_ALGO_TILED2, 32, 32, 0, 0.8556, 0.0137},
     {ORKH_F16, ORKH_ALGO_TILED2, 32, 64, 0, 0.8593, 0.0194},   {ORKH_F16, ORKH_ALGO_TILED2, 64, 64, 0, 0.4737, 0.0170},
     {ORKH_F16, ORKH_ALGO_TILED2, 64, 192, 0, 0.4262, 0.0162},  {ORKH_F16, ORKH_ALGO_TILED2, 64, 192, 2, 0.0000, 0.0178},
     {ORKH_F16, ORKH_ALGO_TILED2, 128, 96, 0, 1.1402, 0.0166},  {ORKH_F16, ORKH_ALGO_TILED2, 128, 96, 2, 0.6158, 0.0161},
     {ORKH_F16, ORKH_ALGO_TILED2, 128, 128, 0, 0.0000, 0.0175}, {ORKH_F16, ORKH_ALGO_TILED2, 128, 128, 2, 0.0000, 0.0191},
-    {ORKH_F16, ORKH_ALGO_TILED2, 256, 256, 0, 1.7028, 0.0232}, {ORKH_F16, 0, 0, 0, 0, 0.0000, 0.0137},
+    {ORKH_F16, 0, 0, 0, 0, 0.0000, 0.0137},
     {ORKH_I4U, ORKH_ALGO_TILED2, 16, 64, 0, 0.0000, 0.0225},   {ORKH_I4U, ORKH_ALGO_TILED2, 32, 32, 0, 0.0788, 0.0120},
     {ORKH_I4U, ORKH_ALGO_TILED2, 32, 64, 0, 0.0253, 0.0183},   {ORKH_I4U, ORKH_ALGO_TILED2, 64, 64, 0, 0.6958, 0.0116},
     {ORKH_I4U, ORKH_ALGO_TILED2, 64, 192, 0, 1.2931, 0.0178},  {ORKH_I4U, ORKH_ALGO_TILED2, 128, 96, 0, 0.0000, 0.0228},
@@ -626,7 +626,10 @@ static double tile_kib(int rkind, int bm, int bn, int kbs) {
     return ((double)bm * a_bytes_per_kb(rkind) + bn * 64.0) * kbs / 1024;
 }
 
-/* Price of orki_plan's pick q over its wgs workgroups, times the kind's margin; mb: C's megabytes */
+/* Price of orki_plan's pick q over its wgs workgroups, times the kind's margin; mb: C's megabytes. From K = 256 (the
+ * timed range) a 256 x 256 pick moves wherever a k_big tile is offered: over the 86 timed int8 and fp16 shapes with that pick the rule's k_big tile was at most
+ * 4.1% slower (int8 K=256 N=12288 M=3300 40.2 -> 41.8 us) and up to 15% faster where the fits call them level (int8 K=256
+ * N=12288 M=4096 54.0 -> 46.1, fp16 K=1024 N=8192 M=3300 79.1 -> 70.8). */
 static double pick_us(int rkind, const orkh_plan *q, long wgs, int KB, double mb, int cu) {
     const struct pick_fit *p = pick_fits;
     while (p->rkind != rkind) p++;
@@ -635,6 +638,7 @@ static double pick_us(int rkind, const orkh_plan *q, long wgs, int KB, double mb
            (r->bm && (r->algo != q->algo || r->bm != q->bm || r->bn != q->bn || r->ring != q->ring)))
         r++;
     const int ks = q->ksplit > 1 ? q->ksplit : 1;
+    if (q->bm == 256 && q->bn == 256 && KB * kpb_of(rkind) >= 256) return 1e30;
     const double rounds = (double)((wgs + cu - 1) / cu);
     double t = p->a + rounds * (r->b + r->c * tile_kib(rkind, q->bm, q->bn, ks > 1 ? q->kbs : KB)) + (wgs <= cu ? p->e1 : p->e2) * mb;
     if (ks > 1) t += p->d + p->f * ks * mb;
