@@ -555,13 +555,15 @@ static int plan_core(const ork_npu *c, int rkind, int M, int K, int N, int KB, o
  *   orki_plan's pick    a + rounds * (b[tile] + c[tile] * KiB) + e * MB + [ks > 1] (d + f * ks * MB)
  *                                                                  (e: e1 on one round, else e2)
  * Each is a least-squares fit in relative error (non-negative terms) to launches timed on MI355X, every k_big tile and
- * orki_plan's pick at 18 (K, N) with K from 256 to 8192 and N from 512 to 12288 and row counts from 65 to 4096, per weight
- * kind (367 shapes a kind, tests/golden/big_plan_sweep.json); 3-8% rms. Total us over them, former picks, this rule, the
- * faster of the two everywhere: int8 6438, 5957, 5951; fp16 10641, 9859, 9834; uniform int4 6099, 5271, 5270; NF4 8172, 7096,
- * 7091. No shape runs 2% slower than its former pick (256 x 256: 5%). (Fits without the costs per launch and round, made from K = 2048 up,
- * took tiles at K = 256 and 512 that ran up to 42% slower: fp16 K=256 N=6144 M=2689 33.4 us on 256 x 256, 23.5 on 128 x
- * 128.) On 876 more shapes at 20 random (K, N), K from 160 to 7360: 12,126 us by the former picks, 11,016 by this rule,
- * 10,909 the faster of the two everywhere; the worst 4.7% slower than its pick (int8 K=288 N=1920 M=3442 9.23 -> 9.66).
+ * orki_plan's pick at 31 (K, N) with K from 256 to 8192 and N from 512 to 16384 and row counts from 65 to 4096, per weight
+ * kind (633 shapes a kind, tests/golden/big_plan_sweep.json); 3-8% rms. Total us over them, former picks, this rule, the
+ * faster of the two everywhere: int8 12105, 11260, 11242; fp16 20187, 18886, 18819; uniform int4 11630, 10031, 10013; NF4
+ * 15668, 13623, 13616. No shape runs 4% slower than its former pick (256 x 256: 11%). Fits without the costs per launch and
+ * round, made from K = 2048 up, took tiles at K = 256 and 512 that ran up to 42% slower: fp16 K=256 N=6144 M=2689 33.4 us on
+ * 256 x 256, 23.5 on 128 x 128. On 876 more shapes at 20 random (K, N), K from 160 to 7360: 12,126 us by the former picks,
+ * 11,015 by this rule, 10,909 the faster of the two everywhere; the worst 4.7% slower than its pick (int8 K=288 N=1920
+ * M=3442 9.23 -> 9.66). What the prices do not see is a memory-bound C: at K=896 N=9728, the worst timed, one tile or the
+ * other is up to 14% ahead of the price's choice (int8 M=4096 62.7 -> 69.5 us, uniform int4 61.0 on k_big, 69.6 kept).
  * The margin keeps a pick whose price is that close. Some shapes, us: int8 K=N=4096 M=4096 65.0 -> 61.3, K=6144 N=2048
  * M=4096 63.3 -> 49.3; fp16 K=2048 N=6144 M=4096 140.6 -> 114.3; uniform int4 K=N=4096 M=4096 89.8 -> 52.3; NF4 112.0 ->
  * 67.3, K=2048 N=6144 M=1000 29.5 -> 24.2. At 512 rows and fewer the smaller tiles fill the CUs better and keep the run
@@ -576,49 +578,49 @@ static const struct big_fit {
     int rkind, bm, bn;
     double a, b, c, e;
 } big_fits[] = {
-    {ORKH_I8, 256, 256, 0.0000, 5.7765, 0.0205, 0.1218},  {ORKH_I8, 256, 192, 0.0000, 5.1089, 0.0211, 0.1093},
-    {ORKH_I8, 128, 256, 0.0000, 4.8479, 0.0162, 0.0922},  {ORKH_I8, 128, 192, 0.2062, 4.4958, 0.0169, 0.0682},
-    {ORKH_F16, 256, 256, 0.0000, 5.6807, 0.0211, 0.1345}, {ORKH_F16, 256, 192, 0.0000, 4.7918, 0.0216, 0.1308},
-    {ORKH_F16, 128, 256, 0.0000, 4.5878, 0.0164, 0.1335}, {ORKH_F16, 128, 192, 0.0000, 4.2631, 0.0172, 0.1092},
-    {ORKH_I4U, 256, 256, 0.0000, 9.0208, 0.0249, 0.0493}, {ORKH_I4U, 256, 192, 0.8432, 4.6144, 0.0227, 0.1034},
-    {ORKH_I4U, 128, 256, 0.0000, 5.4960, 0.0243, 0.0511}, {ORKH_I4U, 128, 192, 0.6367, 4.1975, 0.0214, 0.0625},
-    {ORKH_NF4, 256, 256, 0.0000, 9.7801, 0.0335, 0.0432}, {ORKH_NF4, 256, 192, 0.7795, 5.3498, 0.0317, 0.0895},
-    {ORKH_NF4, 128, 256, 0.2060, 5.6790, 0.0433, 0.0402}, {ORKH_NF4, 128, 192, 0.5242, 4.5105, 0.0393, 0.0465},
+    {ORKH_I8, 256, 256, 0.0000, 5.8445, 0.0207, 0.1215},  {ORKH_I8, 256, 192, 0.0000, 5.0543, 0.0211, 0.1120},
+    {ORKH_I8, 128, 256, 0.0000, 4.8374, 0.0161, 0.0988},  {ORKH_I8, 128, 192, 0.0841, 4.6869, 0.0167, 0.0681},
+    {ORKH_F16, 256, 256, 0.0000, 5.1371, 0.0213, 0.1476}, {ORKH_F16, 256, 192, 0.0000, 4.6484, 0.0215, 0.1365},
+    {ORKH_F16, 128, 256, 0.0000, 4.4193, 0.0163, 0.1458}, {ORKH_F16, 128, 192, 0.0000, 4.2182, 0.0171, 0.1170},
+    {ORKH_I4U, 256, 256, 0.0000, 8.8331, 0.0253, 0.0537}, {ORKH_I4U, 256, 192, 0.6961, 4.8054, 0.0228, 0.1019},
+    {ORKH_I4U, 128, 256, 0.0906, 5.3810, 0.0244, 0.0544}, {ORKH_I4U, 128, 192, 0.6025, 4.2765, 0.0214, 0.0620},
+    {ORKH_NF4, 256, 256, 0.0000, 9.5851, 0.0337, 0.0481}, {ORKH_NF4, 256, 192, 0.7750, 5.3310, 0.0317, 0.0906},
+    {ORKH_NF4, 128, 256, 0.3416, 5.4280, 0.0434, 0.0472}, {ORKH_NF4, 128, 192, 0.5835, 4.4760, 0.0394, 0.0468},
 };
 #define BIG_F16_SUMS(bm) ((bm) == 128 ? 2 : 1) /* BG::CH of the kernel */
 static const struct pick_fit {
     int rkind;
     double margin, a, e1, e2, d, f;
 } pick_fits[] = {
-    {ORKH_I8, 0.99, 2.0978, 0.1376, 0.1707, 2.7595, 0.4158},
-    {ORKH_F16, 0.97, 1.9090, 0.1646, 0.1662, 2.6121, 0.4608},
-    {ORKH_I4U, 0.99, 2.9182, 0.0677, 0.1019, 2.8818, 0.4031},
-    {ORKH_NF4, 0.99, 2.1372, 0.0642, 0.1122, 2.5850, 0.3767},
+    {ORKH_I8, 0.99, 2.2018, 0.1412, 0.1751, 2.8660, 0.3011},
+    {ORKH_F16, 0.96, 1.8442, 0.1792, 0.1781, 2.8651, 0.3646},
+    {ORKH_I4U, 0.97, 2.4471, 0.0620, 0.1151, 1.8313, 0.4186},
+    {ORKH_NF4, 0.99, 2.1421, 0.0546, 0.1092, 2.3528, 0.3783},
 };
 static const struct pick_rate { /* b and c of a tile; bm 0: a tile that no timed shape picked, at the kind's lowest rate */
     int rkind, algo, bm, bn, ring;
     double b, c;
 } pick_rates[] = {
-    {ORKH_I8, ORKH_ALGO_TILED2, 16, 64, 0, 0.0000, 0.0299},    {ORKH_I8, ORKH_ALGO_TILED2, 32, 32, 0, 0.5247, 0.0153},
-    {ORKH_I8, ORKH_ALGO_TILED2, 32, 64, 0, 0.7462, 0.0205},    {ORKH_I8, ORKH_ALGO_TILED2, 64, 64, 0, 0.3034, 0.0162},
-    {ORKH_I8, ORKH_ALGO_TILED2, 64, 192, 0, 0.0311, 0.0160},   {ORKH_I8, ORKH_ALGO_TILED2, 64, 192, 2, 0.1355, 0.0157},
-    {ORKH_I8, ORKH_ALGO_TILED2, 128, 96, 0, 1.5378, 0.0152},   {ORKH_I8, ORKH_ALGO_TILED2, 128, 96, 2, 1.5462, 0.0151},
-    {ORKH_I8, ORKH_ALGO_TILED2, 128, 128, 0, 0.3674, 0.0169},  {ORKH_I8, ORKH_ALGO_TILED2, 128, 128, 2, 0.0000, 0.0179},
-    {ORKH_I8, 0, 0, 0, 0, 0.0000, 0.0151},
-    {ORKH_F16, ORKH_ALGO_TILED2, 16, 64, 0, 0.0000, 0.0234},   {ORKH_F16, ORKH_ALGO_TILED2, 32, 32, 0, 0.8556, 0.0137},
-    {ORKH_F16, ORKH_ALGO_TILED2, 32, 64, 0, 0.8593, 0.0194},   {ORKH_F16, ORKH_ALGO_TILED2, 64, 64, 0, 0.4737, 0.0170},
-    {ORKH_F16, ORKH_ALGO_TILED2, 64, 192, 0, 0.4262, 0.0162},  {ORKH_F16, ORKH_ALGO_TILED2, 64, 192, 2, 0.0000, 0.0178},
-    {ORKH_F16, ORKH_ALGO_TILED2, 128, 96, 0, 1.1402, 0.0166},  {ORKH_F16, ORKH_ALGO_TILED2, 128, 96, 2, 0.6158, 0.0161},
-    {ORKH_F16, ORKH_ALGO_TILED2, 128, 128, 0, 0.0000, 0.0175}, {ORKH_F16, ORKH_ALGO_TILED2, 128, 128, 2, 0.0000, 0.0191},
-    {ORKH_F16, 0, 0, 0, 0, 0.0000, 0.0137},
-    {ORKH_I4U, ORKH_ALGO_TILED2, 16, 64, 0, 0.0000, 0.0225},   {ORKH_I4U, ORKH_ALGO_TILED2, 32, 32, 0, 0.0788, 0.0120},
-    {ORKH_I4U, ORKH_ALGO_TILED2, 32, 64, 0, 0.0253, 0.0183},   {ORKH_I4U, ORKH_ALGO_TILED2, 64, 64, 0, 0.6958, 0.0116},
-    {ORKH_I4U, ORKH_ALGO_TILED2, 64, 192, 0, 1.2931, 0.0178},  {ORKH_I4U, ORKH_ALGO_TILED2, 128, 96, 0, 0.0000, 0.0228},
-    {ORKH_I4U, ORKH_ALGO_TILED2, 128, 128, 0, 0.3711, 0.0220}, {ORKH_I4U, ORKH_ALGO_TILED2, 128, 128, 2, 0.5890, 0.0207},
-    {ORKH_I4U, 0, 0, 0, 0, 0.0000, 0.0116},
-    {ORKH_NF4, ORKH_ALGO_TILED, 64, 64, 0, 4.3708, 0.0232},    {ORKH_NF4, ORKH_ALGO_TILED2, 32, 64, 0, 0.7359, 0.0297},
-    {ORKH_NF4, ORKH_ALGO_TILED2, 64, 64, 0, 0.5259, 0.0326},   {ORKH_NF4, ORKH_ALGO_TILED2, 128, 96, 0, 2.4996, 0.0273},
-    {ORKH_NF4, ORKH_ALGO_TILED2, 128, 128, 0, 1.7391, 0.0284}, {ORKH_NF4, 0, 0, 0, 0, 0.0000, 0.0232},
+    {ORKH_I8, ORKH_ALGO_TILED2, 16, 64, 0, 0.0000, 0.0286},   {ORKH_I8, ORKH_ALGO_TILED2, 32, 32, 0, 0.4549, 0.0149},
+    {ORKH_I8, ORKH_ALGO_TILED2, 32, 64, 0, 0.6428, 0.0206},   {ORKH_I8, ORKH_ALGO_TILED2, 64, 64, 0, 0.2054, 0.0161},
+    {ORKH_I8, ORKH_ALGO_TILED2, 64, 192, 0, 0.3891, 0.0162},  {ORKH_I8, ORKH_ALGO_TILED2, 64, 192, 2, 0.0155, 0.0156},
+    {ORKH_I8, ORKH_ALGO_TILED2, 128, 96, 0, 1.9867, 0.0143},  {ORKH_I8, ORKH_ALGO_TILED2, 128, 96, 2, 2.8802, 0.0133},
+    {ORKH_I8, ORKH_ALGO_TILED2, 128, 128, 0, 0.2091, 0.0169}, {ORKH_I8, ORKH_ALGO_TILED2, 128, 128, 2, 0.0000, 0.0176},
+    {ORKH_I8, 0, 0, 0, 0, 0.0000, 0.0133},
+    {ORKH_F16, ORKH_ALGO_TILED2, 16, 64, 0, 0.0000, 0.0237},   {ORKH_F16, ORKH_ALGO_TILED2, 32, 32, 0, 0.7276, 0.0150},
+    {ORKH_F16, ORKH_ALGO_TILED2, 32, 64, 0, 0.8455, 0.0198},   {ORKH_F16, ORKH_ALGO_TILED2, 64, 64, 0, 0.4332, 0.0171},
+    {ORKH_F16, ORKH_ALGO_TILED2, 64, 192, 0, 1.2045, 0.0164},  {ORKH_F16, ORKH_ALGO_TILED2, 64, 192, 2, 0.2182, 0.0170},
+    {ORKH_F16, ORKH_ALGO_TILED2, 128, 96, 0, 1.6126, 0.0156},  {ORKH_F16, ORKH_ALGO_TILED2, 128, 96, 2, 0.6610, 0.0157},
+    {ORKH_F16, ORKH_ALGO_TILED2, 128, 128, 0, 0.0000, 0.0173}, {ORKH_F16, ORKH_ALGO_TILED2, 128, 128, 2, 0.0000, 0.0184},
+    {ORKH_F16, 0, 0, 0, 0, 0.0000, 0.0150},
+    {ORKH_I4U, ORKH_ALGO_TILED2, 16, 64, 0, 0.0000, 0.0324},   {ORKH_I4U, ORKH_ALGO_TILED2, 32, 32, 0, 0.5442, 0.0121},
+    {ORKH_I4U, ORKH_ALGO_TILED2, 32, 64, 0, 0.5358, 0.0181},   {ORKH_I4U, ORKH_ALGO_TILED2, 64, 64, 0, 1.0193, 0.0132},
+    {ORKH_I4U, ORKH_ALGO_TILED2, 64, 192, 0, 1.9941, 0.0175},  {ORKH_I4U, ORKH_ALGO_TILED2, 128, 96, 0, 2.3002, 0.0201},
+    {ORKH_I4U, ORKH_ALGO_TILED2, 128, 128, 0, 0.8814, 0.0220}, {ORKH_I4U, ORKH_ALGO_TILED2, 128, 128, 2, 0.5425, 0.0210},
+    {ORKH_I4U, 0, 0, 0, 0, 0.0000, 0.0121},
+    {ORKH_NF4, ORKH_ALGO_TILED, 64, 64, 0, 3.8499, 0.0248},    {ORKH_NF4, ORKH_ALGO_TILED2, 32, 64, 0, 0.7575, 0.0299},
+    {ORKH_NF4, ORKH_ALGO_TILED2, 64, 64, 0, 0.5283, 0.0328},   {ORKH_NF4, ORKH_ALGO_TILED2, 128, 96, 0, 2.7709, 0.0275},
+    {ORKH_NF4, ORKH_ALGO_TILED2, 128, 128, 0, 1.8063, 0.0284}, {ORKH_NF4, 0, 0, 0, 0, 0.0000, 0.0248},
 };
 
 /* A and B KiB that one workgroup of a bm x bn tile loads over kbs K-blocks */
@@ -627,8 +629,8 @@ static double tile_kib(int rkind, int bm, int bn, int kbs) {
 }
 
 /* Price of orki_plan's pick q over its wgs workgroups, times the kind's margin; mb: C's megabytes. From K = 256 (the
- * timed range) a 256 x 256 pick moves wherever a k_big tile is offered: over the 86 timed int8 and fp16 shapes with that pick the rule's k_big tile was at most
- * 4.1% slower (int8 K=256 N=12288 M=3300 40.2 -> 41.8 us) and up to 15% faster where the fits call them level (int8 K=256
+ * timed range) a 256 x 256 pick moves wherever a k_big tile is offered: over the 143 timed int8 and fp16 shapes with that pick the rule's k_big tile was more
+ * than 4% slower at three (int8 K=256 N=12288 M=3300 40.2 -> 41.8 us, K=896 N=9728) and up to 15% faster where the fits call them level (int8 K=256
  * N=12288 M=4096 54.0 -> 46.1, fp16 K=1024 N=8192 M=3300 79.1 -> 70.8). */
 static double pick_us(int rkind, const orkh_plan *q, long wgs, int KB, double mb, int cu) {
     const struct pick_fit *p = pick_fits;

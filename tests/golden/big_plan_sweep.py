@@ -23,10 +23,13 @@ import sys
 ROOT = os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 OUT = os.path.join(os.path.dirname(os.path.abspath(__file__)), "big_plan_sweep.json")
 PAIRS = ((256, 2048), (256, 6144), (256, 12288), (512, 4096), (512, 12288), (1024, 1024), (1024, 3072), (1024, 8192), (2048, 512),
-         (2048, 2048), (2048, 4096), (2048, 6144), (2048, 12288), (4096, 1024), (4096, 4096), (4096, 11008), (6144, 2048), (8192, 4096))
+         (2048, 2048), (2048, 4096), (2048, 6144), (2048, 12288), (4096, 1024), (4096, 4096), (4096, 11008), (6144, 2048), (8192, 4096),
+         (896, 4864), (896, 9728), (1536, 1536), (2048, 8192), (2048, 16384), (2560, 9728), (3072, 5120), (4096, 512), (4096, 2560),
+         (6144, 1024), (8192, 512), (8192, 1024), (8192, 2560))
 ROWS = (65, 96, 128, 160, 200, 257, 320, 384, 448, 512, 641, 769, 900, 1024, 1280, 1537, 1793, 2048, 2689, 3300, 4096)
 CHAINS = ((2048, (2048, 1024, 1024)), (2048, (6144, 6144)), (2048, (2048, 2048, 2048)), (2048, (1024, 1024)), (2048, (2048, 512, 512)),
-          (4096, (4096, 2048)), (4096, (4096, 4096, 4096)), (1024, (3072, 1024, 1024)), (4096, (11008, 11008)), (512, (4096, 4096)))
+          (4096, (4096, 2048)), (4096, (4096, 4096, 4096)), (1024, (3072, 1024, 1024)), (4096, (11008, 11008)), (512, (4096, 4096)),
+          (896, (4864, 4864)), (2048, (8192, 8192)), (8192, (2048, 512)), (8192, (1024, 1024)), (6144, (1024, 512, 512)))
 CHAIN_ROWS = (65, 128, 200, 256, 384, 500, 641, 769, 897, 1024, 1281, 1537, 1793, 2048, 2689)
 BIG = ("256x256", "256x192", "128x256", "128x192")
 CHAIN_TILES = ("128x128", "128x96", "64x192", "64x64")   # the smaller tiles of a joint launch
