@@ -6,8 +6,8 @@
  * independent matmuls, each result equal to its single run; -2 for bad arguments (S outside 1..1024,
  * NULL weight, M < 1, wrong dtype), -1 for A/C overlap; C row stride override (cstride) for int8.
  * What changes: no PC-chained NPU programs, cores or doorbells. Every M = 1 task of one resident kind
- * goes into a grouped GEMV launch (ORKH_GROUP_MAX tasks each); tasks of one integer kind, M > 1 and K whose summed
- * columns plan to the LDS-ring kernel unsplit go into one grouped tiled launch (ORKH_TGROUP_MAX each: a
+ * goes into a grouped GEMV launch (ORKH_GROUP_MAX tasks each); tasks of one integer kind, M > 1 and K that
+ * plan to a joint launch (orki_plan_group) go into one grouped tiled launch (ORKH_TGROUP_MAX each: a
  * prefill's q/k/v or gate/up); the remaining tasks launch back to back
  * on the context's stream with their normal plans, and host operands move in one pinned staging pass. An
  * offline context runs each task's host codes on the CPU (cpu_chain below), as the reference's int8 chain
@@ -149,24 +149,22 @@ static int chain_common(const char *who, ork_npu *c, int S, ctask *t, int want_d
         }
         if (orkh_mm_launch_group(&g, wpg, c->stream)) { orki_hip_fail(who); rc = -1; }
     }
-    /* grouped tiled launches: tasks of one integer resident kind, M > 1 and K whose columns together plan to the
-     * LDS-ring kernel unsplit, ORKH_TGROUP_MAX at a time, under the tile planned for their summed N (integer results
+    /* grouped tiled launches: tasks of one integer resident kind, M > 1 and K, ORKH_TGROUP_MAX at a time,
+     * where orki_plan_group joins them: on the LDS-ring kernel unsplit or the many-row kernel (integer results
      * are exact under any tile; fp16 tasks keep their own tiles, so each result still equals its single run) */
     for (int i = 0; i < S && !rc; i++) {
         if (done[i] || t[i].M == 1 || t[i].w->rkind == ORKH_F16) continue;
-        int mem[ORKH_TGROUP_MAX], n = 0, nsum = 0;
+        int mem[ORKH_TGROUP_MAX], Ns[ORKH_TGROUP_MAX], n = 0;
         for (int j = i; j < S && n < ORKH_TGROUP_MAX; j++) {
             if (done[j] || t[j].M != t[i].M || t[j].w->rkind != t[i].w->rkind || t[j].w->K != t[i].w->K ||
                 t[j].w->KB != t[i].w->KB)
                 continue;
+            Ns[n] = t[j].w->N;
             mem[n++] = j;
-            nsum += t[j].w->N;
         }
         if (n < 2) continue;
         orkh_plan gq;
-        size_t gws = 0;
-        orki_plan_mm(c, t[i].w->rkind, t[i].M, t[i].w->K, nsum, t[i].w->KB, &gq, &gws);
-        if ((gq.algo != ORKH_ALGO_TILED2 && gq.algo != ORKH_ALGO_BIG) || gq.ksplit > 1) continue;
+        if (!orki_plan_group(c, t[i].w->rkind, t[i].M, t[i].w->K, Ns, n, t[i].w->KB, &gq)) continue;
         orkh_mm ps[ORKH_TGROUP_MAX];
         memset(ps, 0, sizeof ps);
         for (int k = 0; k < n; k++) {

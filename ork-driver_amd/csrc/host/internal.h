@@ -107,6 +107,9 @@ void   orki_tile_nib_kn(const int8_t *B_kn, int K, int N, int KB, uint8_t *out);
 int orki_plan(const ork_npu *c, int rkind, int M, int K, int N, int KB, orkh_plan *q, size_t *ws_bytes);
 /* The plan of a run: orki_plan's, or the many-row kernel where its model prices it lower. */
 int orki_plan_mm(const ork_npu *c, int rkind, int M, int K, int N, int KB, orkh_plan *q, size_t *ws_bytes);
+/* One launch for n matmuls of one kind, M and K with N[i] columns: 1 and its plan (LDS-ring or many-row kernel, unsplit), or
+ * 0 where they run one by one. */
+int orki_plan_group(const ork_npu *c, int rkind, int M, int K, const int *N, int n, int KB, orkh_plan *q);
 /* Waves per workgroup of the whole-panel GEMV for this weight (the grouped M = 1 launch of the multi-matmul submit). */
 int orki_gemv_panel_wpg(const ork_npu *c, int rkind, int KB, int NB);
 /* Kernel for a grouped-scale run (never K-split). */

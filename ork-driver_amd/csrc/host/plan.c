@@ -660,7 +660,18 @@ static int overridden(const ork_npu *c) {
     return 0;
 }
 
-static void take_big(const ork_npu *c, int bm, int bn, int M, int N, int KB, orkh_plan *q, size_t *ws_bytes) {
+/* Workgroups of a launch of bm x bn tiles over n matmuls of N[i] columns. Each matmul of a joint launch has tiles of its own
+ * and starts on the first XCD (workgroup b runs on XCD b % 8), so it fills whole rows of eight: the first XCD has that many
+ * to run, whatever the others have (int8 K=2048 N=2048+1024+1024 M=1281 on 128 x 192: 253 tiles, 34 of them on the first
+ * XCD's 32 CUs, two rounds). */
+static long tiles_of(int M, const int *N, int n, int bm, int bn) {
+    if (n == 1) return (long)cdiv(M, bm) * cdiv(N[0], bn);
+    long w = 0;
+    for (int i = 0; i < n; i++) w += ((long)cdiv(M, bm) * cdiv(N[i], bn) + 7) / 8 * 8;
+    return w;
+}
+
+static void take_big(const ork_npu *c, int bm, int bn, int M, const int *N, int n, int KB, orkh_plan *q) {
     const int cu = (c && c->cores > 0) ? c->cores : 256;
     memset(q, 0, sizeof *q);
     q->algo = ORKH_ALGO_BIG;
@@ -668,38 +679,82 @@ static void take_big(const ork_npu *c, int bm, int bn, int M, int N, int KB, ork
     q->bn = bn;
     q->ksplit = 1;
     q->kbs = KB;
-    q->cwt = (long)cdiv(M, bm) * cdiv(N, bn) <= cu; /* write-through C on one round, as orki_plan's tiles */
-    *ws_bytes = 0;
+    q->cwt = tiles_of(M, N, n, bm, bn) <= cu; /* write-through C on one round, as orki_plan's tiles */
+}
+
+/* The k_big tile priced below `limit` us for n matmuls of N[i] columns, with at least `sums` fp32 sums an output; 0: none. */
+static const struct big_fit *big_best(int rkind, int M, const int *N, int n, int KB, double mb, int cu, int sums, double limit) {
+    const struct big_fit *best = NULL;
+    for (size_t j = 0; j < sizeof big_fits / sizeof big_fits[0]; j++) {
+        const struct big_fit *g = &big_fits[j];
+        if (g->rkind != rkind || (rkind == ORKH_F16 && BIG_F16_SUMS(g->bm) < sums)) continue;
+        const double t = big_us(g, tiles_of(M, N, n, g->bm, g->bn), KB, mb, cu);
+        if (t < limit) {
+            limit = t;
+            best = g;
+        }
+    }
+    return best;
+}
+
+/* ORK_PLAN=big with ORK_TILE=BMxBN */
+static int forced_big(int *bm, int *bn) {
+    const char *f = getenv("ORK_PLAN"), *t = getenv("ORK_TILE");
+    return f && !strcmp(f, "big") && t && sscanf(t, "%dx%d", bm, bn) == 2;
 }
 
 int orki_plan_mm(const ork_npu *c, int rkind, int M, int K, int N, int KB, orkh_plan *q, size_t *ws_bytes) {
     const int rc = orki_plan(c, rkind, M, K, N, KB, q, ws_bytes);
     if (rc || M <= 64) return rc;
+    int bm, bn;
     if (overridden(c)) {
-        const char *f = getenv("ORK_PLAN"), *t = getenv("ORK_TILE");
-        int bm, bn;
-        if (f && !strcmp(f, "big") && t && sscanf(t, "%dx%d", &bm, &bn) == 2) take_big(c, bm, bn, M, N, KB, q, ws_bytes);
+        if (!forced_big(&bm, &bn)) return 0;
+        take_big(c, bm, bn, M, &N, 1, KB, q);
+        *ws_bytes = 0;
         return 0;
     }
     if (q->algo != ORKH_ALGO_TILED2 && q->algo != ORKH_ALGO_TILED) return 0;
-    const int cu = (c && c->cores > 0) ? c->cores : 256;
-    const int ks = q->ksplit > 1 ? q->ksplit : 1;
+    const int cu = (c && c->cores > 0) ? c->cores : 256, ks = q->ksplit > 1 ? q->ksplit : 1;
     const double mb = (double)M * N * 4 / 1e6;
-    double best = pick_us(rkind, q, (long)cdiv(M, q->bm) * cdiv(N / 16, q->bn / 16) * ks, KB, mb, cu);
+    const double us = pick_us(rkind, q, tiles_of(M, &N, 1, q->bm, q->bn) * ks, KB, mb, cu);
     const int sums = rkind == ORKH_F16 ? tiled2_kgroups(rkind, q->bm, q->bn) * ks : 1;
-    int bm = 0, bn = 0;
-    for (size_t j = 0; j < sizeof big_fits / sizeof big_fits[0]; j++) {
-        const struct big_fit *g = &big_fits[j];
-        if (g->rkind != rkind || (rkind == ORKH_F16 && BIG_F16_SUMS(g->bm) < sums)) continue;
-        const double t = big_us(g, (long)cdiv(M, g->bm) * cdiv(N, g->bn), KB, mb, cu);
-        if (t < best) {
-            best = t;
-            bm = g->bm;
-            bn = g->bn;
-        }
-    }
-    if (bm) take_big(c, bm, bn, M, N, KB, q, ws_bytes);
+    const struct big_fit *g = big_best(rkind, M, &N, 1, KB, mb, cu, sums, us);
+    if (!g) return 0;
+    take_big(c, g->bm, g->bn, M, &N, 1, KB, q);
+    *ws_bytes = 0;
     return 0;
+}
+
+/* The joint launch of n matmuls of one input (the multi-matmul submit): the LDS-ring tile that orki_plan picks for their
+ * summed columns, unsplit, or a k_big tile. Each task has tiles of its own, so both are priced at the tiles launched, not at
+ * the summed columns' (us, the tile priced at the summed columns, then this rule: int8 K=2048 N=2048+1024+1024 M=1281 264
+ * tiles of 128 x 192 30.1, 22.2 on 64 x 192; K=4096 3 x N=4096 M=769 82.0, 61.1; uniform int4 K=2048 3 x N=2048 M=1793 48.1,
+ * 36.2; NF4 K=2048 2 x N=1024 M=2689 45.3, 32.3); the joint LDS-ring launch always has the 4-slot ring. Timed at 15
+ * lists of widths and 15 row counts, us, orki_plan's tile, this rule: int8 4596, 3837; uniform int4 6773, 5330; NF4 8185,
+ * 6685 (one shape over 1% slower: NF4 K=896 2 x N=4864 M=1537, 4.4%). Where orki_plan's pick is no joint launch (K split)
+ * the tasks run one by one: no k_big tile was ahead at the 54 such shapes (NF4 K=8192 2 x N=1024 M=1024 50.6 us, 75.8). */
+int orki_plan_group(const ork_npu *c, int rkind, int M, int K, const int *N, int n, int KB, orkh_plan *q) {
+    int nsum = 0, bm, bn;
+    size_t ws = 0;
+    for (int i = 0; i < n; i++) nsum += N[i];
+    if (orki_plan(c, rkind, M, K, nsum, KB, q, &ws)) return 0;
+    const int joint = q->algo == ORKH_ALGO_TILED2 && q->ksplit <= 1;
+    if (M <= 64) return joint;
+    if (overridden(c)) {
+        if (!forced_big(&bm, &bn)) return joint;
+        take_big(c, bm, bn, M, N, n, KB, q);
+        return 1;
+    }
+    if (!joint) return 0;
+    const int cu = (c && c->cores > 0) ? c->cores : 256;
+    const double mb = (double)M * nsum * 4 / 1e6;
+    orkh_plan ring4 = *q;
+    ring4.ring = 0;
+    const double us = pick_us(rkind, &ring4, tiles_of(M, N, n, q->bm, q->bn), KB, mb, cu);
+    const int sums = rkind == ORKH_F16 ? tiled2_kgroups(rkind, q->bm, q->bn) : 1;
+    const struct big_fit *g = big_best(rkind, M, N, n, KB, mb, cu, sums, us);
+    if (g) take_big(c, g->bm, g->bn, M, N, n, KB, q);
+    return 1;
 }
 
 /* Grouped-scale runs (ork_*_mm_run_grouped). The groups must close in ascending order inside one workgroup, so

@@ -1,5 +1,6 @@
 /* Prints the planner's choice for each "kind M K N" argument quadruple on a 256-CU device, one line each, named as
- * the library names its launches (orkh_mm_variant): orki_plan's, or after a first argument "mm" a run's (orki_plan_mm). Built from the host planner source alone, with no GPU code. */
+ * the library names its launches (orkh_mm_variant): orki_plan's, or after a first argument "mm" a run's (orki_plan_mm); after "chain", for each
+ * "kind M K n N1 .. Nn", the joint launch of n matmuls ("single": none; orki_plan_group). Built from the host planner source alone, with no GPU code. */
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -47,6 +48,18 @@ int main(int argc, char **argv) {
     ork_npu c;
     memset(&c, 0, sizeof c);
     c.cores = 256;
+    if (argc > 1 && !strcmp(argv[1], "chain")) {
+        for (int i = 2; i + 3 < argc;) {
+            const int kind = atoi(argv[i]), M = atoi(argv[i + 1]), K = atoi(argv[i + 2]), n = atoi(argv[i + 3]);
+            const int kpb = kind == ORKH_I8 ? 64 : kind == ORKH_F16 ? 32 : 128;
+            int N[ORKH_TGROUP_MAX];
+            orkh_plan q;
+            for (int k = 0; k < n && k < ORKH_TGROUP_MAX; k++) N[k] = atoi(argv[i + 4 + k]);
+            printf("%d %d %d %d %s\n", kind, M, K, n, orki_plan_group(&c, kind, M, K, N, n, (K + kpb - 1) / kpb, &q) ? name(kind, &q) : "single");
+            i += 4 + n;
+        }
+        return 0;
+    }
     const int mm = argc > 1 && !strcmp(argv[1], "mm");
     for (int i = 1 + mm; i + 3 < argc; i += 4) {
         const int kind = atoi(argv[i]), M = atoi(argv[i + 1]), K = atoi(argv[i + 2]), N = atoi(argv[i + 3]);

@@ -30,8 +30,8 @@ def planner(tmp_path_factory):
                         "-o", exe, "-lm"], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stderr[-3000:]
 
-    def pick(cases, mm=False):
-        args = ["mm"] * mm + [str(x) for c in cases for x in c]
+    def pick(cases, mm=False, chain=False):
+        args = ["mm"] * mm + ["chain"] * chain + [str(x) for c in cases for x in c]
         out = subprocess.run([exe] + args, capture_output=True, text=True, timeout=60, env={}).stdout.split("\n")
         return [ln.split()[4] for ln in out if ln.strip()]
     return pick
@@ -134,6 +134,32 @@ def test_run_picks_against_the_sweep(planner, kind):
         tot_best += min(times.values())
         tot_former += us
     assert tot_pick <= 1.01 * tot_best and tot_pick < 0.94 * tot_former, (tot_pick, tot_best, tot_former)
+
+
+@pytest.mark.parametrize("kind", ["int8", "i4u", "nf4"])
+def test_chain_picks_against_the_sweep(planner, kind):
+    """The joint launch of a chain's matmuls against graph-timed launches (tests/golden/big_plan_sweep.json: 15 lists of
+    widths, M from 65 to 2689) on every many-row tile and on the LDS-ring tiles: where orki_plan's pick for the summed
+    columns is one of those, the joint launch is at most 5% slower than on it, and the total within 1% of the faster of
+    the two everywhere. Each task has tiles of its own: a tile priced at the summed columns' count ran up to 52% slower."""
+    data = json.load(open(os.path.join(ROOT, "tests", "golden", "big_plan_sweep.json")))
+    rows = [r for r in data["chains"] if r[0] == kind]
+    rk, kn = {"int8": (0, "i8"), "i4u": (1, "i4u"), "nf4": (2, "nf4")}[kind]
+    former = planner([(rk, M, K, sum(Ns)) for _, K, Ns, M, *_ in rows])
+    picks = planner([(rk, M, K, len(Ns), *Ns) for _, K, Ns, M, *_ in rows], chain=True)
+    tiles = ["big_%s_%s" % (kn, t) for t in ("256x256", "256x192", "128x256", "128x192")] + \
+            ["tiled2_%s_%s" % (kn, t) for t in ("128x128", "128x96", "64x192", "64x64")]
+    tot_pick = tot_best = n = 0
+    for (_, K, Ns, M, *us), f, p in zip(rows, former, picks):
+        times = {t: x for t, x in zip(tiles, us) if x}
+        f, p = ("_".join(x.split("_")[:3]) if "_ks" not in x else x for x in (f, p))
+        if f not in times:
+            continue
+        assert times[p] <= 1.05 * times[f], (K, Ns, M, f, times[f], p, times[p])
+        tot_pick += times[p]
+        tot_best += min(v for t, v in times.items() if t == f or t.startswith("big_"))
+        n += 1
+    assert n > 100 and tot_pick <= 1.01 * tot_best, (n, tot_pick, tot_best)
 
 
 def _f16_sums(name):
