@@ -22,7 +22,12 @@
 //  - MFMA operands swapped (D = B^T A^T): a lane holds four columns of one row, so a group's close needs one aS value per
 //    row block and one 16-byte read of bS per column block, and C goes out 16 bytes a store;
 //  - where a group is a compile-time number of steps or whole stages (GS), its end is known without a test, and its first
-//    step starts the accumulators from zero (W4A4 M=256 G=512, 64 x 64: 15.0 us with a test a step, 11.0 without);
+//    step starts the accumulators from zero (W4A4 M=256 G=512, 64 x 64: 15.0 us with a test a step, 11.0 without). Where
+//    the steps of a group do not divide a stage's the stage is compiled once for each place a group can stand in it (PH):
+//    us, a run-time count of steps or stages, then this: W4A4 64 x 64 K=6144 N=2048 M=256 G=192 20.5 -> 15.5, G=384 18.5
+//    -> 14.0, G=768 17.3 -> 13.2, K=N=3072 G=512 9.1 -> 8.7; int8 64 x 192 K=N=3072 M=768 G=192 22.0 -> 19.0, G=256 19.8
+//    -> 18.6, K=2048 N=6144 M=384 G=512 13.5 -> 13.0. Groups of whole 128-k spans of any other count are tested once a
+//    span (int8 64 x 64 K=6144 N=2048 M=256 G=384 19.6, tested each step, 17.4);
 //  - a stage's loads go out between the MFMAs of the steps before it, not all after the barrier, where they stall the waves
 //    while no MFMA runs (W4A4 M=256 G=128, 64 x 64: 14.3 -> 12.9); each load's kind is a compile-time one (15.7 to 15.1
 //    at two-line stages);
@@ -45,14 +50,31 @@ struct TG {
     const float *aS, *bS; // [M][K/G], [K/G][N]
 };
 
-// GS: steps per group where they are a compile-time 1, 2 or 4 (G == SK, or G == 128 and 256 at SK 64), -1: whole stages per
-// group, 0: any other count
+// GS: steps per group at compile time, where they divide a stage's or the ends recur after a few stages (launch_g), -1: whole
+// stages per group, -2: whole 128-k spans per group, 0: any other count
+constexpr int lcm_of(int a, int b) {
+    int x = a;
+    while (x % b) x += a;
+    return x;
+}
+constexpr int ends_in(int gs, int t, int ph, int to) { // groups of gs steps that end in the first `to` of a stage's t steps, phase ph
+    int n = 0;
+    for (int i = 0; i < to; i++) n += (ph * t + i + 1) % gs == 0;
+    return n;
+}
+constexpr int most_ends(int gs, int t) {
+    int m = 0;
+    for (int ph = 0; ph < lcm_of(gs, t) / t; ph++) m = ends_in(gs, t, ph, t) > m ? ends_in(gs, t, ph, t) : m;
+    return m;
+}
 template <int KIND, int SK, int GS, int BM, int BN, int SU> struct TGP {
     static constexpr bool NIB = KIND == ORKH_I4U;
     static constexpr int NW = 8, WM = 2, WN = 4;
     static constexpr int MTW = BM / 16 / WM, NTW = BN / 16 / WN;
     static constexpr int T = SU * 128 / SK;                                        // MFMA steps per stage
-    static constexpr int NG = GS < 0 ? 1 : GS == 0 ? (SK == 32 ? 2 : 1) * SU : T / GS; // groups that can end in a stage
+    static constexpr bool RT = GS == 0 || GS == -2;                                // a run-time count of steps or spans
+    static constexpr int PH = GS > 0 ? lcm_of(GS > 0 ? GS : 1, T) / T : 1;         // stages after which the ends recur
+    static constexpr int NG = GS == -1 ? 1 : RT ? (SK == 32 ? 2 : 1) * SU : most_ends(GS > 0 ? GS : 1, T); // groups that can end in a stage
     static constexpr int BPS = (NIB ? 1 : 2) * SU;                                 // panel blocks per panel and stage
     // Direct-to-LDS loads per stage: 1 KiB of A (a line of 8 rows) or B (a panel block), 256 bytes of aS or bS; QA, QB, QS
     // per wave (so that a load's kind is known at compile time), those without work landing in a junk block
@@ -62,7 +84,7 @@ template <int KIND, int SK, int GS, int BM, int BN, int SU> struct TGP {
     static constexpr int SLOT = SCB + NSB * 256, RMAX = (163840 - 1024) / SLOT, R = RMAX < 4 ? RMAX : 4;
     static constexpr int JUNK = R * SLOT, LDS = JUNK + 1024;
     static_assert(R >= 2 && MTW * WM * 16 == BM && NTW * WN * 16 == BN && T % 2 == 0 && QA * NW == NA && (R - 1) * LPW < 64 &&
-                      (GS <= 0 || T % (GS > 0 ? GS : 1) == 0),
+                      (GS != -2 || SK == 64),
                   "tile");
 };
 
@@ -264,8 +286,9 @@ __global__ __launch_bounds__(512, 1) void k_tiled2g(orkh_mm p, TG gp, int mtiles
     else wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    const int gsteps = gp.G / (GS < 0 ? SU * 128 : SK);
-    int cnt = 0; // steps (GS < 0: stages) of the running group done
+    constexpr int GQ = GS == -1 ? SU * 128 : GS == -2 ? 128 : SK; // k of what cnt counts
+    const int gsteps = gp.G / GQ;
+    int cnt = 0; // of the running group done: steps (GS -1: stages, -2: spans)
     // Stage s + 1 has landed (this wave's share; the barrier covers the others'), and every wave's reads of stage s are done,
     // so its slot takes stage s + R
     auto turn = [&](int s) {
@@ -276,14 +299,16 @@ __global__ __launch_bounds__(512, 1) void k_tiled2g(orkh_mm p, TG gp, int mtiles
     };
     rd(0, 0, 0);
     int rs = 0; // slot of stage s
-    for (int s = 0; s < nst; s++) {
+    auto stage = [&](int s, auto phc) {
+        constexpr int ph = decltype(phc)::value, GC = GS > 0 ? GS : 1;
         const int rn = rs + 1 == R ? 0 : rs + 1;
-        int e = 0; // groups ended in this stage
+        int e = 0; // groups ended in this stage (run-time counts)
         auto at = [&](auto tc) {
             constexpr int t = decltype(tc)::value, TI = P::T - 1; // the next stage to issue goes out over the first TI steps
-            const bool ends = GS > 0 ? (t + 1) % (GS > 0 ? GS : 1) == 0 : GS < 0 ? t == TI && cnt + 1 == gsteps : cnt + 1 == gsteps;
-            // (GS == 0: within a stage the close reads them itself: a branch a step, not two)
-            if (ends && (GS != 0 || t == TI)) rdS(rs, GS > 0 ? t / (GS > 0 ? GS : 1) : GS < 0 ? 0 : e);
+            constexpr bool place = (t + 1) * SK % GQ == 0;         // a group can end here
+            const bool ends = GS > 0 ? (ph * P::T + t + 1) % GC == 0 : place && cnt + 1 == gsteps;
+            // (a run-time count: within a stage the close reads them itself: a branch a place, not two)
+            if (ends && (!P::RT || t == TI)) rdS(rs, GS > 0 ? ends_in(GC, P::T, ph, t) : GS == -1 ? 0 : e);
             if constexpr (t < TI) {
                 rd(rs, t + 1, (t + 1) & 1);
             } else {
@@ -291,23 +316,27 @@ __global__ __launch_bounds__(512, 1) void k_tiled2g(orkh_mm p, TG gp, int mtiles
                 if (s + 1 < nst) rd(rn, 0, 0);
             }
             fence();
-            if constexpr (GS > 0 && t % (GS > 0 ? GS : 1) == 0) mm(t & 1, std::true_type{});
+            if constexpr (GS > 0 && (ph * P::T + t) % GC == 0) mm(t & 1, std::true_type{});
             else mm(t & 1, std::false_type{});
             if constexpr (t < TI) issue(std::integral_constant<int, LPW * t / TI>{}, std::integral_constant<int, LPW *(t + 1) / TI>{});
             if constexpr (t == TI - 1) next();
             fence();
             if (ends) {
-                if (GS == 0 && t < TI) rdS(rs, e);
+                if (P::RT && t < TI) rdS(rs, e);
                 close();
                 e++;
                 cnt = 0;
-            } else if (GS == 0 || (GS < 0 && t == TI)) {
+            } else if (GS <= 0 && place) {
                 cnt++;
             }
         };
         each(std::make_integer_sequence<int, P::T>{}, at);
         rs = rn;
-    }
+    };
+    for (int s = 0; s < nst; s += P::PH)
+        each(std::make_integer_sequence<int, P::PH>{}, [&](auto phc) {
+            if (decltype(phc)::value == 0 || s + decltype(phc)::value < nst) stage(s + decltype(phc)::value, phc);
+        });
 
     const int n0 = (nb0 + wn * P::NTW) * 16 + gl * 4;
     const bool vec = p.ldc % 4 == 0 && ((uintptr_t)p.C & 15) == 0;
@@ -354,9 +383,16 @@ template <int KIND, int SK, int BM, int BN, int SU> int launch_g(const orkh_mm *
     if (gp.G == SK) return launch_t<KIND, SK, 1, BM, BN, SU>(p, gp, s);
     if constexpr (SK == 64) {
         if (gp.G == 128) return launch_t<KIND, SK, 2, BM, BN, SU>(p, gp, s);
-        if constexpr (SU == 4)
+        if constexpr (SU == 4 || (KIND == ORKH_I8 && BN == 192)) { // (the tiles that ran slower with run-time counts)
+            if (gp.G == 192) return launch_t<KIND, SK, 3, BM, BN, SU>(p, gp, s);
             if (gp.G == 256) return launch_t<KIND, SK, 4, BM, BN, SU>(p, gp, s);
+            if (gp.G == 384) return launch_t<KIND, SK, 6, BM, BN, SU>(p, gp, s);
+            if (gp.G == 512) return launch_t<KIND, SK, 8, BM, BN, SU>(p, gp, s);
+            if (gp.G == 768) return launch_t<KIND, SK, 12, BM, BN, SU>(p, gp, s);
+        }
         if (gp.G % (SU * 128) == 0) return launch_t<KIND, SK, -1, BM, BN, SU>(p, gp, s);
+        if constexpr (SU > 1)
+            if (gp.G % 128 == 0) return launch_t<KIND, SK, -2, BM, BN, SU>(p, gp, s);
     }
     return launch_t<KIND, SK, 0, BM, BN, SU>(p, gp, s);
 }

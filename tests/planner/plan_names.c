@@ -1,6 +1,7 @@
 /* Prints the planner's choice for each "kind M K N" argument quadruple on a 256-CU device, one line each, named as
  * the library names its launches (orkh_mm_variant): orki_plan's, or after a first argument "mm" a run's (orki_plan_mm); after "chain", for each
- * "kind M K n N1 .. Nn", the joint launch of n matmuls ("single": none; orki_plan_group). Built from the host planner source alone, with no GPU code. */
+ * "kind M K n N1 .. Nn", the joint launch of n matmuls ("single": none; orki_plan_group); after
+ * "grouped", for each "kind M K N G", a grouped-scale run's (orki_plan_grouped). Built from the host planner source alone, with no GPU code. */
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -57,6 +58,18 @@ int main(int argc, char **argv) {
             for (int k = 0; k < n && k < ORKH_TGROUP_MAX; k++) N[k] = atoi(argv[i + 4 + k]);
             printf("%d %d %d %d %s\n", kind, M, K, n, orki_plan_group(&c, kind, M, K, N, n, (K + kpb - 1) / kpb, &q) ? name(kind, &q) : "single");
             i += 4 + n;
+        }
+        return 0;
+    }
+    if (argc > 1 && !strcmp(argv[1], "grouped")) {
+        for (int i = 2; i + 4 < argc; i += 5) {
+            const int kind = atoi(argv[i]), M = atoi(argv[i + 1]), K = atoi(argv[i + 2]), N = atoi(argv[i + 3]), G = atoi(argv[i + 4]);
+            const int kpb = kind == ORKH_I8 ? 64 : 128;
+            orkh_plan q;
+            orki_plan_grouped(&c, kind, M, K, N, (K + kpb - 1) / kpb, G, &q);
+            printf("%d %d %d %d ", kind, M, K, N);
+            if (q.algo == ORKH_ALGO_TILED2) printf("%dx%d\n", q.bm, q.bn);
+            else printf("%s\n", q.algo == ORKH_ALGO_GEMV ? "gemv" : "stream");
         }
         return 0;
     }

@@ -256,6 +256,8 @@ def test_grouped_tiled_exact(npu, tile, kind, M, K, N, G):
     (200, 1152, 320, 192),  # the same, 64-k steps; K tail
     (97, 672, 192, 96),     # 32-k steps; K tail
     (257, 2048, 512, 512),  # whole stages per group; two row tiles and one row
+    (65, 3840, 192, 640),   # whole 128-k spans that divide no stage: groups end inside stages
+    (70, 2304, 128, 768),   # groups whose ends recur every three four-line stages, six one-line ones; K ends inside a stage
 ])
 def test_grouped_tiles_exact(npu, tile, M, K, N, G):
     """Every tile of the grouped kernel in each form of its groups' ends, int8 and W4A4, at partial tiles and stages:
