@@ -429,13 +429,17 @@ int q3_layer_rows(q3_model *m, int l, float *out, int rows) {
     return ork_dev_download(m->ctx, out, m->trace + (size_t)l * m->c.max_rows * H, (size_t)rows * H * 4) ? -1 : 0;
 }
 
-/* Prefill attention by blocks of rows: below BLOCK rows the row-by-row kernel, up to 256 k_attn_block, above that
- * k_attn_scores and k_attn_pv, whose third launch and tiles of 64 keys want more rows. Whole prefills at Qwen3-1.7B
- * widths with new inputs each time, us: two layers, M=20 / 31 block 221 / 226, by row 209 / 222; block / scores and P.V:
- * two layers M=45 236 / 242, M=100 238 / 240, M=256 288 / 290, M=350 357 / 345, M=413 383 / 358, one layer M=224 184 /
- * 186 and 185 / 192, M=300 220 / 213. (One workgroup per row that quantises as well, to save the launch: M=100 249.) */
+/* Prefill attention by blocks of rows: below BLOCK rows the row-by-row kernel, then k_attn_block, and k_attn_scores and
+ * k_attn_pv from MANY rows where the row's width times the rows reaches WORK: their third launch and serial chunks want that
+ * many rows and heads. Whole prefills at Qwen3-1.7B widths with new inputs each time, us: two layers, M=20 / 31 block 221 /
+ * 226, by row 209 / 222; block / scores and P.V: two layers M=45 236 / 242, M=100 238 / 240, M=256 288 / 290, M=350 357 / 345,
+ * M=413 383 / 358, one layer M=224 184 / 186 and 185 / 192, M=300 220 / 213. (One workgroup per row that quantises as well,
+ * to save the launch: M=100 249.) Other heads, two layers, block / scores and P.V (heads / kv heads x head_dim): 4/2x64 M=257
+ * 130 / 157, M=1000 239 / 274; 8/8x128 M=257 168 / 182, M=384 198 / 205, M=512 231 / 230, M=1000 452 / 368; 14/2x64 M=320 180 /
+ * 189, M=512 237 / 237, M=700 318 / 269; 6/2x192 M=384 202 / 208, M=700 326 / 289; 32/32x64 M=257 252 / 226. */
 #define Q3_ATTN_BLOCK_ROWS 32
 #define Q3_ATTN_MANY_ROWS 257
+#define Q3_ATTN_MANY_WORK (1 << 19) /* rows * heads * head_dim */
 
 /* ---- one pass of the decoder over M rows ------------------------------------------------------------------- */
 static int pass(q3_model *m, int M, int decode) {
@@ -496,7 +500,7 @@ static int pass(q3_model *m, int M, int decode) {
                                m->rcos, m->rsin, m->st, m->q, Ly->kc, Ly->vc};
             CK(q3k_qkv_post(&qp, s));
         }
-        if (M >= Q3_ATTN_MANY_ROWS && m->fused) {
+        if (m->fused && M >= Q3_ATTN_MANY_ROWS && M * NH * HD >= Q3_ATTN_MANY_WORK) {
             /* part holds the scores and the chunk statistics: pad64(M) + 2 Sa floats per (row, head), of the
              * S * (HD + 2) it has (HD >= 64); the attention rows replace the queries */
             at.sc = m->part;

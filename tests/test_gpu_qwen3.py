@@ -10,7 +10,7 @@ the GPU's tokens. Checked at every step:
 Graph-replayed and eagerly launched decode steps must give identical tokens and bit-identical logits, and so
 must the fused decode kernels (k_fgemv, k_attn_combine: 6 launches per layer) and the unfused operator sequence
 (9), which do the same float operations in the same order; likewise prefill attention by blocks of rows
-(k_attn_rows) and row by row.
+(k_attn_block, k_attn_scores and k_attn_pv) and row by row.
 """
 import numpy as np
 import pytest
@@ -157,6 +157,13 @@ def test_fused_decode_equals_unfused(npu, case):
     dict(name="mha-hd128", over=dict(heads=2, kv_heads=2), n=(17, 66, 258)),
     dict(name="gqa3-hd192", over=dict(heads=3, kv_heads=1, head_dim=192), n=(5, 70, 260)),
     dict(name="gqa2-hd256", over=dict(heads=2, kv_heads=1, head_dim=256), n=(63, 130, 257)),
+    # rows wide enough for scores and P.V (2^19 floats of attention output), each side of it
+    dict(name="gqa2-hd128-wide", over=dict(heads=16, kv_heads=8), n=(256, 257, 287, 288, 289, 320)),
+    dict(name="gqa4-hd64-wide", over=dict(heads=32, kv_heads=8, head_dim=64), n=(257, 319)),
+    dict(name="mha-hd128-wide", over=dict(heads=14, kv_heads=14), n=(292, 293, 305)),
+    dict(name="gqa3-hd192-wide", over=dict(heads=12, kv_heads=4, head_dim=192), n=(257, 261)),
+    dict(name="gqa2-hd256-wide", over=dict(heads=8, kv_heads=4, head_dim=256), n=(257, 290)),
+    dict(name="mqa16-hd128-wide", over=dict(heads=16, kv_heads=1), n=(259,)),
 ])
 def test_prefill_attention_by_blocks_equals_rows(npu, case):
     """Prefill attention by blocks of rows against row by row, at the edges of the key tiles (64), the chunks (32), the
