@@ -573,7 +573,7 @@ static int plan_core(const ork_npu *c, int rkind, int M, int K, int N, int KB, o
  * fp64 was 1.39 to 1.41 times the pick's (K=2048..8192); with two it is the pick's. k_big has two on its
  * 128-row tiles, one on the 256-row ones.
  * A context's planner overrides (ORK_PLAN, ORK_TILE and the others of orki_plan) turn the rule off, and ORK_PLAN=big with
- * ORK_TILE=BMxBN forces a k_big tile. */
+ * ORK_TILE=BMxBN forces a k_big tile (ORK_CWT=0/1: its store policy). */
 static const struct big_fit {
     int rkind, bm, bn;
     double a, b, c, e;
@@ -679,7 +679,8 @@ static void take_big(const ork_npu *c, int bm, int bn, int M, const int *N, int 
     q->bn = bn;
     q->ksplit = 1;
     q->kbs = KB;
-    q->cwt = tiles_of(M, N, n, bm, bn) <= cu; /* write-through C on one round, as orki_plan's tiles */
+    const char *fc = knob(c, "ORK_CWT");
+    q->cwt = fc ? atoi(fc) != 0 : tiles_of(M, N, n, bm, bn) <= cu; /* write-through C on one round, as orki_plan's tiles */
 }
 
 /* The k_big tile priced below `limit` us for n matmuls of N[i] columns, with at least `sums` fp32 sums an output; 0: none. */

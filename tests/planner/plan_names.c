@@ -8,13 +8,7 @@
 
 #include "internal.h"
 
-/* the planner's one call into the HIP layer (grouped runs: the LDS-ring kernel's ring size); not reached here */
-int orkh_tiled2_ring_lds(int kind, int bm, int bn) {
-    (void)kind, (void)bm, (void)bn;
-    return 163840;
-}
-
-/* the LDS-ring kernel's two-slot ring: the tiles the kernel builds it for (its LDS arithmetic, restated: int8 and
+/* the planner's one call into the HIP layer: the LDS-ring kernel's two-slot ring, the tiles the kernel builds it for (its LDS arithmetic, restated: int8 and
  * fp16 on 64 x 192, 128 x 128 and 128 x 96; uniform int4 on 128 x 128 only, its 64 x 192 and 128 x 96 stages being
  * 41 and 45 KiB; never NF4) */
 int orkh_tiled2_ring2_ok(int kind, int bm, int bn) {

@@ -14,6 +14,7 @@ import pytest
 
 import oracle as O
 import ork
+from devbuf import Filled
 
 pytestmark = pytest.mark.gpu
 
@@ -212,8 +213,7 @@ def _env_run(env, fn, npu, w, A, aS, bS):
 ])
 def test_grouped_tiled_exact(npu, tile, kind, M, K, N, G):
     """The LDS-ring grouped kernel (k_tiled2g; ORK_PLAN=tiled, and ORK_TILE when given) against the oracle bit
-    for bit, and against the panel-streaming k_grouped forced on the same inputs. G % 128 == 0 runs the
-    whole-stage variant, the other group sizes the K-block walk."""
+    for bit, and against the panel-streaming k_grouped forced on the same inputs."""
     _say("grouped tiled", kind, M, K, N, G, tile)
     L = ork.lib()
     if kind == "i8":
@@ -245,8 +245,7 @@ def test_grouped_tiled_exact(npu, tile, kind, M, K, N, G):
     L.ork_mm_free(npu.h, w)
 
 
-@pytest.mark.parametrize("tile", ["64x64", "64x128", "64x192", "128x128", "128x256"])
-@pytest.mark.parametrize("M,K,N,G", [
+GROUPED_SHAPES = [
     (1, 1024, 64, 32),      # one row, one panel group; two closes per 64 k
     (129, 1056, 192, 32),   # one row past a tile; the last stage holds 32 k
     (127, 1088, 320, 64),   # a close per step; the last stage holds 64 k, half a panel block of int4
@@ -258,10 +257,15 @@ def test_grouped_tiled_exact(npu, tile, kind, M, K, N, G):
     (257, 2048, 512, 512),  # whole stages per group; two row tiles and one row
     (65, 3840, 192, 640),   # whole 128-k spans that divide no stage: groups end inside stages
     (70, 2304, 128, 768),   # groups whose ends recur every three four-line stages, six one-line ones; K ends inside a stage
-])
+]
+
+
+@pytest.mark.parametrize("tile,M,K,N,G", [(t, *z) for z in GROUPED_SHAPES for t in ("64x64", "64x128", "64x192", "128x128", "128x256")
+                                          if t != "128x256" or z[3] % 64 == 0])  # (not built with 32-k steps)
 def test_grouped_tiles_exact(npu, tile, M, K, N, G):
     """Every tile of the grouped kernel in each form of its groups' ends, int8 and W4A4, at partial tiles and stages:
-    the oracle's bits (each float operation is the oracle's, in its order), and no store outside C."""
+    the oracle's bits (each float operation is the oracle's, in its order), and no store outside C: a device C between two
+    filled rows, on a 16-byte boundary (vector stores) and 4 bytes past one (word stores), write-through and write-back."""
     L = ork.lib()
     rng = np.random.default_rng(M + K + N + G)
     aS = rng.uniform(1e-3, 1e-2, size=(M, K // G)).astype(np.float32)
@@ -275,13 +279,60 @@ def test_grouped_tiles_exact(npu, tile, M, K, N, G):
         else:
             w = L.ork_i4_mm_pack_grouped(npu.h, K, N, ork.ptr(B), G)
         assert w
-        C = np.full((M + 2, N), -7, np.float32)
+        want = O.gemm_grouped(A, B, aS, bS, G).reshape(-1)
         fn = L.ork_i8_mm_run_grouped if kind == "i8" else L.ork_i4_mm_run_grouped
-        env = {"ORK_PLAN": "tiled", "ORK_TILE": tile}
-        rc, _ = _env_run(env, lambda h, w_, m, a, s, t, c: fn(h, w_, m, a, s, t, ork.ptr(C[1:])), npu, w, A, aS, bS)
-        assert rc == 0 and np.array_equal(C[1:-1], O.gemm_grouped(A, B, aS, bS, G))
-        assert (C[0] == -7).all() and (C[-1] == -7).all()
+        for shift, cwt in ((0, 1), (1, 0), (0, 0), (1, 1)):
+            c = Filled(npu, (M + 2) * N, np.float32, -7)
+            env = {"ORK_PLAN": "tiled", "ORK_TILE": tile, "ORK_CWT": str(cwt)}
+
+            def run(h, w_, m, a, s, t, _):
+                name = npu.grouped_plan_name(w_, m)
+                assert name.startswith("tiled2g_") and name.endswith("_" + tile), name
+                return fn(h, w_, m, a, s, t, c.at(N + shift))
+            rc, _ = _env_run(env, run, npu, w, A, aS, bS)
+            got = c.get()
+            c.free()
+            assert rc == 0 and np.array_equal(got[N + shift:N + shift + M * N], want), (kind, shift, cwt)
+            assert (got[:N + shift] == -7).all() and (got[N + shift + M * N:] == -7).all(), (kind, shift, cwt)
         L.ork_mm_free(npu.h, w)
+
+
+@pytest.mark.parametrize("kind", ["i8", "w4a4"])
+@pytest.mark.parametrize("tile", ["64x64", "64x128", "64x192", "128x128", "128x256"])
+def test_grouped_tiles_bands(npu, kind, tile):
+    """The grouped kernel past its first band of 1024 rows (a last band of fewer tile rows) on a grid of more than 256 tiles
+    that is no multiple of 8 (the XCD order's remainder, write-back stores): the oracle's bits."""
+    _say("grouped bands", kind, tile)
+    L = ork.lib()
+    bm, bn = map(int, tile.split("x"))
+    M, K, G = 1100, 128, 64
+    mt = -(-M // bm)
+    nt = next(n for n in range(1, 300) if mt * n > 256 and mt * n % 8)
+    N = nt * bn - (64 if bn > 64 else 0)
+    lo = -128 if kind == "i8" else -8
+    rng = np.random.default_rng(bm + bn)
+    A, B = (rng.integers(lo, -lo, size=z, dtype=np.int8) for z in ((M, K), (K, N)))
+    aS = rng.uniform(1e-3, 1e-2, size=(M, K // G)).astype(np.float32)
+    bS = rng.uniform(1e-3, 1e-2, size=(K // G, N)).astype(np.float32)
+    if kind == "i8":
+        w = npu.pack_i8(B)
+        assert L.ork_w_set_group(w, G) == 0
+    else:
+        w = L.ork_i4_mm_pack_grouped(npu.h, K, N, ork.ptr(B), G)
+    fn = L.ork_i8_mm_run_grouped if kind == "i8" else L.ork_i4_mm_run_grouped
+
+    def run(h, w_, m, a, s, t, c):
+        name = npu.grouped_plan_name(w_, m)
+        assert name.startswith("tiled2g_") and name.endswith("_" + tile), name
+        return fn(h, w_, m, a, s, t, c)
+    rc, C = _env_run({"ORK_PLAN": "tiled", "ORK_TILE": tile}, run, npu, w, A, aS, bS)
+    # the oracle's sequence, vectorised: exact group sums in fp32 (below 2^24), each product and sum rounded to fp32
+    want = np.zeros((M, N), np.float32)
+    for g in range(K // G):
+        P = A[:, g * G:(g + 1) * G].astype(np.float32) @ B[g * G:(g + 1) * G].astype(np.float32)
+        want += (P * aS[:, g:g + 1]) * bS[g]
+    assert rc == 0 and np.array_equal(C, want)
+    L.ork_mm_free(npu.h, w)
 
 
 @pytest.mark.parametrize("G", [32, 64, 96, 128])
@@ -307,8 +358,8 @@ def test_grouped_rule_either_side(npu, G):
 
 def test_grouped_plan_names(npu):
     """Default plans: one row runs the half-panel VALU kernel (k_grouped_gemv), a few rows stream panels
-    (k_grouped); int8 / uniform int4 take the LDS-ring kernel from 32 rows when G % 128 == 0 and from 128 rows
-    otherwise; NF4 always streams."""
+    (k_grouped); int8 / uniform int4 take k_tiled2g from 32 rows when G % 128 == 0, from 17 with G of 32 or 64
+    where N is at least 512 (here 256) and from 128 rows otherwise; NF4 always streams."""
     L = ork.lib()
     B = np.zeros((1024, 256), np.int8)
     w = npu.pack_i8(B)

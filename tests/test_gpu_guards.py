@@ -9,7 +9,8 @@ bands and fails the run (-1) when a kernel wrote into them.
 
 Covered: the M = 1 GEMV (half and whole panels, split K), the streaming MFMA kernel (one panel and paired panels,
 row tails, split K), the LDS-ring tiles with M and N tails (every tile on offer, split K), the older LDS kernel,
-fp16 / uniform int4 / NF4 / W4A4 panels, the grouped-scale kernels (one row, streaming, LDS ring), the multi-matmul
+fp16 / uniform int4 / NF4 / W4A4 panels, the many-row kernel (every tile and kind, both store policies, an unaligned C),
+the grouped-scale kernels (one row, streaming, every tile of the tiled one), the multi-matmul
 submit with a C row stride, and the no-allocation entry point. Results are checked against the oracle as well.
 """
 import os
@@ -158,6 +159,14 @@ CASES = [
     ("nf4", 100, 1024, 96, {"ORK_PLAN": "tiled"}, "tiled_nf4"),
     ("nf4", 100, 1024, 96, {"ORK_PLAN": "tiled", "ORK_TILE": "128x96"}, "tiled_nf4_128x96"),
     ("i8", 100, 1024, 96, {"ORK_PLAN": "tiled"}, "tiled_i8"),
+    ("i8", 300, 1056, 544, {"ORK_PLAN": "big", "ORK_TILE": "256x256"}, "big_i8_256x256"),
+    ("f16", 300, 1056, 544, {"ORK_PLAN": "big", "ORK_TILE": "256x192"}, "big_f16_256x192"),
+    ("f16", 140, 1056, 272, {"ORK_PLAN": "big", "ORK_TILE": "128x256", "ORK_CWT": 0}, "big_f16_128x256"),
+    ("i8", 140, 1056, 224, {"ORK_PLAN": "big", "ORK_TILE": "128x192", "ORK_CWT": 0}, "big_i8_128x192"),
+    ("i4u", 140, 1056, 288, {"ORK_PLAN": "big", "ORK_TILE": "128x256"}, "big_i4u_128x256"),
+    ("nf4", 300, 1056, 544, {"ORK_PLAN": "big", "ORK_TILE": "256x192", "ORK_CWT": 0}, "big_nf4_256x192"),
+    ("nf4", 140, 1056, 224, {"ORK_PLAN": "big", "ORK_TILE": "128x192"}, "big_nf4_128x192"),
+    ("w4a4", 300, 1056, 576, {"ORK_PLAN": "big", "ORK_TILE": "256x256", "ORK_CWT": 0}, "big_i4u_256x256"),
 ]
 
 
@@ -213,6 +222,9 @@ def test_host_c_guards(gnpu):
     (8, 2048, 160, 64, {}, "grouped_i8_mt"),
     (100, 2080, 224, 160, {"ORK_PLAN": "tiled", "ORK_TILE": "64x64"}, "tiled2g_i8_64x64"),
     (70, 2048, 224, 512, {"ORK_PLAN": "tiled", "ORK_TILE": "64x192"}, "tiled2g_i8_64x192"),
+    (70, 2048, 160, 64, {"ORK_PLAN": "tiled", "ORK_TILE": "64x128"}, "tiled2g_i8_64x128"),
+    (150, 2080, 160, 32, {"ORK_PLAN": "tiled", "ORK_TILE": "128x128"}, "tiled2g_i8_128x128"),
+    (150, 2048, 288, 128, {"ORK_PLAN": "tiled", "ORK_TILE": "128x256", "ORK_CWT": 0}, "tiled2g_i8_128x256"),
 ])
 def test_grouped_guards(gnpu, M, K, N, G, env, want):
     L = ork.lib()
@@ -274,6 +286,39 @@ def test_allwave_epilogue_c_alignment_guards(gnpu, shift, M, kind, tile):
             assert O.fp16_err(body[shift:shift + M * N * 4].view(np.float32).reshape(M, N), ref(A)) <= 2e-3
         else:
             assert np.array_equal(body[shift:shift + M * N * 4].view(np.int32).reshape(M, N), ref(A))
+    finally:
+        g.free()
+        ork.lib().ork_dev_free(gnpu.h, dA)
+        ork.free(w)
+
+
+@pytest.mark.parametrize("cwt", [0, 1])
+@pytest.mark.parametrize("shift", [4, 8])
+@pytest.mark.parametrize("kind,tile", [("i8", "256x256"), ("f16", "128x256"), ("i4u", "256x192"), ("nf4", "128x192")])
+def test_many_row_c_alignment_guards(gnpu, kind, tile, shift, cwt):
+    """The many-row kernel into a C that starts 4 or 8 bytes past a 16-byte boundary (a word at a time, write-back and
+    write-through): exact (fp16: within its bar), and the bytes either side untouched."""
+    rng = np.random.default_rng(990 + shift + cwt + len(kind))
+    M, K, N = 301, 416, 320
+    w, run, gen_a, ref = _weight(gnpu, kind, K, N, rng)
+    A = gen_a(M)
+    g = Guarded(gnpu, M * N * 4 + 16)
+    dA = _dev(gnpu, A)
+    try:
+        with _env({"ORK_PLAN": "big", "ORK_TILE": tile, "ORK_CWT": cwt}):
+            name = gnpu.plan_name(w, M)
+            _say("many-row C alignment", kind, shift, cwt, name)
+            assert name == "big_%s_%s" % (kind, tile), name
+            assert run(gnpu.h, w, M, dA, g.c + shift) == 0
+        got = g.read()
+        g.check(got, name)
+        body, init = got[GUARD:-GUARD], g.init[GUARD:-GUARD]
+        assert np.array_equal(body[:shift], init[:shift]) and np.array_equal(body[shift + M * N * 4:], init[shift + M * N * 4:])
+        C = body[shift:shift + M * N * 4].view(np.float32 if kind == "f16" else np.int32).reshape(M, N)
+        if kind == "f16":
+            assert O.fp16_err(C, ref(A)) <= 2e-3
+        else:
+            assert np.array_equal(C, ref(A))
     finally:
         g.free()
         ork.lib().ork_dev_free(gnpu.h, dA)

@@ -12,6 +12,7 @@ import pytest
 import goldens as G
 import oracle as O
 import ork
+from devbuf import Filled
 
 pytestmark = pytest.mark.gpu
 
@@ -937,11 +938,13 @@ def test_many_row_tiles(npu, kind, tile):
         ork.free(w)
 
 
+@pytest.mark.parametrize("cwt", [0, 1])
 @pytest.mark.parametrize("tile", BIG_TILES)
-def test_many_row_chain_and_stride(npu, tile):
-    """Two projections of one input as one many-row launch (int8 and uniform int4), into one buffer at a row stride that
-    keeps rows 16-byte aligned and one that does not (vector and word stores): exact, and nothing outside the blocks."""
-    _say("many-row chain", tile)
+def test_many_row_chain_and_stride(npu, tile, cwt):
+    """Two projections of one input as one many-row launch (int8 and uniform int4), into one device buffer at a row stride
+    that keeps rows 16-byte aligned and one that does not (vector and word stores), write-back and write-through: exact,
+    and no other word of the buffer written."""
+    _say("many-row chain", tile, cwt)
     bm, bn = map(int, tile.split("x"))
     rng = np.random.default_rng(7 * bm + bn)
     M, K, Ns = bm + 9, 416, (bn + 32, 96)
@@ -958,14 +961,55 @@ def test_many_row_chain_and_stride(npu, tile):
                     w, _ = npu.pack_i4a8(W)
                     refs.append(O.gemm_i32(A, O.pack_i4a8(W)[2]))
                 ws.append(w)
-            C = np.full((M, ld), -77, np.int32)
-            with _env(ORK_PLAN="big", ORK_TILE=tile):
-                t = ork.tasks(ork.TaskI8, [(ws[0], M, A, C, ld), (ws[1], M, A, int(C.ctypes.data) + 4 * Ns[0], ld)])
+            c = Filled(npu, (M + 2, ld), np.int32, -77)
+            with _env(ORK_PLAN="big", ORK_TILE=tile, ORK_CWT=cwt):
+                assert npu.plan_name(ws[0], M).startswith("big_")
+                t = ork.tasks(ork.TaskI8, [(ws[0], M, A, c.at(ld), ld), (ws[1], M, A, c.at(ld + Ns[0]), ld)])
                 assert ork.lib().ork_i8_mm_run_chain(npu.h, 2, t) == 0
-            assert np.array_equal(C[:, :Ns[0]], refs[0]) and np.array_equal(C[:, Ns[0]:sum(Ns)], refs[1]), (kind, ld)
-            assert np.all(C[:, sum(Ns):] == -77)
+            C = c.get()
+            c.free()
+            assert np.array_equal(C[1:-1, :Ns[0]], refs[0]) and np.array_equal(C[1:-1, Ns[0]:sum(Ns)], refs[1]), (kind, ld)
+            assert np.all(C[:, sum(Ns):] == -77) and np.all(C[[0, -1]] == -77), (kind, ld)
             for w in ws:
                 ork.free(w)
+
+
+@pytest.mark.parametrize("M", [1100, 2300])
+@pytest.mark.parametrize("tile", BIG_TILES)
+@pytest.mark.parametrize("kind", ["i8", "i4a8", "nf4", "w4a4", "f16"])
+def test_many_row_bands(npu, kind, tile, M):
+    """The many-row kernel past its first bands of 1024 rows (a last band of fewer tile rows) on grids of more than 256 tiles
+    that are no multiple of 8 (the XCD order's remainder, several rounds, write-back stores). Integers exact; fp16 within
+    the bar of fp64 accumulation."""
+    _say("many-row bands", kind, tile, M)
+    bm, bn = map(int, tile.split("x"))
+    mt, K = -(-M // bm), 160
+    N = next(n for n in range(1, 300) if mt * n > 256 and mt * n % 8) * bn - 64
+    rng = np.random.default_rng(bm + bn + M)
+    if kind == "f16":
+        B = (rng.standard_normal((K, N)) * 0.02).astype(np.float16)
+        A = rng.standard_normal((M, K)).astype(np.float16)
+        w, run, codes = npu.pack_f16(B), npu.run_f16, B
+    elif kind in ("w4a4", "i8"):
+        lo = -8 if kind == "w4a4" else -128
+        codes = rng.integers(lo, -lo, size=(K, N), dtype=np.int8)
+        A = rng.integers(lo, -lo, size=(M, K), dtype=np.int8)
+        w, run = (npu.pack_i4(codes), npu.run_i4) if kind == "w4a4" else (npu.pack_i8(codes), npu.run_i8)
+    else:
+        W = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+        with _env(**({"ORK_NF4": 1} if kind == "nf4" else {})):
+            w, _ = npu.pack_i4a8(W)
+        A = rng.integers(-128, 128, size=(M, K), dtype=np.int8)
+        run, codes = npu.run_i8, O.pack_i4a8(W, nf4=kind == "nf4")[2]
+    with _env(ORK_PLAN="big", ORK_TILE=tile):
+        rc, C = run(w, A)
+        name = npu.plan_name(w, M)
+    assert rc == 0 and name.startswith("big_") and name.endswith(tile), name
+    if kind == "f16":
+        assert O.fp16_err(C, A.astype(np.float64) @ codes.astype(np.float64)) <= FP16_TOL
+    else:  # fp32 holds these sums exactly (160 products below 2^14)
+        assert np.array_equal(C, (A.astype(np.float32) @ codes.astype(np.float32)).astype(np.int32))
+    ork.free(w)
 
 
 def test_many_row_rule(npu):
