@@ -166,7 +166,7 @@ typedef struct orkh_group {
  * int8 and uniform int4). 0 / -2 bad arguments / -1 HIP error. */
 int orkh_mm_launch_grouped(const orkh_mm *p, const orkh_plan *plan, int G, const float *aS, const float *bS, float *C,
                            int ldc, void *stream);
-/* its ORKH_ALGO_TILED2 launch (orkh_grouped.hip; p carries C, ldc and c_wt): 64 x 64, 64 x 192, 128 x 128, 128 x 256 */
+/* its ORKH_ALGO_TILED2 launch (orkh_grouped.hip; p carries C, ldc and c_wt): 64 x 64, 64 x 128, 64 x 192, 128 x 128, 128 x 256 */
 int orkh_tiled2g_launch(const orkh_mm *p, const orkh_plan *plan, int G, const float *aS, const float *bS, void *stream);
 int orkh_mm_launch_group(const orkh_group *g, int wpg, void *stream);
 /* One-row run with a fused row prologue and column epilogue (k_gemv_row, orkh_rowrun.hip): every workgroup builds the

@@ -72,17 +72,6 @@ template <int KIND> __device__ __forceinline__ v4i step_op(v4i raw, int kk, cons
     }
 }
 
-// Direct-to-LDS load at a per-lane offset plus a scalar one (the range check covers the per-lane offset only: a lane
-// whose sum would leave the resource carries OOB)
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void lds_dma16s(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, uint32_t lds_byte) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_byte), "v"(voff), "s"(r),
-                 "s"(soff)
-                 : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
 template <int KIND, int BM, int BN>
 __device__ __forceinline__ void big_body(const orkh_mm &p, int mtiles, int ntiles, int bid) {
     using T = KT<KIND>;

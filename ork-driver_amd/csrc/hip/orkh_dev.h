@@ -1,5 +1,6 @@
-// orkh_dev.h -- device helpers shared by the matmul kernels on resident panels (orkh_kernels.hip, orkh_big.hip): the
-// panel kinds, nibble and NF4 decode, MFMA, raw buffer loads, direct-to-LDS loads, write-through stores.
+// orkh_dev.h -- device helpers shared by the matmul kernels on resident panels (orkh_kernels.hip, orkh_big.hip,
+// orkh_grouped.hip): the panel kinds, nibble and NF4 decode, MFMA, raw buffer loads, direct-to-LDS loads, write-through
+// stores.
 #ifndef ORKH_DEV_H
 #define ORKH_DEV_H
 #include <hip/hip_runtime.h>
@@ -131,6 +132,18 @@ template <int SITE = 0>
 __device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t lds_byte) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds ; site %3" ::"s"(lds_byte),
                  "v"(voff), "s"(r), "i"(SITE)
+                 : "memory", "m0");
+}
+// At a per-lane offset plus a scalar one, 16 and 4 bytes a lane (the range check covers the per-lane offset only: a lane
+// whose sum would leave the resource carries OOB)
+__device__ __forceinline__ void lds_dma16s(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, uint32_t lds_byte) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_byte), "v"(voff), "s"(r),
+                 "s"(soff)
+                 : "memory", "m0");
+}
+__device__ __forceinline__ void lds_dma4s(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, uint32_t lds_byte) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds_byte), "v"(voff), "s"(r),
+                 "s"(soff)
                  : "memory", "m0");
 }
 #pragma clang diagnostic pop

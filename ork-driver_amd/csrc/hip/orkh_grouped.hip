@@ -88,22 +88,6 @@ template <int KIND, int SK, int GS, int BM, int BN, int SU> struct TGP {
                   "tile");
 };
 
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-// Direct-to-LDS loads at a per-lane offset plus a scalar one: 16 and 4 bytes a lane (the range check covers the per-lane
-// offset only: a lane whose sum would leave the resource carries OOB)
-__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, uint32_t lds_byte) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_byte), "v"(voff), "s"(r),
-                 "s"(soff)
-                 : "memory", "m0");
-}
-__device__ __forceinline__ void dma4(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, uint32_t lds_byte) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds_byte), "v"(voff), "s"(r),
-                 "s"(soff)
-                 : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
 template <int... T, class F> __device__ __forceinline__ void each(std::integer_sequence<int, T...>, F &&f) {
     (f(std::integral_constant<int, T>{}), ...);
 }
@@ -173,17 +157,17 @@ __global__ __launch_bounds__(512, 1) void k_tiled2g(orkh_mm p, TG gp, int mtiles
         for (int z = decltype(q0)::value; z < decltype(q1)::value; z++) {
             if (z < P::QA) {
                 const int q = z, i = wv + q * NW;
-                dma16(Ar, k0 + (uint32_t)(i / (BM / 8)) * 128u + ch < (uint32_t)p.K ? va[q] : OOB, k0, slot + i * 1024);
+                lds_dma16s(Ar, k0 + (uint32_t)(i / (BM / 8)) * 128u + ch < (uint32_t)p.K ? va[q] : OOB, k0, slot + i * 1024);
             } else if (z < P::QA + P::QB) {
                 const int q = z - P::QA, i = wv + q * NW;
-                dma16(Br, ist * P::BPS + i % P::BPS < p.KB ? vb[q] : OOB, (uint32_t)ist * (P::BPS * 1024),
+                lds_dma16s(Br, ist * P::BPS + i % P::BPS < p.KB ? vb[q] : OOB, (uint32_t)ist * (P::BPS * 1024),
                       i < P::NB ? slot + (P::NA + i) * 1024 : lds0 + P::JUNK);
             } else {
                 const int q = z - P::QA - P::QB, i = wv + q * NW, is = i - P::NSA;
                 const bool isa = i < P::NSA;
                 const int g = ig + (isa ? i / (BM / 64) : is / (BN / 64));
                 const bool ok = g < Sk;
-                dma4(isa ? Sa : Sb, ok ? vs[q] : OOB, ok ? (uint32_t)g * (isa ? 4u : (uint32_t)p.N * 4u) : 0u,
+                lds_dma4s(isa ? Sa : Sb, ok ? vs[q] : OOB, ok ? (uint32_t)g * (isa ? 4u : (uint32_t)p.N * 4u) : 0u,
                      i < P::NSA + P::NSB ? slot + P::SCA + i * 256 : lds0 + P::JUNK);
             }
         }
