@@ -628,10 +628,11 @@ static double tile_kib(int rkind, int bm, int bn, int kbs) {
     return ((double)bm * a_bytes_per_kb(rkind) + bn * 64.0) * kbs / 1024;
 }
 
-/* Price of orki_plan's pick q over its wgs workgroups, times the kind's margin; mb: C's megabytes. From K = 256 (the
- * timed range) a 256 x 256 pick moves wherever a k_big tile is offered: over the 143 timed int8 and fp16 shapes with that pick the rule's k_big tile was more
- * than 4% slower at three (int8 K=256 N=12288 M=3300 40.2 -> 41.8 us, K=896 N=9728) and up to 15% faster where the fits call them level (int8 K=256
- * N=12288 M=4096 54.0 -> 46.1, fp16 K=1024 N=8192 M=3300 79.1 -> 70.8). */
+/* Price of orki_plan's pick q over its wgs workgroups, times the kind's margin; mb: C's megabytes. From K = 256
+ * (the timed range) a 256 x 256 pick moves wherever a k_big tile is offered, so k_tiled2's runs below that and where an fp16
+ * pick has four sums: over the 143 timed int8 and fp16 shapes with that pick the rule's k_big tile was more than 4% slower
+ * at three (int8 K=256 N=12288 M=3300 40.2 -> 41.8 us, K=896 N=9728) and up to 15% faster where the fits call them level
+ * (int8 K=256 N=12288 M=4096 54.0 -> 46.1, fp16 K=1024 N=8192 M=3300 79.1 -> 70.8). */
 static double pick_us(int rkind, const orkh_plan *q, long wgs, int KB, double mb, int cu) {
     const struct pick_fit *p = pick_fits;
     while (p->rkind != rkind) p++;
