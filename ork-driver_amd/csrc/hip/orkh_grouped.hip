@@ -10,7 +10,7 @@
 // (four float operations per output and group: at G=32 they are 16 per 16 x 16 x 32 MFMA, which takes 16 cycles against
 // their 64), else by operand delivery: one CU's loads and LDS reads (M=64 and M=256 take the same time on 64 x 64, 64 and
 // 256 of 256 CUs). Against the former kernel (16 waves, a masked MFMA per group and 128-k block, the tile's scales whole
-// in LDS), us at K=N=4096: W4A4 M=256 G=32 57.2 -> 27.3, G=64 36.1 -> 16.3, G=128 15.4 -> 12.8, G=512 11.1 -> 11.0; int8
+// in LDS), us at K=N=4096: W4A4 M=256 G=32 57.2 -> 27.3, G=64 36.1 -> 16.3, G=128 15.4 -> 12.8, G=512 11.1 -> 10.5; int8
 // M=256 G=32 46.0 -> 24.9, G=64 21.9 -> 16.3, G=128 18.3 -> 13.6, G=512 14.8 -> 12.4; M=2048 G=128 W4A4 95.0 -> 56.5
 // (1.21 PFLOP/s), int8 85.1 -> 53.5. What the layout is for:
 //  - MFMA steps hold SK consecutive k, SK dividing every group: 64 (v_mfma_i32_16x16x64_i8) where G % 64 == 0, else 32
@@ -22,7 +22,7 @@
 //  - MFMA operands swapped (D = B^T A^T): a lane holds four columns of one row, so a group's close needs one aS value per
 //    row block and one 16-byte read of bS per column block, and C goes out 16 bytes a store;
 //  - where a group is a compile-time number of steps or whole stages (GS), its end is known without a test, and its first
-//    step starts the accumulators from zero (W4A4 M=256 G=512, 64 x 64: 15.0 us with a test a step, 11.0 without). Where
+//    step starts the accumulators from zero (W4A4 M=256 G=512, 64 x 64: 15.0 us with a test a step, 10.5 without). Where
 //    the steps of a group do not divide a stage's the stage is compiled once for each place a group can stand in it (PH):
 //    us, a run-time count of steps or stages, then this: W4A4 64 x 64 K=6144 N=2048 M=256 G=192 20.5 -> 15.5, G=384 18.5
 //    -> 14.0, G=768 17.3 -> 13.2, K=N=3072 G=512 9.1 -> 8.7; int8 64 x 192 K=N=3072 M=768 G=192 22.0 -> 19.0, G=256 19.8

@@ -406,8 +406,8 @@ __global__ __launch_bounds__(256) void k_attn_block(q3_att p) {
     }
 }
 
-// Prefill attention (more than 256 rows, rotated queries in p.q): scores and softmax terms of every (row, query head, key) by
-// k_attn_scores, then P.V and the chunk combine in registers by k_attn_pv, with k_attn_part's and attn_quant_body's
+// Prefill attention (more than 256 rows of many heads, q3_model.c; rotated queries in p.q): scores and softmax terms of
+// every (row, query head, key) by k_attn_scores, then P.V and the chunk combine in registers by k_attn_pv, with k_attn_part's and attn_quant_body's
 // operations in their order (the four score sums, the 32-key chunk's max and sum, the chunk's P.V accumulation over
 // ascending keys, the log-sum-exp combine over ascending chunks), so the rows are bit-identical to the row-by-row
 // kernels'. Both are bound by the VALU: mul and add round separately (no FMA), 4 * HD operations per (row, head, key).
@@ -415,8 +415,8 @@ __global__ __launch_bounds__(256) void k_attn_block(q3_att p) {
 // sits in one register and is broadcast by the multiply itself, the other comes from registers or one LDS read per 16
 // products, and only the probabilities cross HBM (4 bytes per score), where one workgroup per (32-key chunk, 4 rows)
 // wrote every chunk's P.V row (HD + 2 floats) and a combine launch read it back. Per layer at Qwen3-1.7B widths,
-// traced, k_attn_block -> this (with the row quantisation): M=1000 295 -> 184 us, M=500 81 -> 68; whole prefills of
-// two layers M=500 377 -> 353, M=700 574 -> 461, M=1000 855 -> 634.
+// traced, k_attn_block -> this (with the row quantisation): M=1000 280 -> 175 us, M=500 78 -> 65; whole prefills of
+// two layers M=500 359 -> 327, M=700 545 -> 435, M=1000 864 -> 634.
 // At M=1000 the mul / add pairs alone take 104 us at the VALU's rate.
 // Lane N of each 16-lane row, in every lane of the row: folded into the multiply that uses it (a DPP operand).
 template <int N> __device__ __forceinline__ float bc16(float x) {
