@@ -1,4 +1,5 @@
-"""The planner's NF4 picks against measurements, on the CPU.
+"""The planner's picks against measurements, on the CPU: single runs (orki_plan, and orki_plan_mm above 64 rows), chains'
+joint launches and grouped-scale runs, each against its sweep under tests/golden.
 
 tests/planner/plan_names.c prints the planner's choice (plan.c alone, a 256-CU device) for each shape of
 tests/golden/nf4_plan_sweep.json, which holds graph-timed MI355X launches of every NF4 kernel, tile and K split on
@@ -125,7 +126,8 @@ def test_run_picks_against_the_sweep(planner, kind):
     tot_pick = tot_best = tot_former = 0.0
     for (_, K, N, M, former, us, *big), old, p in zip(runs, planner(cases), planner(cases, mm=True)):
         assert old == former, (K, N, M, old, former)
-        times = {"big_" + {"int8": "i8", "fp16": "f16"}.get(kind, kind) + "_" + t: x for t, x in zip(("256x256", "256x192", "128x256", "128x192"), big)}
+        kn = {"int8": "i8", "fp16": "f16"}.get(kind, kind)
+        times = {"big_%s_%s" % (kn, t): x for t, x in zip(("256x256", "256x192", "128x256", "128x192"), big)}
         if kind == "fp16":
             times = {t: x for t, x in times.items() if _f16_sums(t) >= _f16_sums(former)}
         times[former] = us
